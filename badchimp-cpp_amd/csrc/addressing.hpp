@@ -1,4 +1,4 @@
-// Where a bulk node pulls each population from: three address layouts.
+// Where a bulk node pulls each population from: the address layouts.
 //
 // Every layout provides sources<L>(i, src): the population element index
 // (pidx, context.hpp) of the post-collision value that becomes f_q of node i,
@@ -21,16 +21,32 @@
 //            popcount(mask below the bit).  The table is a few MB and stays in
 //            L2 / MALL.  One lookup per direction.
 //
-// RowWin     as RowAddr for boxes that are not periodic along the row axis:
-//            per row and word w it keeps a 64-bit window of the row's fluid
-//            bits over cells [32w-16, 32w+48) and the compact index of the
-//            window's first fluid cell.  The node's own word then covers the
-//            cells z-1, z, z+1 of every neighbouring row, so the 9 (D3Q19) or
-//            3 (D2Q9) neighbouring rows are one 16-byte load each, and the
-//            three sources in a row follow from one popcount: with b0 the
-//            index of the first fluid cell at or after z, the source at z is
-//            b0, at z-1 it is b0-1, at z+1 it is b0 + bit(z).  The window
-//            table has a halo of rows, so no wrap logic runs per node.
+// RowWin     per row and word w of 8 cells it keeps, in one 32-bit word, the
+//            fluid bits of the 10 cells 8w-1 .. 8w+8 (bit kWinBase+k: cell
+//            8w-1+k) and the compact index of the first fluid cell at or after
+//            8w.  The node's own word then covers the cells z-1, z, z+1 of
+//            every neighbouring row, so the 9 (D3Q19) or 3 (D2Q9) neighbouring
+//            rows are one 4-byte load each, and the three sources in a row
+//            follow from one popcount: with b0 the index of the first fluid
+//            cell at or after z, the source at z is b0, at z-1 it is b0-1, at
+//            z+1 it is b0 + bit(z).  The window table has a halo of rows, so
+//            no wrap logic runs per node.  22 bits hold the index of up to
+//            4.19 M nodes; larger node lists count it from the first node of
+//            the cell's x plane, three more loads per node.
+//            One dword per row and not more: a wave's load of up to 4 bytes
+//            per lane takes the vector L1 about 5 cycles where 16 lanes read
+//            neighbouring words (the nodes of a row do), one of 8 or 16 bytes
+//            takes 17 whatever it reads (measured on tables in L2), and the
+//            step keeps that unit busy 80-90 % of its time.  Against 16-byte
+//            entries over 32 cells a step takes, on the 256^3 pack, 127 us for
+//            142 (FP16S), 187 for 192 (FP32S) and 350 as before (FP64, bound
+//            by the memory); on a 161 x 143 x 150 pack 26.8 for 30.1 (FP16S).
+//            The struct stays at 32 bytes: 48 bytes of it made the step of the
+//            256 x 128 channel 4 % slower, which waits for its arguments.
+// RowWinZ    RowWin for boxes that are periodic along the row axis: the bits of
+//            the first and the last word wrap, and the nodes at z = 0 and
+//            z = E_Z - 1 read the neighbouring rows' fluid counts, by which
+//            the compact index steps at the wrap.
 //
 // Rows are ordered in tiles of 2^lx x 2^ly rows, which keeps the neighbour
 // rows of a tile close in the compact order.  The row layouts are validated on
@@ -112,6 +128,14 @@ struct RowGeom {
   }
 };
 
+// Cells of a row window's word, and the bits of its base.
+constexpr uint32_t kWinLog = 3;
+constexpr uint32_t kWinCells = 1u << kWinLog;
+constexpr uint32_t kWinBase = 22;
+__host__ __device__ __forceinline__ constexpr int32_t win_words(int32_t ez) {
+  return (ez + static_cast<int32_t>(kWinCells) - 1) >> kWinLog;
+}
+
 // lattice direction components mapped to (X, Y, Z)
 template <class L>
 __host__ __device__ __forceinline__ constexpr int cx(int q) { return L::c(q, 0); }
@@ -153,86 +177,133 @@ struct RowAddr {
   }
 };
 
-struct RowWin {
+// PZ: the box is periodic along the row axis.
+template <bool PZ>
+struct WinWrap {};
+template <>
+struct WinWrap<true> {
+  const uint32_t* __restrict__ count;  // fluid cells of each padded row
+  int32_t EZ;                          // cells per row
+};
+template <bool PZ>
+struct RowWinT : WinWrap<PZ> {
   static constexpr bool kOff32 = true;
   const uint32_t* __restrict__ coord;  // X << 22 | Y << 12 | Z
-  const uint4* __restrict__ win;       // {base, mask lo, mask hi, 0} per (padded row, word)
-  uint32_t NP;
+  const uint32_t* __restrict__ win;    // fluid bits << kWinBase | base, per (padded row, word)
+  const uint32_t* __restrict__ plane;  // first node of each padded X; null: the bases count from node 0
   int32_t PY;  // padded rows along Y: E_Y + 2
-  int32_t W;   // words per row
+  int32_t W;   // words per row (win_words)
+
+  // What a node reads of its 9 (D3Q19) or 3 (D2Q9) neighbouring rows: the
+  // words, and the index of the first fluid cell at or after z.
+  template <class L>
+  struct Rows {
+    static constexpr int NY = L::nD == 3 ? 3 : 1;
+    uint32_t b0[3 * NY], m[3 * NY];
+    uint32_t t;  // bit of cell z - 1
+    // PZ: what to add for a source at z - 1 (z = 0) and to take away for one
+    // at z + 1 (z = E_Z - 1): the row's fluid cells, else 0
+    uint32_t lo[3 * NY], hi[3 * NY];
+    // row, step along z and fluid mask (all ones or zero) of the source cell r - c_q
+    __device__ __forceinline__ static constexpr int row(int q) {
+      return (1 - cx<L>(q)) * NY + (NY > 1 ? 1 - cy<L>(q) : 0);
+    }
+    // row k has sources at z - 1 and z + 1 (the rows along x = y hold only c_z = 0)
+    __device__ __forceinline__ static constexpr bool off_z(int k) { return NY == 1 || k / NY == 1 || k % NY == 1; }
+    __device__ __forceinline__ uint32_t fluid(int q) const {
+      return static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int32_t>(m[row(q)]), t + 1 - cz<L>(q), 1));
+    }
+    // compact index of the source cell, where it is fluid
+    __device__ __forceinline__ uint32_t node(int q) const {
+      const int k = row(q), dz = -cz<L>(q);
+      if (dz == 0) return b0[k];
+      if (dz < 0) return PZ ? b0[k] - 1u + lo[k] : b0[k] - 1u;
+      const uint32_t j = b0[k] + ((m[k] >> (t + 1u)) & 1u);
+      return PZ ? j - hi[k] : j;
+    }
+  };
 
   // The window table is indexed by the halo-padded row (X+1, Y+1): halo rows
   // of a periodic axis repeat the rows they wrap to, those of a closed axis
-  // are empty (all solid).  The 9 (D3Q19) or 3 (D2Q9) neighbouring rows of a
-  // node are then one vector offset plus a per-direction uniform base.
+  // are empty (all solid).  The neighbouring rows of a node are then one
+  // vector offset plus a per-direction uniform base.
   template <class L>
-  __device__ __forceinline__ void sources(int32_t i, uint32_t (&src)[L::nQ - 1]) const {
+  __device__ __forceinline__ void rows(int32_t i, Rows<L>& r) const {
     const uint32_t c = coord[i];
     const uint32_t X = c >> 22, Y = (c >> 12) & 1023u, Z = c & 4095u;
-    const uint32_t w = Z >> 5;
-    const uint32_t t = Z - 32u * w + 16u;  // bit of z in the window, 16..47
-    const uint32_t base = ((X + 1u) * static_cast<uint32_t>(PY) + (Y + 1u)) * static_cast<uint32_t>(W) + w;
-    constexpr int NY = L::nD == 3 ? 3 : 1;
-    uint4 e[3 * NY];
+    r.t = kWinBase + (Z & (kWinCells - 1u));
+    const uint32_t pr = (X + 1u) * static_cast<uint32_t>(PY) + (Y + 1u);
+    const uint32_t at = pr * static_cast<uint32_t>(W) + (Z >> kWinLog);
+    constexpr int NY = Rows<L>::NY;
 #pragma unroll
     for (int k = 0; k < 3 * NY; ++k) {
       const int dx = k / NY - 1, dy = NY > 1 ? k % NY - 1 : 0;
-      const uint4* __restrict__ wk = win + (dx * PY + dy) * W;
-      e[k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(wk) + base * 16u);
+      r.m[k] = ld32(win + (dx * PY + dy) * W, at);
     }
-    // per row: index of the first fluid cell at or after z, fluid bits of z-1, z, z+1
-    uint32_t b0[3 * NY];
-    uint32_t bm[3 * NY];
-    const uint64_t below = (1ull << t) - 1ull;
+    uint32_t first[3] = {0u, 0u, 0u};
+    if (plane) {
 #pragma unroll
-    for (int k = 0; k < 3 * NY; ++k) {
-      const uint64_t m = (static_cast<uint64_t>(e[k].z) << 32) | e[k].y;
-      b0[k] = e[k].x + static_cast<uint32_t>(__popcll(m & below));
-      bm[k] = static_cast<uint32_t>(m >> (t - 1u)) & 7u;  // bit0: z-1, bit1: z, bit2: z+1
+      for (int d = 0; d < 3; ++d) first[d] = ld32(plane + d, X);
     }
+    if constexpr (PZ) {
+      const uint32_t last = static_cast<uint32_t>(this->EZ) - 1u;
+#pragma unroll
+      for (int k = 0; k < 3 * NY; ++k) r.lo[k] = r.hi[k] = 0u;
+      if (Z == 0u || Z == last) {
+#pragma unroll
+        for (int k = 0; k < 3 * NY; ++k) {
+          if (!Rows<L>::off_z(k)) continue;
+          const int dx = k / NY - 1, dy = NY > 1 ? k % NY - 1 : 0;
+          const uint32_t n = ld32(this->count + (dx * PY + dy), pr);
+          r.lo[k] = Z == 0u ? n : 0u;
+          r.hi[k] = Z == last ? n : 0u;
+        }
+      }
+    }
+    const uint32_t below = (2u << r.t) - (2u << kWinBase);  // cells of the word before z
+#pragma unroll
+    for (int k = 0; k < 3 * NY; ++k)
+      r.b0[k] = (r.m[k] & ((1u << kWinBase) - 1u)) + (static_cast<uint32_t>(__popc(r.m[k] & below)) + first[k / NY]);
+  }
+
+  template <class L>
+  __device__ __forceinline__ void sources(int32_t i, uint32_t (&src)[L::nQ - 1]) const {
+    Rows<L> r;
+    rows<L>(i, r);
 #pragma unroll
     for (int q = 0; q < L::nQ - 1; ++q) {
-      // source cell r - c_q
-      const int k = (1 - cx<L>(q)) * NY + (NY > 1 ? 1 - cy<L>(q) : 0);
-      const int dz = -cz<L>(q);
-      const uint32_t fluid = (bm[k] >> (dz + 1)) & 1u;
-      const uint32_t j = dz == 0 ? b0[k] : (dz < 0 ? b0[k] - 1u : b0[k] + ((bm[k] >> 1) & 1u));
       // both candidates, combined by a mask: a per-lane select, not a branch
-      const uint32_t m = 0u - fluid;
-      src[q] = (pidx<L::nQ>(q, j) & m) | (pidx<L::nQ>(L::rev(q), i) & ~m);
+      const uint32_t m = r.fluid(q);
+      src[q] = (pidx<L::nQ>(q, r.node(q)) & m) | (pidx<L::nQ>(L::rev(q), i) & ~m);
     }
   }
-};
 
-// RowWin::links: the source node of every direction: bit q of fluid is set
-// when the source cell of direction q is the fluid node j[q] (else a solid,
-// and j[q] is undefined).
-template <class L>
-__device__ __forceinline__ void rowwin_links(const RowWin& ad, int32_t i, uint32_t (&j)[L::nQ - 1], uint32_t& fluid) {
-  const uint32_t c = ad.coord[i];
-  const uint32_t X = c >> 22, Y = (c >> 12) & 1023u, Z = c & 4095u;
-  const uint32_t w = Z >> 5;
-  const uint32_t t = Z - 32u * w + 16u;
-  const uint32_t base = ((X + 1u) * static_cast<uint32_t>(ad.PY) + (Y + 1u)) * static_cast<uint32_t>(ad.W) + w;
-  constexpr int NY = L::nD == 3 ? 3 : 1;
-  uint4 e[3 * NY];
-#pragma unroll
-  for (int k = 0; k < 3 * NY; ++k) {
-    const int dx = k / NY - 1, dy = NY > 1 ? k % NY - 1 : 0;
-    const uint4* __restrict__ wk = ad.win + (dx * ad.PY + dy) * ad.W;
-    e[k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(wk) + base * 16u);
+  // element at a 32-bit byte offset from a uniform base (tables below 4 GiB)
+  __device__ __forceinline__ static uint32_t ld32(const uint32_t* __restrict__ p, uint32_t e) {
+    return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(p) + e * 4u);
   }
-  const uint64_t below = (1ull << t) - 1ull;
+};
+using RowWin = RowWinT<false>;
+using RowWinZ = RowWinT<true>;
+
+// Windows of a batched solve.
+__host__ __device__ __forceinline__ RowWin solve_windows(const BatchSolve& s) {
+  return RowWin{{}, s.coord, s.win, s.plane, s.PY, s.W};
+}
+
+// The source node of every direction: bit q of fluid is set when the source
+// cell of direction q is the fluid node j[q] (else a solid, and j[q] is
+// undefined).
+template <class L, bool PZ>
+__device__ __forceinline__ void rowwin_links(const RowWinT<PZ>& ad, int32_t i, uint32_t (&j)[L::nQ - 1],
+                                             uint32_t& fluid) {
+  typename RowWinT<PZ>::template Rows<L> r;
+  ad.template rows<L>(i, r);
   fluid = 0u;
 #pragma unroll
   for (int q = 0; q < L::nQ - 1; ++q) {
-    const int k = (1 - cx<L>(q)) * NY + (NY > 1 ? 1 - cy<L>(q) : 0);
-    const int dz = -cz<L>(q);
-    const uint64_t m = (static_cast<uint64_t>(e[k].z) << 32) | e[k].y;
-    const uint32_t b0 = e[k].x + static_cast<uint32_t>(__popcll(m & below));
-    const uint32_t bm = static_cast<uint32_t>(m >> (t - 1u)) & 7u;
-    fluid |= ((bm >> (dz + 1)) & 1u) << q;
-    j[q] = dz == 0 ? b0 : (dz < 0 ? b0 - 1u : b0 + ((bm >> 1) & 1u));
+    fluid |= r.fluid(q) & (1u << q);
+    j[q] = r.node(q);
   }
 }
 
@@ -259,8 +330,8 @@ __device__ __forceinline__ void neighbour_phi(const TableAddr& ad, int32_t i, co
   pn[L::nQ - 1] = static_cast<T>(0);
 }
 
-template <class L, typename T>
-__device__ __forceinline__ void neighbour_phi(const RowWin& ad, int32_t i, const T* __restrict__ phi,
+template <class L, typename T, bool PZ>
+__device__ __forceinline__ void neighbour_phi(const RowWinT<PZ>& ad, int32_t i, const T* __restrict__ phi,
                                               const WallPhi& wp, T (&pn)[L::nQ]) {
   uint32_t j[L::nQ - 1], fluid;
   rowwin_links<L>(ad, i, j, fluid);

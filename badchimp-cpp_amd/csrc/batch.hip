@@ -122,11 +122,17 @@ Footprint footprint_of(int Q, size_t esz, int64_t n, int64_t nwin, int nf) {
   fp.off_f1 = fb;
   fp.off_coord = 2 * fb;
   fp.off_win = fp.off_coord + align_up(fp.NP * 4);
-  fp.off_part = fp.off_win + align_up(nwin * 16);
+  fp.off_part = fp.off_win + align_up(nwin * static_cast<int64_t>(sizeof(uint32_t)));
   fp.off_phi = fp.off_part + align_up((nf == 2 ? 3 : 1) * fp.nblk * 8);
   // colour field: double in FP64, float otherwise
   fp.bytes = fp.off_phi + (nf == 2 ? align_up(fp.NP * (esz == 8 ? 8 : 4)) : 0);
   return fp;
+}
+
+// 32-bit words of a solve's window table and its first nodes of the x planes
+int64_t window_words(const RowBuild& rb) {
+  const int64_t px = rb.g.E[0] + 2;
+  return px * (rb.g.E[1] + 2) * win_words(rb.g.E[2]) + (rb.coord.size() >> kWinBase ? px : 0);
 }
 
 struct Slot {
@@ -572,7 +578,7 @@ int lb_batch_footprint(int lattice, int precision, int32_t n_fields, int32_t nd,
   std::string why;
   if (!rows_from_geometry(lattice, dims, geo, periodic_mask, rb, why))
     return fail_global(LB_ERR_UNSUPPORTED, "lb_batch_footprint: %s", why.c_str());
-  const int64_t nwin = static_cast<int64_t>(rb.g.E[0] + 2) * (rb.g.E[1] + 2) * rb.g.W;
+  const int64_t nwin = window_words(rb);
   const Footprint fp = footprint_of(lattice == LB_D2Q9 ? 9 : 19, elem_bytes(precision),
                                     static_cast<int64_t>(rb.coord.size()), nwin, n_fields);
   if (bytes) *bytes = fp.bytes;
@@ -600,15 +606,14 @@ struct AddArgs {
 // checked node by node.  Pure host work, so many run in parallel.
 struct Prepared {
   RowBuild rb;
-  std::vector<uint4> win;
-  int32_t PY = 0;
+  WinBuild wb;
   int code = LB_OK;
   std::string why;
 };
 
 void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t periodic_mask, Prepared& pr) {
   if (!rows_from_geometry(lattice, dims, geo, periodic_mask, pr.rb, pr.why) ||
-      !build_windows(pr.rb, pr.win, pr.PY, pr.why)) {
+      !build_windows(pr.rb, false, pr.wb, pr.why)) {
     pr.code = LB_ERR_UNSUPPORTED;
     return;
   }
@@ -616,11 +621,8 @@ void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t perio
   const int64_t n = static_cast<int64_t>(rb.coord.size());
   // every node's own window must name it (a cheap check of the construction)
   for (int64_t i = 0; i < n; ++i) {
-    const uint32_t c = rb.coord[i];
-    const uint32_t X = c >> 22, Y = (c >> 12) & 1023u, Z = c & 4095u, w = Z >> 5, t = Z - 32 * w + 16;
-    const uint4 e = pr.win[(static_cast<size_t>(X + 1) * pr.PY + (Y + 1)) * rb.g.W + w];
-    const uint64_t m = (static_cast<uint64_t>(e.z) << 32) | e.y;
-    if (!((m >> t) & 1u) || e.x + static_cast<uint32_t>(__builtin_popcountll(m & ((1ull << t) - 1ull))) != i) {
+    const auto own = win_cell(rb, pr.wb, static_cast<int32_t>(i), 0, 0, 0);
+    if (!own.first || own.second != i) {
       pr.code = LB_ERR_STATE;
       pr.why = "row windows inconsistent at node " + std::to_string(i);
       return;
@@ -648,13 +650,12 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
   }
   if (pre->code != LB_OK) return bfail(b, pre->code, "lb_batch_add: %s", pre->why.c_str());
   const RowBuild& rb = pre->rb;
-  const std::vector<uint4>& win = pre->win;
-  const int32_t PY = pre->PY;
+  const WinBuild& wb = pre->wb;
   const int64_t n = static_cast<int64_t>(rb.coord.size());
   const int nf = p.kind == 1 ? 2 : 1;
   const int prec = b->prec[p.kind];
   const size_t esz = elem_bytes(prec);
-  const Footprint fp = footprint_of(b->Q, esz, n, static_cast<int64_t>(win.size()), nf);
+  const Footprint fp = footprint_of(b->Q, esz, n, window_words(rb), nf);
   if (static_cast<uint64_t>(nf) * b->Q * static_cast<uint64_t>(fp.NP) * esz >= (1ull << 32) ||
       fp.nblk > static_cast<int64_t>(kItemMask) + 1)
     return bfail(b, LB_ERR_UNSUPPORTED, "lb_batch_add: %lld fluid nodes exceed one solve", (long long)n);
@@ -676,15 +677,17 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
   }
   char* base = b->pool + off;
   BatchSolve d{};
+  uint32_t* dwin = reinterpret_cast<uint32_t*>(base + fp.off_win);
   d.coord = reinterpret_cast<const uint32_t*>(base + fp.off_coord);
-  d.win = reinterpret_cast<const uint4*>(base + fp.off_win);
+  d.win = dwin;
+  d.plane = wb.plane.empty() ? nullptr : dwin + wb.win.size();
+  d.PY = wb.PY;
+  d.W = wb.W;
   d.f[0] = base + fp.off_f0;
   d.f[1] = base + fp.off_f1;
   d.partial = reinterpret_cast<double*>(base + fp.off_part);
   d.phi = nf == 2 ? static_cast<void*>(base + fp.off_phi) : nullptr;
   d.NP = static_cast<uint32_t>(fp.NP);
-  d.PY = PY;
-  d.W = rb.g.W;
   d.n = static_cast<int32_t>(n);
   // the solve starts at the global step of the next launch sequence (the
   // host counter already covers a sequence in flight)
@@ -726,7 +729,10 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
   hipError_t e = hipMemcpyAsync(base + fp.off_coord, rb.coord.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice,
                                 up);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(base + fp.off_win, win.data(), win.size() * sizeof(uint4), hipMemcpyHostToDevice, up);
+    e = hipMemcpyAsync(dwin, wb.win.data(), wb.win.size() * sizeof(uint32_t), hipMemcpyHostToDevice, up);
+  if (e == hipSuccess && d.plane)
+    e = hipMemcpyAsync(dwin + wb.win.size(), wb.plane.data(), wb.plane.size() * sizeof(uint32_t),
+                       hipMemcpyHostToDevice, up);
   if (e == hipSuccess) {
     if (p.kind == 0) {
       // rest state f = w: zero in the shifted forms; a pull from it is the
@@ -760,11 +766,9 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
       double* r0d = reinterpret_cast<double*>(base + fp.off_f1);
       e = hipMemcpyAsync(r0d, r0c.data(), r0c.size() * sizeof(double), hipMemcpyHostToDevice, up);
       if (e == hipSuccess) {
-        const RowWin ad{reinterpret_cast<const uint32_t*>(base + fp.off_coord),
-                        reinterpret_cast<const uint4*>(base + fp.off_win), static_cast<uint32_t>(fp.NP), PY, rb.g.W};
-        e = prec == LB_FP64 ? prestream_f64(b->lattice, ad, r0d, static_cast<int32_t>(n), fp.NP,
+        e = prec == LB_FP64 ? prestream_f64(b->lattice, solve_windows(d), r0d, static_cast<int32_t>(n), fp.NP,
                                             reinterpret_cast<double*>(base + fp.off_f0), up)
-                            : prestream_lowp(prec, b->lattice, ad, r0d, static_cast<int32_t>(n), fp.NP,
+                            : prestream_lowp(prec, b->lattice, solve_windows(d), r0d, static_cast<int32_t>(n), fp.NP,
                                              base + fp.off_f0, up);
       }
     }

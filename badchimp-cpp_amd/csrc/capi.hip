@@ -502,11 +502,10 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
     rows_ok = false;
     why = "row layout disagrees with the neighbour index";
   }
-  // row windows when the row axis is not periodic, checked link by link
-  std::vector<uint4> win;
-  int32_t PY = 0;
-  bool win_ok = rows_ok && win_allowed && build_windows(rb, win, PY, why);
-  if (win_ok && !agrees([&](int q, int32_t i) { return win_source(c->lattice, rb, win, PY, q, i); })) {
+  // row windows, checked link by link
+  WinBuild wb;
+  bool win_ok = rows_ok && win_allowed && build_windows(rb, true, wb, why);
+  if (win_ok && !agrees([&](int q, int32_t i) { return win_source(c->lattice, rb, wb, q, i); })) {
     win_ok = false;
     why = "row windows disagree with the neighbour index";
   }
@@ -546,13 +545,30 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
     c->addr.layout = 1;
     c->addr.rows = RowAddr{c->d_coord, c->d_rows, static_cast<uint32_t>(NP), rb.g};
     if (win_ok) {
-      if ((rc = dev_alloc(c, &c->d_win, win.size())) != LB_OK) return rc;
-      LB_HIP(c, hipMemcpy(c->d_win, win.data(), win.size() * sizeof(uint4), hipMemcpyHostToDevice));
-      c->addr.layout = 2;
-      c->addr.win = RowWin{c->d_coord, c->d_win, static_cast<uint32_t>(NP), PY, rb.g.W};
+      const size_t nw = wb.win.size(), np = wb.plane.size(), nc = wb.count.size();
+      if ((rc = dev_alloc(c, &c->d_win, nw + np + nc)) != LB_OK) return rc;
+      LB_HIP(c, hipMemcpy(c->d_win, wb.win.data(), nw * sizeof(uint32_t), hipMemcpyHostToDevice));
+      if (np) LB_HIP(c, hipMemcpy(c->d_win + nw, wb.plane.data(), np * sizeof(uint32_t), hipMemcpyHostToDevice));
+      if (nc) LB_HIP(c, hipMemcpy(c->d_win + nw + np, wb.count.data(), nc * sizeof(uint32_t), hipMemcpyHostToDevice));
+      auto set = [&](auto& w) {
+        w.coord = c->d_coord;
+        w.win = c->d_win;
+        w.plane = np ? c->d_win + nw : nullptr;
+        w.PY = wb.PY;
+        w.W = wb.W;
+      };
+      c->addr.layout = nc ? kLayWinZ : kLayWin;
+      if (nc) {
+        set(c->addr.winz);
+        c->addr.winz.count = c->d_win + nw + np;
+        c->addr.winz.EZ = wb.EZ;
+      } else {
+        set(c->addr.win);
+      }
     }
   }
-  c->layout_note = win_ok ? "row windows" : (rows_ok ? "rows (" + why + ")" : why);
+  c->layout_note = win_ok ? (c->addr.layout == kLayWinZ ? "rows (periodic along the row axis)" : "row windows")
+                          : (rows_ok ? "rows (" + why + ")" : why);
   c->n_blocks = (n_bulk + kBlock - 1) / kBlock;
   if (c->n_blocks == 0) c->n_blocks = 1;
   if ((rc = dev_alloc(c, &c->d_rho, 2 * NP)) != LB_OK) return rc;
@@ -672,7 +688,11 @@ int lb_set_topology_grid(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, co
   return setup_topology(c, n_nodes, neighbor, node_type, bulk, n_bulk, pos, flags);
 }
 
-int32_t lb_layout(const lb_ctx* c) { return c && c->has_topo ? c->addr.layout : -1; }
+int32_t lb_layout(const lb_ctx* c) {
+  if (!c || !c->has_topo) return -1;
+  // the windows of a box that is periodic along the row axis are a row layout
+  return c->addr.layout == kLayWinZ ? kLayRows : c->addr.layout;
+}
 
 const char* lb_layout_note(const lb_ctx* c) { return c ? c->layout_note.c_str() : "null context"; }
 
@@ -1314,32 +1334,34 @@ CgArgs cg_args(const lb_ctx* c, double tau0, double tau1, double sigma, double b
 
 // Row windows when every solid neighbour has one colour and both fields fit
 // the 32-bit byte offsets of that layout; else the link table.
-bool cg_rowwin(const lb_ctx* c) {
-  return c->addr.layout == 2 && c->wall_uniform &&
-         rowwin_fits(c->Q, c->NP, 2, static_cast<int64_t>(elem_size(c->precision)));
+int cg_layout(const lb_ctx* c) {
+  return c->addr.layout >= kLayWin && c->wall_uniform &&
+                 rowwin_fits(c->Q, c->NP, 2, static_cast<int64_t>(elem_size(c->precision)))
+             ? c->addr.layout
+             : kLayTable;
 }
 
 // The colour pass of the iteration at step_count: phi of every bulk node,
 // and with momx the per-block partial sums of the x-momentum.  The phi
 // buffer holds float values in the reduced-precision forms.
-hipError_t colour_pass(lb_ctx* c, bool rowwin, bool momx) {
+hipError_t colour_pass(lb_ctx* c, int layout, bool momx) {
   if (c->precision == LB_FP64)
-    return cg_phi_f64(c->lattice, !c->post, momx, static_cast<const double*>(c->d_f[c->cur]), c->addr, rowwin,
+    return cg_phi_f64(c->lattice, !c->post, momx, static_cast<const double*>(c->d_f[c->cur]), c->addr, layout,
                       c->n_bulk, c->NP, c->d_phi, c->d_partial, c->stream);
-  return cg_phi_lowp(c->precision, c->lattice, !c->post, momx, c->d_f[c->cur], c->addr, rowwin, c->n_bulk, c->NP,
+  return cg_phi_lowp(c->precision, c->lattice, !c->post, momx, c->d_f[c->cur], c->addr, layout, c->n_bulk, c->NP,
                      reinterpret_cast<float*>(c->d_phi), c->d_partial, c->stream);
 }
 
 // The collision pass of the same iteration; macroscopic fields stored when
 // `store`.  The caller then advances the state (advance_cg).
-hipError_t collision_pass(lb_ctx* c, bool rowwin, bool store, CgArgs a) {
+hipError_t collision_pass(lb_ctx* c, int layout, bool store, CgArgs a) {
   const WallPhi wp{c->d_phi_wall, c->wall_phi};
   if (c->precision == LB_FP64)
     return cg_f64(c->lattice, !c->post, store, static_cast<const double*>(c->d_f[c->cur]),
-                  static_cast<double*>(c->d_f[1 - c->cur]), c->addr, rowwin, c->n_bulk, c->NP, a, c->d_phi, wp,
+                  static_cast<double*>(c->d_f[1 - c->cur]), c->addr, layout, c->n_bulk, c->NP, a, c->d_phi, wp,
                   c->d_scalar, c->d_rho, c->d_vel, c->stream);
   a.step = c->step_count;
-  return cg_lowp(c->precision, c->lattice, !c->post, store, c->d_f[c->cur], c->d_f[1 - c->cur], c->addr, rowwin,
+  return cg_lowp(c->precision, c->lattice, !c->post, store, c->d_f[c->cur], c->d_f[1 - c->cur], c->addr, layout,
                  c->n_bulk, c->NP, a, reinterpret_cast<const float*>(c->d_phi), wp, c->d_scalar, c->d_rho, c->d_vel,
                  c->stream);
 }
@@ -1378,14 +1400,14 @@ int lb_step_cg(lb_ctx* c, int32_t nsteps, double tau0, double tau1, double sigma
   hipSetDevice(c->device);
   const CgArgs a = cg_args(c, tau0, tau1, sigma, beta, force_mode, force);
   const bool momx = a.momx_mode != 0;
-  const bool rowwin = cg_rowwin(c);
+  const int layout = cg_layout(c);
   Timer t(c);
   int64_t launches = 0;
   for (int32_t s = 0; s < nsteps; ++s) {
-    hipError_t e = colour_pass(c, rowwin, momx);
+    hipError_t e = colour_pass(c, layout, momx);
     if (e == hipSuccess && momx)
       e = finish_momx(c->d_partial, c->n_blocks, a.momx, c->n_global, c->d_scalar, c->stream);
-    if (e == hipSuccess) e = collision_pass(c, rowwin, s == nsteps - 1, a);
+    if (e == hipSuccess) e = collision_pass(c, layout, s == nsteps - 1, a);
     if (e != hipSuccess) return fail(c, LB_ERR_HIP, "two-phase launch: %s", hipGetErrorString(e));
     launches += momx ? 3 : 2;
     advance_cg(c);
@@ -1409,7 +1431,7 @@ int lb_step_cg_colour(lb_ctx* c, double* flux_x) {
   hipSetDevice(c->device);
   const bool momx = flux_x != nullptr;
   Timer t(c);
-  hipError_t e = colour_pass(c, cg_rowwin(c), momx);
+  hipError_t e = colour_pass(c, cg_layout(c), momx);
   // the block partials summed as the momentum-controlled step sums them
   // (slot 1 of the scalar buffer; slot 0 receives -2 sum, unused)
   if (e == hipSuccess && momx) e = finish_momx(c->d_partial, c->n_blocks, 0.0, 1, c->d_scalar, c->stream);
@@ -1438,7 +1460,7 @@ int lb_step_cg_collide(lb_ctx* c, double tau0, double tau1, double sigma, double
     a.momx_mode = 0;
   }
   Timer t(c);
-  hipError_t e = collision_pass(c, cg_rowwin(c), true, a);
+  hipError_t e = collision_pass(c, cg_layout(c), true, a);
   if (e != hipSuccess) return fail(c, LB_ERR_HIP, "two-phase launch: %s", hipGetErrorString(e));
   advance_cg(c);
   rc = t.stop(1);

@@ -83,7 +83,8 @@ constexpr int kBgk = 0, kTrt = 1, kRheology = 2;
 // at even global steps.
 struct BatchSolve {
   const uint32_t* coord;
-  const uint4* win;
+  const uint32_t* win;    // row windows (RowWin): words,
+  const uint32_t* plane;  // and the first nodes of the x planes, or null
   void* f[2];
   double* partial;  // [ncomp][blocks]: 1 component single-phase, 3 two-phase
   void* phi;        // two-phase colour field (NP; float, double in FP64), null for single-phase

@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk_lp(const BatchSolve* 
     const bool act = it < end && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
-    const RowWin ad{s.coord, s.win, s.NP, s.PY, s.W};
+    const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     // the running sum of this block over the interval, read before the node
     // work so that its latency overlaps the gathers
@@ -685,7 +685,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi_lp(const BatchSolv
     const bool act = it < end && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
-    const RowWin ad{s.coord, s.win, s.NP, s.PY, s.W};
+    const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     if (act && i < s.n) {
@@ -730,7 +730,7 @@ __global__ __launch_bounds__(kBlock * NS, 4) void k_batch_cg_lp(const BatchSolve
     if (!s.live) continue;  // stopped at an earlier check of this launch sequence
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
-    const RowWin ad{s.coord, s.win, s.NP, s.PY, s.W};
+    const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     if (i >= s.n) continue;
     double t[Q], dd[Q];
@@ -815,8 +815,9 @@ inline dim3 grid_for(int32_t n) { return dim3(static_cast<unsigned>((n + kBlock 
 template <typename F>
 hipError_t dispatch(int precision, int lattice, const Addr& ad, F&& f) {
   auto by_addr = [&](auto l, auto st) {
-    if (ad.layout == 2) f(l, st, ad.win);
-    else if (ad.layout == 1) f(l, st, ad.rows);
+    if (ad.layout == kLayWin) f(l, st, ad.win);
+    else if (ad.layout == kLayWinZ) f(l, st, ad.winz);
+    else if (ad.layout == kLayRows) f(l, st, ad.rows);
     else f(l, st, ad.table);
   };
   if (lattice == 0) {
@@ -980,10 +981,10 @@ hipError_t batch_cg_lowp(int precision, int lattice, bool reduce, const BatchSol
 }
 
 hipError_t cg_phi_lowp(int precision, int lattice, bool first, bool momx, const void* gin, const Addr& ad,
-                       bool rowwin, int32_t n, int64_t NP, float* phi, double* partial, hipStream_t s) {
+                       int layout, int32_t n, int64_t NP, float* phi, double* partial, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   Addr sel = ad;
-  sel.layout = rowwin ? 2 : 0;
+  sel.layout = layout;
   return dispatch(precision, lattice, sel, [&](auto l, auto st, auto addr) {
     using L = decltype(l);
     using S = decltype(st);
@@ -1005,14 +1006,14 @@ hipError_t cg_phi_lowp(int precision, int lattice, bool first, bool momx, const 
 }
 
 hipError_t cg_lowp(int precision, int lattice, bool first, bool store, const void* gin, void* gout, const Addr& ad,
-                   bool rowwin, int32_t n, int64_t NP, const CgArgs& a, const float* phi, const WallPhi& wp,
+                   int layout, int32_t n, int64_t NP, const CgArgs& a, const float* phi, const WallPhi& wp,
                    const double* dscalar, double* rho, double* vel, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (a.q0 != 0.0 || a.q1 != 0.0) return hipErrorInvalidValue;  // no mass sources in this form
   const double n0 = a.nu0Inv, n1 = a.nu1Inv, sg = a.sigma, be = a.beta;
   const double F0 = a.F[0], F1 = a.F[1], F2 = a.F[2];
   Addr sel = ad;
-  sel.layout = rowwin ? 2 : 0;
+  sel.layout = layout;
   return dispatch(precision, lattice, sel, [&](auto l, auto st, auto addr) {
     using L = decltype(l);
     using S = decltype(st);

@@ -49,11 +49,11 @@ hipError_t batch_cg_lowp(int precision, int lattice, bool reduce, const BatchSol
                          int32_t n_items, int32_t grid, int32_t per_wg, int32_t parity, const uint32_t* step0,
                          int32_t koff, int ns, hipStream_t s);
 // Two-phase populations are stored as (t, d) = (f0 + f1 - w, f0 - f1).
-// rowwin: the row windows of ad with one wall colour, else the link table.
+// layout: row windows with one wall colour, or the link table.
 hipError_t cg_phi_lowp(int precision, int lattice, bool first, bool momx, const void* gin, const Addr& ad,
-                       bool rowwin, int32_t n, int64_t NP, float* phi, double* partial, hipStream_t s);
+                       int layout, int32_t n, int64_t NP, float* phi, double* partial, hipStream_t s);
 hipError_t cg_lowp(int precision, int lattice, bool first, bool store, const void* gin, void* gout, const Addr& ad,
-                   bool rowwin, int32_t n, int64_t NP, const CgArgs& a, const float* phi, const WallPhi& wp,
+                   int layout, int32_t n, int64_t NP, const CgArgs& a, const float* phi, const WallPhi& wp,
                    const double* dscalar, double* rho, double* vel, hipStream_t s);
 
 }  // namespace lbamd

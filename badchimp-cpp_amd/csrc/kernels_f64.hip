@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk(const BatchSolve* __r
     const bool act = it < end && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
-    const RowWin ad{s.coord, s.win, s.NP, s.PY, s.W};
+    const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     // the running sum of this block over the interval, read before the node
     // work so that its latency overlaps the gathers
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi(const BatchSolve* 
     const bool act = it < end && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
-    const RowWin ad{s.coord, s.win, s.NP, s.PY, s.W};
+    const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     if (act && i < s.n) {
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg(const BatchSolve* __re
     if (!s.live) continue;  // stopped at an earlier check of this launch sequence
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
-    const RowWin ad{s.coord, s.win, s.NP, s.PY, s.W};
+    const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     if (i >= s.n) continue;
     CgArgs a{};
@@ -845,16 +845,18 @@ hipError_t bgk_f64(int lattice, bool first, bool store, bool reduce, const doubl
   if (n <= 0) return hipSuccess;
   const dim3 g = grid_for(n);
   LB_DISPATCH_LATTICE(lattice, L, {
-    if (ad.layout == 2)
+    if (ad.layout == kLayWin)
       launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.win, n, NP, a, rho, vel, partial, accum);
-    else if (ad.layout == 1)
+    else if (ad.layout == kLayWinZ)
+      launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.winz, n, NP, a, rho, vel, partial, accum);
+    else if (ad.layout == kLayRows)
       launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.rows, n, NP, a, rho, vel, partial, accum);
     else launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.table, n, NP, a, rho, vel, partial, accum);
   });
   return hipGetLastError();
 }
 
-hipError_t cg_phi_f64(int lattice, bool first, bool momx, const double* fin, const Addr& ad, bool rowwin,
+hipError_t cg_phi_f64(int lattice, bool first, bool momx, const double* fin, const Addr& ad, int layout,
                       int32_t n, int64_t NP, double* phi, double* partial, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const dim3 g = grid_for(n), b(kBlock);
@@ -867,13 +869,14 @@ hipError_t cg_phi_f64(int lattice, bool first, bool momx, const double* fin, con
       else k_cg_phi<L, false, false, A><<<g, b, 0, s>>>(fin, addr, n, NP, phi, partial);
     });
   };
-  if (rowwin) go(ad.win);
+  if (layout == kLayWin) go(ad.win);
+  else if (layout == kLayWinZ) go(ad.winz);
   else go(ad.table);
   return hipGetLastError();
 }
 
 hipError_t cg_f64(int lattice, bool first, bool store, const double* fin, double* fout, const Addr& ad,
-                  bool rowwin, int32_t n, int64_t NP, const CgArgs& a, const double* phi, const WallPhi& wp,
+                  int layout, int32_t n, int64_t NP, const CgArgs& a, const double* phi, const WallPhi& wp,
                   const double* dscalar, double* rho, double* vel, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const dim3 g = grid_for(n), b(kBlock);
@@ -886,7 +889,8 @@ hipError_t cg_f64(int lattice, bool first, bool store, const double* fin, double
       else k_cg<L, false, false, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
     });
   };
-  if (rowwin) go(ad.win);
+  if (layout == kLayWin) go(ad.win);
+  else if (layout == kLayWinZ) go(ad.winz);
   else go(ad.table);
   return hipGetLastError();
 }
@@ -895,8 +899,9 @@ hipError_t gather_f64(int lattice, int nfields, const double* fin, double* fout,
                       const Addr& ad, int32_t n, int64_t NP, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   LB_DISPATCH_LATTICE(lattice, L, {
-    if (ad.layout == 2) k_gather<L, RowWin><<<grid_for(n), dim3(kBlock), 0, s>>>(fin, fout, ad.win, n, NP, nfields);
-    else if (ad.layout == 1) k_gather<L, RowAddr><<<grid_for(n), dim3(kBlock), 0, s>>>(fin, fout, ad.rows, n, NP, nfields);
+    if (ad.layout == kLayWin) k_gather<L, RowWin><<<grid_for(n), dim3(kBlock), 0, s>>>(fin, fout, ad.win, n, NP, nfields);
+    else if (ad.layout == kLayWinZ) k_gather<L, RowWinZ><<<grid_for(n), dim3(kBlock), 0, s>>>(fin, fout, ad.winz, n, NP, nfields);
+    else if (ad.layout == kLayRows) k_gather<L, RowAddr><<<grid_for(n), dim3(kBlock), 0, s>>>(fin, fout, ad.rows, n, NP, nfields);
     else k_gather<L, TableAddr><<<grid_for(n), dim3(kBlock), 0, s>>>(fin, fout, ad.table, n, NP, nfields);
   });
   return hipGetLastError();
@@ -922,8 +927,9 @@ hipError_t flux_f64(int lattice, int nfields, bool first, const double* fin, con
   LB_DISPATCH_LATTICE(lattice, L, {
     // two fields may not fit the row windows' 32-bit offsets
     const int lay = launch_layout(ad.layout, L::nQ, NP, nfields, sizeof(double));
-    if (lay == 2) launch_flux<L>(nfields, first, g, s, fin, ad.win, n, NP, dir, partial, nb);
-    else if (lay == 1) launch_flux<L>(nfields, first, g, s, fin, ad.rows, n, NP, dir, partial, nb);
+    if (lay == kLayWin) launch_flux<L>(nfields, first, g, s, fin, ad.win, n, NP, dir, partial, nb);
+    else if (lay == kLayWinZ) launch_flux<L>(nfields, first, g, s, fin, ad.winz, n, NP, dir, partial, nb);
+    else if (lay == kLayRows) launch_flux<L>(nfields, first, g, s, fin, ad.rows, n, NP, dir, partial, nb);
     else launch_flux<L>(nfields, first, g, s, fin, ad.table, n, NP, dir, partial, nb);
   });
   return hipGetLastError();

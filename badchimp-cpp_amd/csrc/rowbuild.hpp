@@ -114,78 +114,104 @@ inline bool rows_from_geometry(int lattice, const int32_t* dims, const int32_t* 
   return true;
 }
 
-// Row windows (addressing.hpp, RowWin): for the halo-padded row (X+1, Y+1)
-// and word w, the fluid bits of cells [32w-16, 32w+48) and the compact index
-// of the first fluid cell at or after 32w-16.  Halo rows of a periodic axis
-// repeat the rows they wrap to; those of a closed axis stay empty.  Needs a
-// box that is not periodic along the row axis.
-inline bool build_windows(const RowBuild& rb, std::vector<uint4>& win, int32_t& PY, std::string& why) {
+// Row windows (addressing.hpp, RowWin and RowWinZ): for the halo-padded row
+// (X+1, Y+1) and word w, the compact index of the first fluid cell at or after
+// 8w (from node 0, or from the first node of the x plane) and the fluid bits
+// of cells 8w-1 .. 8w+8.  Halo rows of a periodic axis repeat the rows they
+// wrap to; those of a closed axis stay empty.
+struct WinBuild {
+  std::vector<uint32_t> win;
+  std::vector<uint32_t> plane;  // first node of each padded X; empty: bases from node 0
+  std::vector<uint32_t> count;  // fluid cells of each padded row (box periodic along the row axis)
+  int32_t PY = 0, W = 0, EZ = 0;
+};
+
+// planes: bases from the first node of the x plane also where the node list
+// fits without (for tests).
+inline bool build_windows(const RowBuild& rb, bool allow_periodic, WinBuild& wb, std::string& why,
+                          bool planes = false) {
   const RowGeom& g = rb.g;
-  if (g.periodic & 4) {
+  const bool pz = (g.periodic & 4) != 0;
+  if (pz && !allow_periodic) {
     why = "periodic along the row axis";
     return false;
   }
-  const int32_t PX = g.E[0] + 2;
-  PY = g.E[1] + 2;
-  win.assign(static_cast<size_t>(PX) * PY * g.W, uint4{0u, 0u, 0u, 0u});
-  auto first_at_or_after = [&](size_t r, int32_t z) -> uint32_t {
-    // compact index of the first fluid cell of row r at or after z (or the
-    // index one past the row's last fluid cell)
-    const int32_t zc = std::max(z, 0);
-    if (zc >= 32 * g.W) {
-      const uint2 e = rb.rows[r * g.W + g.W - 1];
-      return e.x + static_cast<uint32_t>(__builtin_popcount(e.y));
-    }
-    const uint2 e = rb.rows[r * g.W + (zc >> 5)];
-    return e.x + static_cast<uint32_t>(__builtin_popcount(e.y & ((1u << (zc & 31)) - 1u)));
-  };
-  for (int32_t px = 0; px < PX; ++px)
-    for (int32_t py = 0; py < PY; ++py) {
-      int32_t X = px - 1, Y = py - 1;
-      bool inside = RowGeom::wrap(X, g.E[0], g.periodic & 1);
-      inside = RowGeom::wrap(Y, g.E[1], g.periodic & 2) && inside;
-      if (!inside) continue;
-      const size_t r = static_cast<size_t>(g.row(X, Y));
-      const uint2* words = &rb.rows[r * g.W];
-      for (int32_t w = 0; w < g.W; ++w) {
-        // cells 32w - 16 .. 32w + 47 of the row: the upper half of word
-        // w - 1, word w, the lower half of word w + 1 (no cells before z = 0
-        // or after the row's last word; a word holds no bits beyond E_Z)
-        const uint64_t prev = w > 0 ? words[w - 1].y : 0u;
-        const uint64_t cur = words[w].y;
-        const uint64_t next = w + 1 < g.W ? words[w + 1].y : 0u;
-        const uint64_t m = (prev >> 16) | (cur << 16) | (next << 48);
-        win[(static_cast<size_t>(px) * PY + py) * g.W + w] =
-            uint4{first_at_or_after(r, 32 * w - 16), static_cast<uint32_t>(m), static_cast<uint32_t>(m >> 32), 0u};
+  constexpr uint32_t kMax = 1u << kWinBase;
+  const int32_t PX = g.E[0] + 2, EZ = g.E[2];
+  wb.PY = g.E[1] + 2;
+  wb.W = win_words(EZ);
+  wb.EZ = EZ;
+  wb.win.assign(static_cast<size_t>(PX) * wb.PY * wb.W, 0u);
+  wb.count.assign(pz ? static_cast<size_t>(PX) * wb.PY : 0u, 0u);
+  wb.plane.assign(planes || rb.coord.size() >= kMax ? static_cast<size_t>(PX) : 0u, 0u);
+  for (int32_t px = 0; px < PX; ++px) {
+    int32_t X = px - 1;
+    if (!RowGeom::wrap(X, g.E[0], g.periodic & 1)) continue;
+    // the nodes of a plane are consecutive (one plane per tile along X)
+    static_assert(kTileLogX == 0, "x planes are not consecutive in the compact order");
+    const uint32_t base = wb.plane.empty() ? 0u : rb.rows[static_cast<size_t>(g.row(X, 0)) * g.W].x;
+    if (!wb.plane.empty()) wb.plane[px] = base;
+    for (int32_t py = 0; py < wb.PY; ++py) {
+      int32_t Y = py - 1;
+      if (!RowGeom::wrap(Y, g.E[1], g.periodic & 2)) continue;
+      const uint2* words = &rb.rows[static_cast<size_t>(g.row(X, Y)) * g.W];  // 32 cells each, no bits beyond E_Z
+      const size_t pr = static_cast<size_t>(px) * wb.PY + py;
+      auto cell = [&](int32_t z) -> uint32_t {
+        if (pz) z = z < 0 ? z + EZ : (z >= EZ ? z - EZ : z);
+        return z < 0 || z >= EZ ? 0u : (words[z >> 5].y >> (z & 31)) & 1u;
+      };
+      for (int32_t w = 0; w < wb.W; ++w) {
+        const int32_t z0 = w << kWinLog, h = z0 & 31;
+        const uint2 e = words[z0 >> 5];
+        const uint32_t first = e.x + static_cast<uint32_t>(__builtin_popcount(e.y & ((1u << h) - 1u))) - base;
+        if (first >= kMax) {
+          why = "x plane above 2^22 nodes";
+          return false;
+        }
+        // cells 8w .. 8w+7 lie in one 32-cell word; the two beside them by cell
+        uint32_t bits = ((e.y >> h) & ((1u << kWinCells) - 1u)) << 1;
+        bits |= cell(z0 - 1);
+        const int32_t end = z0 + static_cast<int32_t>(kWinCells);
+        if (end <= EZ) {
+          bits |= cell(end) << (kWinCells + 1);
+        } else {
+          // the row ends inside the word: the cell after the last one wraps
+          bits |= cell(EZ) << (EZ - z0 + 1);
+        }
+        wb.win[pr * wb.W + w] = (bits << kWinBase) | first;
+      }
+      if (pz) {
+        const uint2 last = words[g.W - 1];
+        wb.count[pr] = last.x + static_cast<uint32_t>(__builtin_popcount(last.y)) - words[0].x;
       }
     }
+  }
   return true;
 }
 
-// Source of direction q for compact node i under the row windows, as RowWin
-// computes it on the device.
-inline std::pair<bool, int64_t> win_source(int lattice, const RowBuild& rb, const std::vector<uint4>& win, int32_t PY,
-                                    int q, int32_t i) {
-  const int nD = lattice == LB_D2Q9 ? 2 : 3;
-  auto C = [&](int a) -> int {
-    const int d = nD == 3 ? a : (a == 0 ? 0 : (a == 2 ? 1 : -1));
-    if (d < 0) return 0;
-    return lattice == LB_D2Q9 ? D2Q9::c(q, d) : D3Q19::c(q, d);
-  };
-  const RowGeom& g = rb.g;
+// The cell (dx, dy, dz) off compact node i's under the row windows, as RowWin
+// and RowWinZ find it on the device: {fluid, compact index}, or {false, i}.
+inline std::pair<bool, int64_t> win_cell(const RowBuild& rb, const WinBuild& wb, int32_t i, int dx, int dy, int dz) {
   const uint32_t cc = rb.coord[i];
   const int32_t X = static_cast<int32_t>(cc >> 22), Y = static_cast<int32_t>((cc >> 12) & 1023u),
                 Z = static_cast<int32_t>(cc & 4095u);
-  const int32_t w = Z >> 5;
-  const uint32_t t = static_cast<uint32_t>(Z - 32 * w + 16);
-  const size_t slot = (static_cast<size_t>(X + 1 - C(0)) * PY + (Y + 1 - C(1))) * g.W + w;
-  const uint4 e = win[slot];
-  const uint64_t m = (static_cast<uint64_t>(e.z) << 32) | e.y;
-  const int64_t b0 = static_cast<int64_t>(e.x) + __builtin_popcountll(m & ((1ull << t) - 1ull));
-  const uint32_t bm = static_cast<uint32_t>(m >> (t - 1)) & 7u;
-  const int dz = -C(2);
-  if (!((bm >> (dz + 1)) & 1u)) return {false, i};
-  return {true, dz == 0 ? b0 : (dz < 0 ? b0 - 1 : b0 + ((bm >> 1) & 1u))};
+  const uint32_t t = kWinBase + (static_cast<uint32_t>(Z) & (kWinCells - 1u));
+  const size_t pr = static_cast<size_t>(X + 1 + dx) * wb.PY + (Y + 1 + dy);
+  const uint32_t m = wb.win[pr * wb.W + (Z >> kWinLog)];
+  const uint32_t below = (2u << t) - (2u << kWinBase);
+  const uint32_t b0 = (m & ((1u << kWinBase) - 1u)) + static_cast<uint32_t>(__builtin_popcount(m & below)) +
+                      (wb.plane.empty() ? 0u : wb.plane[X + 1 + dx]);
+  if (!((m >> (t + 1 + dz)) & 1u)) return {false, i};
+  const uint32_t n = wb.count.empty() ? 0u : wb.count[pr];
+  if (dz == 0) return {true, static_cast<int64_t>(b0)};
+  if (dz < 0) return {true, static_cast<int64_t>(b0 - 1u + (Z == 0 ? n : 0u))};
+  return {true, static_cast<int64_t>(b0 + ((m >> (t + 1u)) & 1u) - (Z == wb.EZ - 1 ? n : 0u))};
+}
+
+// Source of direction q for compact node i under the row windows.
+inline std::pair<bool, int64_t> win_source(int lattice, const RowBuild& rb, const WinBuild& wb, int q, int32_t i) {
+  if (lattice == LB_D2Q9) return win_cell(rb, wb, i, -D2Q9::c(q, 0), 0, -D2Q9::c(q, 1));
+  return win_cell(rb, wb, i, -D3Q19::c(q, 0), -D3Q19::c(q, 1), -D3Q19::c(q, 2));
 }
 
 
