@@ -41,7 +41,7 @@
 //            entries over 32 cells a step takes, on the 256^3 pack, 127 us for
 //            142 (FP16S), 187 for 192 (FP32S) and 350 as before (FP64, bound
 //            by the memory); on a 161 x 143 x 150 pack 26.8 for 30.1 (FP16S).
-//            The struct stays at 32 bytes: 48 bytes of it made the step of the
+//            The struct is kept small: 16 bytes more made the step of the
 //            256 x 128 channel 4 % slower, which waits for its arguments.
 // RowWinZ    RowWin for boxes that are periodic along the row axis: the bits of
 //            the first and the last word wrap, and the nodes at z = 0 and
@@ -85,11 +85,25 @@ __device__ __forceinline__ int32_t node_block(int32_t b, int32_t nb) {
 // MALL.  The two-phase collision pass runs this way after the colour pass.
 __device__ __forceinline__ int32_t node_block_rev(int32_t b, int32_t nb) { return node_block(nb - 1 - b, nb); }
 
+// Block of workgroup wg of nb: the layout's block order where it has one
+// (block_order in rowbuild.hpp), else node_block.
+template <class A>
+__device__ __forceinline__ int32_t block_of(const A& ad, int32_t wg, int32_t nb) {
+  if constexpr (A::kOrdered) {
+    if (ad.order) return ad.order[wg];
+  }
+  return node_block(wg, nb);
+}
+template <class A>
+__device__ __forceinline__ int32_t block_of_rev(const A& ad, int32_t wg, int32_t nb) {
+  return block_of(ad, nb - 1 - wg, nb);
+}
+
 // Element indices are 32-bit: a context keeps Q * NP * fields below 2^32.
 // kOff32: the layout is only used for population buffers below 4 GiB, so the
 // kernels may address them with 32-bit byte offsets from the buffer base.
 struct TableAddr {
-  static constexpr bool kOff32 = false;
+  static constexpr bool kOff32 = false, kOrdered = false;
   const uint32_t* __restrict__ link;
   uint32_t NP;
   template <class L>
@@ -145,7 +159,7 @@ template <class L>
 __host__ __device__ __forceinline__ constexpr int cz(int q) { return L::nD == 3 ? L::c(q, 2) : L::c(q, 1); }
 
 struct RowAddr {
-  static constexpr bool kOff32 = false;
+  static constexpr bool kOff32 = false, kOrdered = false;
   const uint32_t* __restrict__ coord;  // X << 22 | Y << 12 | Z
   const uint2* __restrict__ rows;      // {base, mask} per (row, word)
   uint32_t NP;
@@ -187,12 +201,13 @@ struct WinWrap<true> {
 };
 template <bool PZ>
 struct RowWinT : WinWrap<PZ> {
-  static constexpr bool kOff32 = true;
+  static constexpr bool kOff32 = true, kOrdered = true;
   const uint32_t* __restrict__ coord;  // X << 22 | Y << 12 | Z
   const uint32_t* __restrict__ win;    // fluid bits << kWinBase | base, per (padded row, word)
   const uint32_t* __restrict__ plane;  // first node of each padded X; null: the bases count from node 0
   int32_t PY;  // padded rows along Y: E_Y + 2
   int32_t W;   // words per row (win_words)
+  const int32_t* __restrict__ order = nullptr;  // block order, or null
 
   // What a node reads of its 9 (D3Q19) or 3 (D2Q9) neighbouring rows: the
   // words, and the index of the first fluid cell at or after z.
@@ -288,7 +303,7 @@ using RowWinZ = RowWinT<true>;
 
 // Windows of a batched solve.
 __host__ __device__ __forceinline__ RowWin solve_windows(const BatchSolve& s) {
-  return RowWin{{}, s.coord, s.win, s.plane, s.PY, s.W};
+  return RowWin{{}, s.coord, s.win, s.plane, s.PY, s.W, nullptr};
 }
 
 // The source node of every direction: bit q of fluid is set when the source

@@ -146,6 +146,12 @@ int alloc_fields(lb_ctx* c, int nf) {
     c->bytes += static_cast<int64_t>(bytes);
   }
   c->n_fields = nf;
+  // Block order of the row windows.  Measured (order against node_block, us per
+  // step): FP32S 128^3 26.1 / 27.3, 165^3 50.9 / 52.9, 256^3 187 / 188; FP64
+  // 64^3 9.7 / 10.4, 128^3 47.6 / 49.0, 256^3 358 / 351 (1.0 GB per buffer,
+  // bound by the HBM, which the wider front serves less well); two-phase
+  // FP64 192^3 439 / 453 (0.8 GB per buffer), FP32S 222 / 239.
+  c->addr.win.order = c->addr.winz.order = nf == 1 && bytes > (size_t{900} << 20) ? nullptr : c->d_order;
   c->cur = 0;
   c->post = false;
   c->step_count = 0;
@@ -523,8 +529,10 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
   free_halos(c);
   c->n_ghost = 0;
   c->slot_of.clear();
-  for (void* p : {static_cast<void*>(c->d_coord), static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win)})
+  for (void* p : {static_cast<void*>(c->d_coord), static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win),
+                  static_cast<void*>(c->d_order)})
     if (p) hipFree(p);
+  c->d_order = nullptr;
   c->d_coord = nullptr;
   c->d_rows = nullptr;
   c->d_win = nullptr;
@@ -557,6 +565,11 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
         w.PY = wb.PY;
         w.W = wb.W;
       };
+      const std::vector<int32_t> order = block_order(rb.coord);
+      if (!order.empty()) {
+        if ((rc = dev_alloc(c, &c->d_order, order.size())) != LB_OK) return rc;
+        LB_HIP(c, hipMemcpy(c->d_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+      }
       c->addr.layout = nc ? kLayWinZ : kLayWin;
       if (nc) {
         set(c->addr.winz);
@@ -666,7 +679,7 @@ int lb_ctx_destroy(lb_ctx* c) {
                   static_cast<void*>(c->d_phi), static_cast<void*>(c->d_phi_wall), static_cast<void*>(c->d_partial),
                   static_cast<void*>(c->d_scalar), static_cast<void*>(c->d_coord),
                   static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win), static_cast<void*>(c->d_table),
-                  static_cast<void*>(c->d_rank)})
+                  static_cast<void*>(c->d_rank), static_cast<void*>(c->d_order)})
     if (p) hipFree(p);
   hipEventDestroy(c->ev0);
   hipEventDestroy(c->ev1);

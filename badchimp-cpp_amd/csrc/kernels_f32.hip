@@ -328,7 +328,7 @@ __global__ __launch_bounds__(kBlock) void k_bgk_lp(const S* __restrict__ gin, S*
                                                    float tauA_factor, const float* __restrict__ sr,
                                                    const float* __restrict__ nu, int tab_n, uint32_t step,
                                                    int32_t accum) {
-  const int32_t b = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   // the block's running sum, read before the node work (latency overlapped)
   const double prev = REDUCE && accum && threadIdx.x == 0 ? partial[b] : 0.0;
@@ -628,7 +628,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_phi_lp(const S* __restrict__ gin,
                                                       int64_t NP, float* __restrict__ phi,
                                                       double* __restrict__ partial) {
   constexpr int Q = L::nQ;
-  const int32_t b = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   double mx = 0.0;
   if (i < n) {
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_lp(const S* __restrict__ gin, S* 
                                                   double* __restrict__ rho_o, double* __restrict__ vel_o,
                                                   uint32_t step) {
   constexpr int Q = L::nQ;
-  const int32_t b = node_block_rev(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of_rev(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   if (i >= n) return;
   double t[Q], dd[Q];

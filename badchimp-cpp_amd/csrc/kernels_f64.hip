@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
                                                 int64_t NP, BgkArgs a, double* __restrict__ rho_o,
                                                 double* __restrict__ vel_o,
                                                 double* __restrict__ partial, int32_t accum) {
-  const int32_t b = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   // the block's running sum, read before the node work (latency overlapped)
   const double prev = REDUCE && accum && threadIdx.x == 0 ? partial[b] : 0.0;
@@ -392,7 +392,7 @@ template <class L, bool FIRST>
 __global__ __launch_bounds__(kBlock) void k_tag_mass(const double* __restrict__ fin, TableAddr ad, int32_t n,
                                                      int64_t NP, const uint32_t* __restrict__ info, int n_label,
                                                      double* __restrict__ partial) {
-  const int32_t b = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   double v = 0.0;
   int lab = 0;
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_phi(const double* __restrict__ fi
                                                    int32_t n, int64_t NP, double* __restrict__ phi,
                                                    double* __restrict__ partial) {
   constexpr int Q = L::nQ;
-  const int32_t b = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   double mx = 0.0;
   if (i < n) {
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(kBlock) void k_cg(const double* __restrict__ fin,
                                                double* __restrict__ rho_o,
                                                double* __restrict__ vel_o) {
   constexpr int D = L::nD;
-  const int32_t b = node_block_rev(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+  const int32_t b = block_of_rev(ad, static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t i = b * kBlock + threadIdx.x;
   if (i >= n) return;
   double F[D];
