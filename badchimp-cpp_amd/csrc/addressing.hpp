@@ -371,6 +371,14 @@ __device__ __forceinline__ T ld_elem(const T* __restrict__ base, uint32_t e) {
   if (OFF32) return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + e * static_cast<uint32_t>(sizeof(T)));
   return base[e];
 }
+// Store of a population.  NT (streaming): the line leaves the L2 and takes no
+// place in the MALL, for buffers that the MALL does not hold anyway; else the
+// next step finds it there (stream_stores in layout_select.hpp).
+template <bool NT, typename T>
+__device__ __forceinline__ void st_elem(T v, T* p) {
+  if (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
 template <bool OFF32, typename T>
 __device__ __forceinline__ T* elem_ptr(T* __restrict__ base, uint32_t e) {
   if (OFF32) return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + e * static_cast<uint32_t>(sizeof(T)));

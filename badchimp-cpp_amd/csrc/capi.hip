@@ -152,6 +152,7 @@ int alloc_fields(lb_ctx* c, int nf) {
   // bound by the HBM, which the wider front serves less well); two-phase
   // FP64 192^3 439 / 453 (0.8 GB per buffer), FP32S 222 / 239.
   c->addr.win.order = c->addr.winz.order = nf == 1 && bytes > (size_t{900} << 20) ? nullptr : c->d_order;
+  c->addr.nt = stream_stores(2 * static_cast<int64_t>(bytes));
   c->cur = 0;
   c->post = false;
   c->step_count = 0;

@@ -17,6 +17,7 @@ struct Addr {
   RowAddr rows{};
   RowWin win{};
   RowWinZ winz{};
+  bool nt = true;  // streaming stores (stream_stores)
 };
 
 // ---- FP64 (reference arithmetic, -ffp-contract=off) ----------------------

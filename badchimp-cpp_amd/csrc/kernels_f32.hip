@@ -219,7 +219,7 @@ __device__ __forceinline__ float rheology_visc_lp(const float (&g)[L::nQ], float
 // tauAnti_factor = tauA_factor; tau_inv, tau_factor are then the symmetric
 // ones.  MODE kRheology: tau_inv, tau_factor from the node's viscosity
 // (table sr/nu of n rows), stored beside rho (rho_o[NP + i]) when STORE.
-template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk>
+template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
 __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __restrict__ gout, const A& ad,
                                               int32_t i, int64_t NP, float tau_inv, float tau_factor,
                                               const float (&F)[3], double* __restrict__ rho_o,
@@ -281,14 +281,14 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
       const float ga = 0.5f * (g[q] - g[rq]);
       const float sym = omt * gs + (w * tau_inv) * (a0 + r45 * cu * cu) + (w * tau_factor) * (9.0f * cF * cu + m3uF);
       const float anti = oma * ga + (w * tauA_inv) * (r3 * cu) + (w * tauA_factor) * (3.0f * cF);
-      __builtin_nontemporal_store(Store<S>::put_sr(sym + anti, sr_bits(hn, q)), out + (q << kPLog));
-      __builtin_nontemporal_store(Store<S>::put_sr(sym - anti, sr_bits(hn, rq)), out + (rq << kPLog));
+      st_elem<NT>(Store<S>::put_sr(sym + anti, sr_bits(hn, q)), out + (q << kPLog));
+      st_elem<NT>(Store<S>::put_sr(sym - anti, sr_bits(hn, rq)), out + (rq << kPLog));
     }
     {
       constexpr int q = Q - 1;  // rest: even only
       const float w = float(L::w(q));
       const float gq = omt * g[q] + (w * tau_inv) * a0 + (w * tau_factor) * m3uF;
-      __builtin_nontemporal_store(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
+      st_elem<NT>(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
     }
     return REDUCE ? static_cast<double>(jd[0]) : 0.0;
   }
@@ -306,19 +306,19 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
     const float fod = 3.0f * cF;
     const float gq = omt * g[q] + wt * (ev + od) + wf * (fev + fod);
     const float gr = omt * g[rq] + wt * (ev - od) + wf * (fev - fod);
-    __builtin_nontemporal_store(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
-    __builtin_nontemporal_store(Store<S>::put_sr(gr, sr_bits(hn, rq)), out + (rq << kPLog));
+    st_elem<NT>(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
+    st_elem<NT>(Store<S>::put_sr(gr, sr_bits(hn, rq)), out + (rq << kPLog));
   }
   {
     constexpr int q = Q - 1;  // rest: c = 0
     const float w = float(L::w(q));
     const float gq = omt * g[q] + (w * tau_inv) * a0 + (w * tau_factor) * m3uF;
-    __builtin_nontemporal_store(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
+    st_elem<NT>(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
   }
   return REDUCE ? static_cast<double>(jd[0]) : 0.0;
 }
 
-template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE>
+template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE, bool NT>
 __global__ __launch_bounds__(kBlock) void k_bgk_lp(const S* __restrict__ gin, S* __restrict__ gout, A ad,
                                                    int32_t n, int64_t NP, float tau_inv, float tau_factor,
                                                    float F0, float F1, float F2,
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void k_bgk_lp(const S* __restrict__ gin, S*
   double jx = 0.0;
   if (i < n) {
     const float F[3] = {F0, F1, F2};
-    jx = bgk_node_lp<L, S, A, FIRST, STORE, REDUCE, MODE>(gin, gout, ad, i, NP, tau_inv, tau_factor, F, rho_o,
+    jx = bgk_node_lp<L, S, A, FIRST, STORE, REDUCE, MODE, NT>(gin, gout, ad, i, NP, tau_inv, tau_factor, F, rho_o,
                                                           vel_o, tauA_inv, tauA_factor, sr, nu, tab_n, step);
   }
   if (REDUCE) {
@@ -549,7 +549,7 @@ __device__ __forceinline__ void flux_td(const double (&t)[L::nQ], const double (
 // (64^3-128^3) the phase permeabilities differed from FP64 by 4e-4-1.2e-3 of
 // k0 + k1, against 2e-6-3.5e-5 with FP64 arithmetic on the same FP32
 // storage; the step time is the same (the passes are memory-bound).
-template <class L, typename S, bool O, bool STORE>
+template <class L, typename S, bool O, bool STORE, bool NT>
 __device__ __forceinline__ void cg_collide(const double (&t)[L::nQ], const double (&dd)[L::nQ],
                                            const float (&pn)[L::nQ], const double (&F)[3], double nu0Inv,
                                            double nu1Inv, double sigma, double beta, S* __restrict__ gout,
@@ -617,7 +617,7 @@ __device__ __forceinline__ void cg_collide(const double (&t)[L::nQ], const doubl
     const float bt = static_cast<float>(bs);
     const float bd = static_cast<float>(phi_n * (w + bs) + 2.0 * rc);
     const Pair<S> v{Store<S>::put_sr(bt, sr_bits(hn, q)), Store<S>::put_sr(bd, sr_bits(hn, q + 32))};
-    __builtin_nontemporal_store(v, out + (q << kPLog));
+    st_elem<NT>(v, out + (q << kPLog));
   }
 }
 
@@ -644,7 +644,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_phi_lp(const S* __restrict__ gin,
 }
 
 // Two-phase pass 3; solid neighbours take their wall colour (neighbour_phi).
-template <class L, typename S, bool FIRST, bool STORE, class A>
+template <class L, typename S, bool FIRST, bool STORE, bool NT, class A>
 __global__ __launch_bounds__(kBlock) void k_cg_lp(const S* __restrict__ gin, S* __restrict__ gout, A ad,
                                                   int32_t n, int64_t NP, double nu0Inv, double nu1Inv,
                                                   double sigma, double beta, double F0, double F1, double F2,
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_lp(const S* __restrict__ gin, S* 
   if (momx_mode) F[0] = dscalar[0];
   float pn[Q];
   neighbour_phi<L>(ad, i, phi, wp, pn);
-  cg_collide<L, S, A::kOff32, STORE>(t, dd, pn, F, nu0Inv, nu1Inv, sigma, beta, gout, i, NP, rho_o, vel_o,
+  cg_collide<L, S, A::kOff32, STORE, NT>(t, dd, pn, F, nu0Inv, nu1Inv, sigma, beta, gout, i, NP, rho_o, vel_o,
                                      step);
 }
 
@@ -746,7 +746,7 @@ __global__ __launch_bounds__(kBlock * NS, 4) void k_batch_cg_lp(const BatchSolve
       pn[qq] = f ? v : pw;
     }
     const double F[3] = {s.a.F[0], s.a.F[1], s.a.F[2]};
-    cg_collide<L, S, true, false>(t, dd, pn, F, s.nu0Inv, s.nu1Inv, s.sigma, s.beta, static_cast<S*>(s.f[p ^ 1]),
+    cg_collide<L, S, true, false, true>(t, dd, pn, F, s.nu0Inv, s.nu1Inv, s.sigma, s.beta, static_cast<S*>(s.f[p ^ 1]),
                                   i, s.NP, nullptr, nullptr, gstep - s.step_base);
   }
 }
@@ -811,7 +811,33 @@ __global__ __launch_bounds__(kBlock) void k_flux_td(const S* __restrict__ gin, T
 
 inline dim3 grid_for(int32_t n) { return dim3(static_cast<unsigned>((n + kBlock - 1) / kBlock)); }
 
-// f(lattice tag, storage tag, address layout) for the runtime choices
+// f(lattice tag, storage tag, address layout) for the runtime choices; with
+// stores: f(..., streaming stores) of a step launch, where the first step after
+// an upload (it reads every node's own slots, whatever the layout) is the link
+// table's instance.
+template <typename F>
+hipError_t step_dispatch(int precision, int lattice, const Addr& ad, int layout, bool first, F&& f) {
+  auto by_addr = [&](auto l, auto st) {
+    auto by_store = [&](const auto& a) {
+      if (ad.nt) f(l, st, a, std::true_type{});
+      else f(l, st, a, std::false_type{});
+    };
+    if (first) f(l, st, ad.table, std::true_type{});
+    else if (layout == kLayWin) by_store(ad.win);
+    else if (layout == kLayWinZ) by_store(ad.winz);
+    else if (layout == kLayRows) f(l, st, ad.rows, std::true_type{});  // buffers above 4 GiB
+    else by_store(ad.table);
+  };
+  if (lattice == 0) {
+    if (precision == 1) by_addr(D2Q9{}, float{});
+    else by_addr(D2Q9{}, uint16_t{});
+  } else {
+    if (precision == 1) by_addr(D3Q19{}, float{});
+    else by_addr(D3Q19{}, uint16_t{});
+  }
+  return hipGetLastError();
+}
+
 template <typename F>
 hipError_t dispatch(int precision, int lattice, const Addr& ad, F&& f) {
   auto by_addr = [&](auto l, auto st) {
@@ -883,38 +909,34 @@ hipError_t bgk_lowp(int precision, int lattice, bool first, bool store, bool red
   const float ti = static_cast<float>(a.tau_inv), tf = static_cast<float>(a.tau_factor);
   const float F0 = static_cast<float>(a.F[0]), F1 = static_cast<float>(a.F[1]), F2 = static_cast<float>(a.F[2]);
   const float tai = static_cast<float>(a.tauA_inv), taf = static_cast<float>(a.tauA_factor);  // TRT only
-  // (first, store, reduce)
-  const int key = (first ? 4 : 0) | (store ? 2 : 0) | (reduce ? 1 : 0);
-  return dispatch(precision, lattice, ad, [&](auto l, auto st, auto addr) {
+  return step_dispatch(precision, lattice, ad, ad.layout, first, [&](auto l, auto st, const auto& addr, auto nt) {
     using L = decltype(l);
     using S = decltype(st);
-    using A = decltype(addr);
+    using A = std::decay_t<decltype(addr)>;
+    constexpr bool NT = decltype(nt)::value;
     const S* gi = static_cast<const S*>(gin);
     S* go = static_cast<S*>(gout);
     const dim3 g = grid_for(n), b(kBlock);
-#define LB_K(F_, S_, R_, T_)                                                                             \
-  k_bgk_lp<L, S, A, F_, S_, R_, T_><<<g, b, 0, s>>>(gi, go, addr, n, NP, ti, tf, F0, F1, F2, rho, vel, partial, \
-                                                    tai, taf, a.tab_srf, a.tab_nuf, a.tab_n, a.step, ac)
-#define LB_KEYS(T_)                                 \
-  switch (key) {                                    \
-    case 0: LB_K(false, false, false, T_); break;   \
-    case 1: LB_K(false, false, true, T_); break;    \
-    case 2: LB_K(false, true, false, T_); break;    \
-    case 3: LB_K(false, true, true, T_); break;     \
-    case 4: LB_K(true, false, false, T_); break;    \
-    case 5: LB_K(true, false, true, T_); break;     \
-    case 6: LB_K(true, true, false, T_); break;     \
-    default: LB_K(true, true, true, T_); break;     \
-  }
-    if (a.mode == kTrt) {
-      LB_KEYS(kTrt)
-    } else if (a.mode == kRheology) {
-      LB_KEYS(kRheology)
-    } else {
-      LB_KEYS(kBgk)
-    }
-#undef LB_KEYS
+    auto modes = [&](auto fi, auto sto, auto re) {
+      constexpr bool F = decltype(fi)::value, W = decltype(sto)::value, R = decltype(re)::value;
+#define LB_K(T_)                                                                                            \
+  k_bgk_lp<L, S, A, F, W, R, T_, NT><<<g, b, 0, s>>>(gi, go, addr, n, NP, ti, tf, F0, F1, F2, rho, vel, partial, \
+                                                     tai, taf, a.tab_srf, a.tab_nuf, a.tab_n, a.step, ac)
+      if (a.mode == kTrt) LB_K(kTrt);
+      else if (a.mode == kRheology) LB_K(kRheology);
+      else LB_K(kBgk);
 #undef LB_K
+    };
+    auto keys = [&](auto fi) {
+      if (store && reduce) modes(fi, std::true_type{}, std::true_type{});
+      else if (store) modes(fi, std::true_type{}, std::false_type{});
+      else if (reduce) modes(fi, std::false_type{}, std::true_type{});
+      else modes(fi, std::false_type{}, std::false_type{});
+    };
+    if constexpr (std::is_same_v<A, TableAddr> && NT) {
+      if (first) return keys(std::true_type{});
+    }
+    keys(std::false_type{});
   });
 }
 
@@ -1012,28 +1034,27 @@ hipError_t cg_lowp(int precision, int lattice, bool first, bool store, const voi
   if (a.q0 != 0.0 || a.q1 != 0.0) return hipErrorInvalidValue;  // no mass sources in this form
   const double n0 = a.nu0Inv, n1 = a.nu1Inv, sg = a.sigma, be = a.beta;
   const double F0 = a.F[0], F1 = a.F[1], F2 = a.F[2];
-  Addr sel = ad;
-  sel.layout = layout;
-  return dispatch(precision, lattice, sel, [&](auto l, auto st, auto addr) {
+  return step_dispatch(precision, lattice, ad, layout, first, [&](auto l, auto st, const auto& addr, auto nt) {
     using L = decltype(l);
     using S = decltype(st);
-    using A = decltype(addr);
-    if constexpr (std::is_same<A, RowAddr>::value) {
-      return;  // not used for two-phase
-    } else {
+    using A = std::decay_t<decltype(addr)>;
+    constexpr bool NT = decltype(nt)::value;
+    if constexpr (!std::is_same_v<A, RowAddr>) {  // the two-phase layouts are the link table and the windows
       const S* gi = static_cast<const S*>(gin);
       S* go = static_cast<S*>(gout);
       const dim3 g = grid_for(n), b(kBlock);
-#define LB_K(F_, S_)                                                                                        \
-  k_cg_lp<L, S, F_, S_, A><<<g, b, 0, s>>>(gi, go, addr, n, NP, n0, n1, sg, be, F0, F1, F2, a.momx_mode, phi, \
-                                           wp, dscalar, rho, vel, a.step)
-      if (first) {
-        if (store) LB_K(true, true);
-        else LB_K(true, false);
-      } else {
-        if (store) LB_K(false, true);
-        else LB_K(false, false);
+#define LB_K(F_, S_)                                                                                            \
+  k_cg_lp<L, S, F_, S_, NT, A><<<g, b, 0, s>>>(gi, go, addr, n, NP, n0, n1, sg, be, F0, F1, F2, a.momx_mode, phi, \
+                                               wp, dscalar, rho, vel, a.step)
+      if constexpr (std::is_same_v<A, TableAddr> && NT) {
+        if (first) {
+          if (store) LB_K(true, true);
+          else LB_K(true, false);
+          return;
+        }
       }
+      if (store) LB_K(false, true);
+      else LB_K(false, false);
 #undef LB_K
     }
   });

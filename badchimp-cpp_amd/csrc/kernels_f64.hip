@@ -12,6 +12,8 @@
 // post-collision values and each step starts with the gather.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "lattice.hpp"
 #include "layout_select.hpp"
@@ -144,7 +146,7 @@ __device__ __forceinline__ double rheology_visc(const double (&f)[L::nQ], double
 // kRheology: polymer_viscosity_tabulation/main.cpp:105-155, the relaxation
 // time from the node's strain rate and the viscosity table; the viscosity
 // is stored beside rho (rho_o[NP + i]) when STORE.
-template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk>
+template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
 __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, double* __restrict__ fout, const A& ad,
                                            int32_t i, int64_t NP, const BgkArgs& a, double* __restrict__ rho_o,
                                            double* __restrict__ vel_o) {
@@ -183,7 +185,7 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
       const double feq = (L::w(q) * rho) * ((1 + L::c2Inv * cu) + L::c4Inv0_5 * (cu * cu - c2u2));
       const double om = (-tau_inv) * (f[0][q] - feq);
       const double dF = (L::w(q) * tau_factor) * (L::c2Inv * cF + L::c4Inv * (cF * cu - c2uF));
-      __builtin_nontemporal_store((f[0][q] + om) + dF, out + (q << kPLog));
+      st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
     }
     return jx;
   }
@@ -201,7 +203,7 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
                         a.tauA_inv * (fqAnti - (rw * L::c2Inv) * cu);
       // calcDeltaOmegaFTRT, phi = 1 (LBcollision.h:229): w * 1.0 == w
       const double dF = L::w(q) * ((a.tauA_factor * L::c2Inv) * cF + (a.tau_factor * L::c4Inv) * (cF * cu - c2uF));
-      __builtin_nontemporal_store((f[0][q] + om) + dF, out + (q << kPLog));
+      st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
     }
     return jx;
   }
@@ -214,14 +216,14 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
     const double om = (-a.tau_inv) * (f[0][q] - feq);
     // calcDeltaOmegaF (LBcollision.h:206-211)
     const double dF = (L::w(q) * a.tau_factor) * (L::c2Inv * cF + L::c4Inv * (cF * cu - c2uF));
-    __builtin_nontemporal_store((f[0][q] + om) + dF, out + (q << kPLog));
+    st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
   }
   return jx;
 }
 
 // REDUCE: the block's sum of j_x goes to partial[b], or is added to it
 // (accum), so that a check interval's partials hold the sum over its steps.
-template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE>
+template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE, bool NT>
 __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
                                                 double* __restrict__ fout, A ad, int32_t n,
                                                 int64_t NP, BgkArgs a, double* __restrict__ rho_o,
@@ -232,7 +234,7 @@ __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
   // the block's running sum, read before the node work (latency overlapped)
   const double prev = REDUCE && accum && threadIdx.x == 0 ? partial[b] : 0.0;
   double jx = 0.0;
-  if (i < n) jx = bgk_node<L, A, FIRST, STORE, REDUCE, MODE>(fin, fout, ad, i, NP, a, rho_o, vel_o);
+  if (i < n) jx = bgk_node<L, A, FIRST, STORE, REDUCE, MODE, NT>(fin, fout, ad, i, NP, a, rho_o, vel_o);
   if (REDUCE) {
     const double s = block_sum(jx);
     if (threadIdx.x == 0) partial[b] = accum ? prev + s : s;
@@ -497,7 +499,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_phi(const double* __restrict__ fi
 // ------------------------------------------------------------------ two-phase pass 3
 // One node of the colour-gradient collision (main_TWOPHASE.cpp:318-392) with
 // the body force F; phi: the colour field of this step (pass 1).
-template <class L, bool FIRST, bool STORE, class A>
+template <class L, bool FIRST, bool STORE, bool NT, class A>
 __device__ __forceinline__ void cg_node(const double* __restrict__ fin, double* __restrict__ fout, const A& ad,
                                         int32_t i, int64_t NP, const CgArgs& a, const double* __restrict__ phi,
                                         const WallPhi& wp, const double (&F)[L::nD], double* __restrict__ rho_o,
@@ -568,11 +570,11 @@ __device__ __forceinline__ void cg_node(const double* __restrict__ fin, double* 
     }
     const double base = ((ft[q] + om) + dF) + st;
     const Double2 v{((c0 * base) + rc) + dQ0, ((c1 * base) - rc) + dQ1};
-    __builtin_nontemporal_store(v, out + (q << kPLog));
+    st_elem<NT>(v, out + (q << kPLog));
   }
 }
 
-template <class L, bool FIRST, bool STORE, class A>
+template <class L, bool FIRST, bool STORE, bool NT, class A>
 __global__ __launch_bounds__(kBlock) void k_cg(const double* __restrict__ fin,
                                                double* __restrict__ fout, A ad, int32_t n,
                                                int64_t NP, CgArgs a,
@@ -588,7 +590,7 @@ __global__ __launch_bounds__(kBlock) void k_cg(const double* __restrict__ fin,
 #pragma unroll
   for (int d = 0; d < D; ++d) F[d] = a.F[d];
   if (a.momx_mode) F[0] = dscalar[0];
-  cg_node<L, FIRST, STORE>(fin, fout, ad, i, NP, a, phi, wp, F, rho_o, vel_o);
+  cg_node<L, FIRST, STORE, NT>(fin, fout, ad, i, NP, a, phi, wp, F, rho_o, vel_o);
 }
 
 // Batched colour-gradient step in FP64 (items as k_batch_bgk; fixed force;
@@ -674,7 +676,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg(const BatchSolve* __re
 #pragma unroll
     for (int d = 0; d < D; ++d) F[d] = s.a.F[d];
     const WallPhi wp{nullptr, s.phi_w};
-    cg_node<L, false, false>(static_cast<const double*>(s.f[p]), static_cast<double*>(s.f[p ^ 1]), ad, i, s.NP, a,
+    cg_node<L, false, false, true>(static_cast<const double*>(s.f[p]), static_cast<double*>(s.f[p ^ 1]), ad, i, s.NP, a,
                              static_cast<const double*>(s.phi), wp, F, nullptr, nullptr);
   }
 }
@@ -807,51 +809,50 @@ inline dim3 grid_for(int32_t n) { return dim3(static_cast<unsigned>((n + kBlock 
     }                                    \
   } while (0)
 
-template <class L, class A>
-static void launch_bgk(bool first, bool store, bool reduce, dim3 g, hipStream_t s, const double* fin,
-                       double* fout, const A& ad, int32_t n, int64_t NP, const BgkArgs& a, double* rho,
-                       double* vel, double* partial, bool accum) {
-  const dim3 b(kBlock);
-  // (first, store, reduce)
-  const int key = (first ? 4 : 0) | (store ? 2 : 0) | (reduce ? 1 : 0);
-  const int32_t ac = accum ? 1 : 0;
-#define LB_K(F_, S_, R_, T_) \
-  k_bgk<L, A, F_, S_, R_, T_><<<g, b, 0, s>>>(fin, fout, ad, n, NP, a, rho, vel, partial, ac)
-#define LB_KEYS(T_)                            \
-  switch (key) {                               \
-    case 0: LB_K(false, false, false, T_); break; \
-    case 1: LB_K(false, false, true, T_); break;  \
-    case 2: LB_K(false, true, false, T_); break;  \
-    case 3: LB_K(false, true, true, T_); break;   \
-    case 4: LB_K(true, false, false, T_); break;  \
-    case 5: LB_K(true, false, true, T_); break;   \
-    case 6: LB_K(true, true, false, T_); break;   \
-    default: LB_K(true, true, true, T_); break;   \
-  }
-  if (a.mode == kTrt) {
-    LB_KEYS(kTrt)
-  } else if (a.mode == kRheology) {
-    LB_KEYS(kRheology)
-  } else {
-    LB_KEYS(kBgk)
-  }
-#undef LB_KEYS
-#undef LB_K
+// f(address layout, streaming stores) of a step launch.  The first step after
+// an upload reads every node's own slots, whatever the layout: one instance,
+// the link table's.
+template <class F>
+static void step_dispatch(const Addr& ad, int layout, bool first, F&& f) {
+  auto by_store = [&](const auto& a) {
+    if (ad.nt) f(a, std::true_type{});
+    else f(a, std::false_type{});
+  };
+  if (first) f(ad.table, std::true_type{});
+  else if (layout == kLayWin) by_store(ad.win);
+  else if (layout == kLayWinZ) by_store(ad.winz);
+  else if (layout == kLayRows) f(ad.rows, std::true_type{});  // buffers above 4 GiB
+  else by_store(ad.table);
 }
 
 hipError_t bgk_f64(int lattice, bool first, bool store, bool reduce, const double* fin,
                    double* fout, const Addr& ad, int32_t n, int64_t NP, const BgkArgs& a,
                    double* rho, double* vel, double* partial, hipStream_t s, bool accum) {
   if (n <= 0) return hipSuccess;
-  const dim3 g = grid_for(n);
+  const dim3 g = grid_for(n), b(kBlock);
+  const int32_t ac = accum ? 1 : 0;
   LB_DISPATCH_LATTICE(lattice, L, {
-    if (ad.layout == kLayWin)
-      launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.win, n, NP, a, rho, vel, partial, accum);
-    else if (ad.layout == kLayWinZ)
-      launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.winz, n, NP, a, rho, vel, partial, accum);
-    else if (ad.layout == kLayRows)
-      launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.rows, n, NP, a, rho, vel, partial, accum);
-    else launch_bgk<L>(first, store, reduce, g, s, fin, fout, ad.table, n, NP, a, rho, vel, partial, accum);
+    step_dispatch(ad, ad.layout, first, [&](const auto& addr, auto nt) {
+      using A = std::decay_t<decltype(addr)>;
+      constexpr bool NT = decltype(nt)::value;
+      // the link table serves first steps too; (store, reduce)
+      auto modes = [&](auto fi, auto st, auto re) {
+        constexpr bool F = decltype(fi)::value, S = decltype(st)::value, R = decltype(re)::value;
+        if (a.mode == kTrt) k_bgk<L, A, F, S, R, kTrt, NT><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, rho, vel, partial, ac);
+        else if (a.mode == kRheology) k_bgk<L, A, F, S, R, kRheology, NT><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, rho, vel, partial, ac);
+        else k_bgk<L, A, F, S, R, kBgk, NT><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, rho, vel, partial, ac);
+      };
+      auto keys = [&](auto fi) {
+        if (store && reduce) modes(fi, std::true_type{}, std::true_type{});
+        else if (store) modes(fi, std::true_type{}, std::false_type{});
+        else if (reduce) modes(fi, std::false_type{}, std::true_type{});
+        else modes(fi, std::false_type{}, std::false_type{});
+      };
+      if constexpr (std::is_same_v<A, TableAddr> && NT) {
+        if (first) return keys(std::true_type{});
+      }
+      keys(std::false_type{});
+    });
   });
   return hipGetLastError();
 }
@@ -880,18 +881,20 @@ hipError_t cg_f64(int lattice, bool first, bool store, const double* fin, double
                   const double* dscalar, double* rho, double* vel, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const dim3 g = grid_for(n), b(kBlock);
-  auto go = [&](auto addr) {
-    using A = decltype(addr);
-    LB_DISPATCH_LATTICE(lattice, L, {
-      if (first && store) k_cg<L, true, true, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
-      else if (first) k_cg<L, true, false, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
-      else if (store) k_cg<L, false, true, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
-      else k_cg<L, false, false, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
+  LB_DISPATCH_LATTICE(lattice, L, {
+    step_dispatch(ad, layout, first, [&](const auto& addr, auto nt) {
+      using A = std::decay_t<decltype(addr)>;
+      constexpr bool NT = decltype(nt)::value;
+      if constexpr (!std::is_same_v<A, RowAddr>) {  // the two-phase layouts are the link table and the windows
+        if constexpr (std::is_same_v<A, TableAddr> && NT) {
+          if (first && store) return k_cg<L, true, true, NT, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
+          if (first) return k_cg<L, true, false, NT, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
+        }
+        if (store) k_cg<L, false, true, NT, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
+        else k_cg<L, false, false, NT, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
+      }
     });
-  };
-  if (layout == kLayWin) go(ad.win);
-  else if (layout == kLayWinZ) go(ad.winz);
-  else go(ad.table);
+  });
   return hipGetLastError();
 }
 
