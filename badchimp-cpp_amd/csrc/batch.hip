@@ -143,6 +143,7 @@ struct Slot {
   Footprint fp;
   int64_t steps_seen = 0;  // steps of the solve at the last read-back of its stop state
   double t_admit = 0.0;
+  std::vector<uint8_t> xcd;  // XCD of each 256-node block (block_xcd)
 };
 
 struct Result {
@@ -228,42 +229,35 @@ void drop_graphs(lb_batch* b) {
     }
 }
 
-// grid and items per workgroup of a shape (workgroups per CU; 0: one
-// workgroup per ns items) with ns items in flight per workgroup
-void shape_dims(const lb_batch* b, int32_t shape, int32_t ns, int32_t n_items, int32_t* grid, int32_t* per) {
-  if (shape <= 0 || n_items <= b->n_cu * shape * ns) {
-    *per = ns;
-    *grid = (n_items + ns - 1) / ns;
-    return;
-  }
-  const int32_t g = b->n_cu * shape;
-  *per = (n_items + g - 1) / g;
-  *grid = (n_items + *per - 1) / *per;
+// grid of a shape (workgroups per CU, in multiples of 8; 0: one workgroup per
+// ns items) with ns items in flight per workgroup
+int32_t shape_grid(const lb_batch* b, int32_t shape, int32_t ns, int32_t n_items) {
+  const int32_t all = ns == 2 ? batch_positions<2>(n_items) : batch_positions<1>(n_items);
+  return shape <= 0 ? all : std::min(all, (b->n_cu * shape + 7) / 8 * 8);
 }
 
 hipError_t launch_step(lb_batch* b, bool reduce, int32_t shape, int32_t ns, int32_t koff) {
   const int32_t parity = static_cast<int32_t>(b->global_step & 1);
-  int32_t grid, per;
   hipError_t e = hipSuccess;
   if (b->n_items_bgk > 0) {
     // single-phase: j_x summed over every step of the interval (the first
     // step of the interval overwrites the partials)
     const int32_t n = b->n_items_bgk;
-    shape_dims(b, shape, ns, n, &grid, &per);
+    const int32_t grid = shape_grid(b, shape, ns, n);
     if (b->prec[0] == LB_FP64)
-      e = batch_bgk_f64(b->lattice, true, b->d_solves, b->d_items, n, grid, per, parity, ns, koff > 0, b->stream);
+      e = batch_bgk_f64(b->lattice, true, b->d_solves, b->d_items, n, grid, parity, ns, koff > 0, b->stream);
     else
-      e = batch_bgk_lowp(b->prec[0], b->lattice, true, b->d_solves, b->d_items, n, grid, per, parity,
+      e = batch_bgk_lowp(b->prec[0], b->lattice, true, b->d_solves, b->d_items, n, grid, parity,
                          b->d_step, koff, ns, koff > 0, b->stream);
   }
   if (e == hipSuccess && b->n_items_cg > 0) {
     const int32_t n = b->n_items_cg;
     const uint32_t* it = b->d_items + b->n_items_bgk;
-    shape_dims(b, shape, ns, n, &grid, &per);
+    const int32_t grid = shape_grid(b, shape, ns, n);
     if (b->prec[1] == LB_FP64)
-      e = batch_cg_f64(b->lattice, reduce, b->d_solves, it, n, grid, per, parity, ns, b->stream);
+      e = batch_cg_f64(b->lattice, reduce, b->d_solves, it, n, grid, parity, ns, b->stream);
     else
-      e = batch_cg_lowp(b->prec[1], b->lattice, reduce, b->d_solves, it, n, grid, per, parity, b->d_step, koff,
+      e = batch_cg_lowp(b->prec[1], b->lattice, reduce, b->d_solves, it, n, grid, parity, b->d_step, koff,
                         ns, b->stream);
   }
   return e;
@@ -276,14 +270,19 @@ int refresh(lb_batch* b) {
   b->active.clear();
   b->resident_nodes = 0;
   for (int kind = 0; kind < 2; ++kind) {
+    std::vector<uint32_t> items;
+    std::vector<uint8_t> xcd;
     for (int32_t s = 0; s < static_cast<int32_t>(b->slots.size()); ++s) {
       const Slot& sl = b->slots[s];
       if (!sl.used || sl.kind != kind) continue;
       b->active.push_back(s);
       b->resident_nodes += sl.fp.n;
       for (int64_t k = 0; k < sl.fp.nblk; ++k)
-        b->items.push_back((static_cast<uint32_t>(s) << kItemShift) | static_cast<uint32_t>(k));
+        items.push_back((static_cast<uint32_t>(s) << kItemShift) | static_cast<uint32_t>(k));
+      xcd.insert(xcd.end(), sl.xcd.begin(), sl.xcd.end());
     }
+    items = interleave_xcds(items, xcd);
+    b->items.insert(b->items.end(), items.begin(), items.end());
     if (kind == 0) b->n_items_bgk = static_cast<int32_t>(b->items.size());
   }
   b->n_items_cg = static_cast<int32_t>(b->items.size()) - b->n_items_bgk;
@@ -607,6 +606,7 @@ struct AddArgs {
 struct Prepared {
   RowBuild rb;
   WinBuild wb;
+  std::vector<uint8_t> xcd;
   int code = LB_OK;
   std::string why;
 };
@@ -619,6 +619,7 @@ void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t perio
   }
   const RowBuild& rb = pr.rb;
   const int64_t n = static_cast<int64_t>(rb.coord.size());
+  pr.xcd = block_xcd(rb.coord);
   // every node's own window must name it (a cheap check of the construction)
   for (int64_t i = 0; i < n; ++i) {
     const auto own = win_cell(rb, pr.wb, static_cast<int32_t>(i), 0, 0, 0);
@@ -796,6 +797,7 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
   sl.off = off;
   sl.fp = fp;
   sl.t_admit = now_s();
+  sl.xcd = pre->xcd;
   b->dirty = true;
   return LB_OK;
 }

@@ -349,39 +349,37 @@ __global__ __launch_bounds__(kBlock) void k_bgk_lp(const S* __restrict__ gin, S*
 template <class L, typename S, bool REDUCE, int NS>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk_lp(const BatchSolve* __restrict__ solves,
                                                               const uint32_t* __restrict__ items, int32_t n_items,
-                                                              int32_t per_wg, int32_t parity,
+                                                              int32_t parity,
                                                               const uint32_t* __restrict__ step0, int32_t koff,
                                                               int32_t accum) {
   const uint32_t gstep = *step0 + static_cast<uint32_t>(koff);  // global step of this launch
-  const int32_t g = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t sub = static_cast<int32_t>(threadIdx.x) / kBlock, tid = static_cast<int32_t>(threadIdx.x) % kBlock;
-  const int32_t beg = g * per_wg;
-  const int32_t end = beg + per_wg < n_items ? beg + per_wg : n_items;
-  for (int32_t base = beg; base < end; base += NS) {
-    const int32_t it = base + sub;
-    const uint32_t item = items[it < end ? it : base];
+  const int32_t np = batch_positions<NS>(n_items);
+  for (int32_t pos = static_cast<int32_t>(blockIdx.x); pos < np; pos += static_cast<int32_t>(gridDim.x)) {
+    const int32_t it = batch_item<NS>(pos, sub);
+    const uint32_t item = wave_item(items, it < n_items ? it : n_items - 1);
     const BatchSolve& s = solves[item >> kItemShift];
     // a slice past the run, or a solve stopped at an earlier check of this
     // launch sequence, computes nothing (but joins the slice sums)
-    const bool act = it < end && s.live;
+    const bool act = it < n_items && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
     const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     // the running sum of this block over the interval, read before the node
     // work so that its latency overlaps the gathers
-    const double prev = REDUCE && accum && tid == 0 && act ? s.partial[lb] : 0.0;
+    const double prev = REDUCE && accum && tid == 0 && act ? device_ptr(s.partial)[lb] : 0.0;
     double jx = 0.0;
     if (act && i < s.n) {
       const float F[3] = {static_cast<float>(s.a.F[0]), static_cast<float>(s.a.F[1]), static_cast<float>(s.a.F[2])};
       jx = bgk_node_lp<L, S, RowWin, false, false, REDUCE>(
-          static_cast<const S*>(s.f[p]), static_cast<S*>(s.f[p ^ 1]), ad, i, s.NP, static_cast<float>(s.a.tau_inv),
+          static_cast<const S*>(device_ptr(s.f[p])), static_cast<S*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, static_cast<float>(s.a.tau_inv),
           static_cast<float>(s.a.tau_factor), F, nullptr, nullptr, 0.0f, 0.0f, nullptr, nullptr, 0,
           gstep - s.step_base);
     }
     if (REDUCE) {
       const double t = slice_sum<NS>(jx);
-      if (act && tid == 0) s.partial[lb] = accum ? prev + t : t;
+      if (act && tid == 0) device_ptr(s.partial)[lb] = accum ? prev + t : t;
     }
   }
 }
@@ -672,17 +670,15 @@ __global__ __launch_bounds__(kBlock) void k_cg_lp(const S* __restrict__ gin, S* 
 template <class L, typename S, bool REDUCE, int NS>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi_lp(const BatchSolve* __restrict__ solves,
                                                                  const uint32_t* __restrict__ items,
-                                                                 int32_t n_items, int32_t per_wg, int32_t parity) {
+                                                                 int32_t n_items, int32_t parity) {
   constexpr int Q = L::nQ;
-  const int32_t g = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t sub = static_cast<int32_t>(threadIdx.x) / kBlock, tid = static_cast<int32_t>(threadIdx.x) % kBlock;
-  const int32_t beg = g * per_wg;
-  const int32_t end = beg + per_wg < n_items ? beg + per_wg : n_items;
-  for (int32_t base = beg; base < end; base += NS) {
-    const int32_t it = base + sub;
-    const uint32_t item = items[it < end ? it : base];
+  const int32_t np = batch_positions<NS>(n_items);
+  for (int32_t pos = static_cast<int32_t>(blockIdx.x); pos < np; pos += static_cast<int32_t>(gridDim.x)) {
+    const int32_t it = batch_item<NS>(pos, sub);
+    const uint32_t item = wave_item(items, it < n_items ? it : n_items - 1);
     const BatchSolve& s = solves[item >> kItemShift];
-    const bool act = it < end && s.live;
+    const bool act = it < n_items && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
     const RowWin ad = solve_windows(s);
@@ -690,8 +686,8 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi_lp(const BatchSolv
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     if (act && i < s.n) {
       double t[Q], d[Q];
-      load_td<L, S, false>(static_cast<const S*>(s.f[p]), ad, i, t, d);
-      static_cast<float*>(s.phi)[i] = static_cast<float>(phi_td<L>(t, d));
+      load_td<L, S, false>(static_cast<const S*>(device_ptr(s.f[p])), ad, i, t, d);
+      static_cast<float*>(device_ptr(s.phi))[i] = static_cast<float>(phi_td<L>(t, d));
       if (REDUCE) flux_td<L>(t, d, 0, s0, s1, s2);
     }
     if (REDUCE) {
@@ -700,9 +696,9 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi_lp(const BatchSolv
       s1 = slice_sum<NS>(s1);
       s2 = slice_sum<NS>(s2);
       if (act && tid == 0) {
-        s.partial[lb] = s0;
-        s.partial[nb + lb] = s1;
-        s.partial[2 * nb + lb] = s2;
+        device_ptr(s.partial)[lb] = s0;
+        device_ptr(s.partial)[nb + lb] = s1;
+        device_ptr(s.partial)[2 * nb + lb] = s2;
       }
     }
   }
@@ -714,18 +710,16 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi_lp(const BatchSolv
 template <class L, typename S, int NS>
 __global__ __launch_bounds__(kBlock * NS, 4) void k_batch_cg_lp(const BatchSolve* __restrict__ solves,
                                                              const uint32_t* __restrict__ items, int32_t n_items,
-                                                             int32_t per_wg, int32_t parity,
+                                                             int32_t parity,
                                                              const uint32_t* __restrict__ step0, int32_t koff) {
   constexpr int Q = L::nQ;
   const uint32_t gstep = *step0 + static_cast<uint32_t>(koff);  // global step of this launch
-  const int32_t g = node_block_rev(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t sub = static_cast<int32_t>(threadIdx.x) / kBlock, tid = static_cast<int32_t>(threadIdx.x) % kBlock;
-  const int32_t beg = g * per_wg;
-  const int32_t end = beg + per_wg < n_items ? beg + per_wg : n_items;
-  for (int32_t base = beg; base < end; base += NS) {
-    const int32_t it = base + sub;
-    if (it >= end) continue;
-    const uint32_t item = items[it];
+  const int32_t np = batch_positions<NS>(n_items);
+  for (int32_t pos = static_cast<int32_t>(blockIdx.x); pos < np; pos += static_cast<int32_t>(gridDim.x)) {
+    const int32_t it = batch_item<NS>(np - 1 - pos, sub);  // from the end, where pass 1 ended
+    if (it >= n_items) continue;
+    const uint32_t item = wave_item(items, it);
     const BatchSolve& s = solves[item >> kItemShift];
     if (!s.live) continue;  // stopped at an earlier check of this launch sequence
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
@@ -735,18 +729,18 @@ __global__ __launch_bounds__(kBlock * NS, 4) void k_batch_cg_lp(const BatchSolve
     if (i >= s.n) continue;
     double t[Q], dd[Q];
     uint32_t j[Q - 1], fluid;
-    load_td_links<L, S>(static_cast<const S*>(s.f[p]), ad, i, t, dd, j, fluid);
+    load_td_links<L, S>(static_cast<const S*>(device_ptr(s.f[p])), ad, i, t, dd, j, fluid);
     const float pw = static_cast<float>(s.phi_w);
     float pn[Q];
 #pragma unroll
     for (int qq = 0; qq < Q - 1; ++qq) {
       const int q = L::rev(qq);
       const bool f = (fluid >> q) & 1u;
-      const float v = static_cast<const float*>(s.phi)[f ? j[q] : static_cast<uint32_t>(i)];
+      const float v = static_cast<const float*>(device_ptr(s.phi))[f ? j[q] : static_cast<uint32_t>(i)];
       pn[qq] = f ? v : pw;
     }
     const double F[3] = {s.a.F[0], s.a.F[1], s.a.F[2]};
-    cg_collide<L, S, true, false, true>(t, dd, pn, F, s.nu0Inv, s.nu1Inv, s.sigma, s.beta, static_cast<S*>(s.f[p ^ 1]),
+    cg_collide<L, S, true, false, true>(t, dd, pn, F, s.nu0Inv, s.nu1Inv, s.sigma, s.beta, static_cast<S*>(device_ptr(s.f[p ^ 1])),
                                   i, s.NP, nullptr, nullptr, gstep - s.step_base);
   }
 }
@@ -965,7 +959,7 @@ hipError_t flux_lowp(int precision, int lattice, int nf, bool first, const void*
 }
 
 hipError_t batch_bgk_lowp(int precision, int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                          int32_t n_items, int32_t grid, int32_t per_wg, int32_t parity, const uint32_t* step0,
+                          int32_t n_items, int32_t grid, int32_t parity, const uint32_t* step0,
                           int32_t koff, int ns, bool accum, hipStream_t s) {
   return dispatch(precision, lattice, Addr{}, [&](auto l, auto st, auto) {
     using L = decltype(l);
@@ -973,17 +967,17 @@ hipError_t batch_bgk_lowp(int precision, int lattice, bool reduce, const BatchSo
     const dim3 g(grid), b(kBlock);
     if (ns == 2) {
       const dim3 b2(2 * kBlock);
-      if (reduce) k_batch_bgk_lp<L, S, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity, step0, koff, accum ? 1 : 0);
-      else k_batch_bgk_lp<L, S, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity, step0, koff, accum ? 1 : 0);
+      if (reduce) k_batch_bgk_lp<L, S, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
+      else k_batch_bgk_lp<L, S, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
     } else {
-      if (reduce) k_batch_bgk_lp<L, S, true, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity, step0, koff, accum ? 1 : 0);
-      else k_batch_bgk_lp<L, S, false, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity, step0, koff, accum ? 1 : 0);
+      if (reduce) k_batch_bgk_lp<L, S, true, 1><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
+      else k_batch_bgk_lp<L, S, false, 1><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
     }
   });
 }
 
 hipError_t batch_cg_lowp(int precision, int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                         int32_t n_items, int32_t grid, int32_t per_wg, int32_t parity, const uint32_t* step0,
+                         int32_t n_items, int32_t grid, int32_t parity, const uint32_t* step0,
                          int32_t koff, int ns, hipStream_t s) {
   return dispatch(precision, lattice, Addr{}, [&](auto l, auto st, auto) {
     using L = decltype(l);
@@ -991,13 +985,13 @@ hipError_t batch_cg_lowp(int precision, int lattice, bool reduce, const BatchSol
     const dim3 g(grid), b(kBlock);
     if (ns == 2) {
       const dim3 b2(2 * kBlock);
-      if (reduce) k_batch_cg_phi_lp<L, S, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity);
-      else k_batch_cg_phi_lp<L, S, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity);
-      k_batch_cg_lp<L, S, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity, step0, koff);
+      if (reduce) k_batch_cg_phi_lp<L, S, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
+      else k_batch_cg_phi_lp<L, S, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
+      k_batch_cg_lp<L, S, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity, step0, koff);
     } else {
-      if (reduce) k_batch_cg_phi_lp<L, S, true, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity);
-      else k_batch_cg_phi_lp<L, S, false, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity);
-      k_batch_cg_lp<L, S, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity, step0, koff);
+      if (reduce) k_batch_cg_phi_lp<L, S, true, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      else k_batch_cg_phi_lp<L, S, false, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      k_batch_cg_lp<L, S, 1><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff);
     }
   });
 }

@@ -242,9 +242,10 @@ __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
 }
 
 // Batched form: one launch advances every resident solve one step.  Work
-// items are 256-node blocks of the solves (item = slot << kItemShift | block);
-// each workgroup takes a contiguous run of per_wg items, so the resident
-// workgroups sweep the items as one compact front.  A solve's buffers, address table and parameters come from its
+// items are 256-node blocks of the solves (item = slot << kItemShift | block),
+// in an order that gives each XCD its runs (interleave_xcds); a workgroup takes
+// every grid-th position, so the resident workgroups sweep the items as one
+// compact front.  A solve's buffers, address table and parameters come from its
 // descriptor (uniform per item), and the per-node arithmetic is the single
 // solve's (bgk_node), so a solve gets the same bits alone or in any mix.
 // NS: items a workgroup works on at a time, one per 256-thread slice; every
@@ -252,33 +253,31 @@ __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
 template <class L, bool REDUCE, int NS>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk(const BatchSolve* __restrict__ solves,
                                                            const uint32_t* __restrict__ items, int32_t n_items,
-                                                           int32_t per_wg, int32_t parity, int32_t accum) {
-  const int32_t g = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+                                                           int32_t parity, int32_t accum) {
   const int32_t sub = static_cast<int32_t>(threadIdx.x) / kBlock, tid = static_cast<int32_t>(threadIdx.x) % kBlock;
-  const int32_t beg = g * per_wg;
-  const int32_t end = beg + per_wg < n_items ? beg + per_wg : n_items;
-  for (int32_t base = beg; base < end; base += NS) {
-    const int32_t it = base + sub;
-    const uint32_t item = items[it < end ? it : base];
+  const int32_t np = batch_positions<NS>(n_items);
+  for (int32_t pos = static_cast<int32_t>(blockIdx.x); pos < np; pos += static_cast<int32_t>(gridDim.x)) {
+    const int32_t it = batch_item<NS>(pos, sub);
+    const uint32_t item = wave_item(items, it < n_items ? it : n_items - 1);
     const BatchSolve& s = solves[item >> kItemShift];
     // a slice past the run, or a solve stopped at an earlier check of this
     // launch sequence, computes nothing (but joins the slice sums)
-    const bool act = it < end && s.live;
+    const bool act = it < n_items && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
     const RowWin ad = solve_windows(s);
     const int32_t i = lb * kBlock + tid;
     // the running sum of this block over the interval, read before the node
     // work so that its latency overlaps the gathers
-    const double prev = REDUCE && accum && tid == 0 && act ? s.partial[lb] : 0.0;
+    const double prev = REDUCE && accum && tid == 0 && act ? device_ptr(s.partial)[lb] : 0.0;
     double jx = 0.0;
     if (act && i < s.n)
-      jx = bgk_node<L, RowWin, false, false, REDUCE>(static_cast<const double*>(s.f[p]),
-                                                     static_cast<double*>(s.f[p ^ 1]), ad, i, s.NP, s.a,
+      jx = bgk_node<L, RowWin, false, false, REDUCE>(static_cast<const double*>(device_ptr(s.f[p])),
+                                                     static_cast<double*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, s.a,
                                                      nullptr, nullptr);
     if (REDUCE) {
       const double t = slice_sum<NS>(jx);
-      if (act && tid == 0) s.partial[lb] = accum ? prev + t : t;
+      if (act && tid == 0) device_ptr(s.partial)[lb] = accum ? prev + t : t;
     }
   }
 }
@@ -600,17 +599,15 @@ __global__ __launch_bounds__(kBlock) void k_cg(const double* __restrict__ fin,
 template <class L, bool REDUCE, int NS>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi(const BatchSolve* __restrict__ solves,
                                                               const uint32_t* __restrict__ items, int32_t n_items,
-                                                              int32_t per_wg, int32_t parity) {
+                                                              int32_t parity) {
   constexpr int Q = L::nQ;
-  const int32_t g = node_block(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t sub = static_cast<int32_t>(threadIdx.x) / kBlock, tid = static_cast<int32_t>(threadIdx.x) % kBlock;
-  const int32_t beg = g * per_wg;
-  const int32_t end = beg + per_wg < n_items ? beg + per_wg : n_items;
-  for (int32_t base = beg; base < end; base += NS) {
-    const int32_t it = base + sub;
-    const uint32_t item = items[it < end ? it : base];
+  const int32_t np = batch_positions<NS>(n_items);
+  for (int32_t pos = static_cast<int32_t>(blockIdx.x); pos < np; pos += static_cast<int32_t>(gridDim.x)) {
+    const int32_t it = batch_item<NS>(pos, sub);
+    const uint32_t item = wave_item(items, it < n_items ? it : n_items - 1);
     const BatchSolve& s = solves[item >> kItemShift];
-    const bool act = it < end && s.live;
+    const bool act = it < n_items && s.live;
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
     const int p = (parity ^ s.parity) & 1;
     const RowWin ad = solve_windows(s);
@@ -618,10 +615,10 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi(const BatchSolve* 
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     if (act && i < s.n) {
       double f[2][Q];
-      load_node<L, 2, false>(static_cast<const double*>(s.f[p]), ad, i, s.NP, f);
+      load_node<L, 2, false>(static_cast<const double*>(device_ptr(s.f[p])), ad, i, s.NP, f);
       const double r0 = qsum<L>(f[0]);
       const double r1 = qsum<L>(f[1]);
-      static_cast<double*>(s.phi)[i] = (r0 - r1) / (r0 + r1);
+      static_cast<double*>(device_ptr(s.phi))[i] = (r0 - r1) / (r0 + r1);
       if (REDUCE) {
         double ft[Q];
 #pragma unroll
@@ -639,9 +636,9 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi(const BatchSolve* 
       s1 = slice_sum<NS>(s1);
       s2 = slice_sum<NS>(s2);
       if (act && tid == 0) {
-        s.partial[lb] = s0;
-        s.partial[nb + lb] = s1;
-        s.partial[2 * nb + lb] = s2;
+        device_ptr(s.partial)[lb] = s0;
+        device_ptr(s.partial)[nb + lb] = s1;
+        device_ptr(s.partial)[2 * nb + lb] = s2;
       }
     }
   }
@@ -650,16 +647,14 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi(const BatchSolve* 
 template <class L, int NS>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_cg(const BatchSolve* __restrict__ solves,
                                                           const uint32_t* __restrict__ items, int32_t n_items,
-                                                          int32_t per_wg, int32_t parity) {
+                                                          int32_t parity) {
   constexpr int D = L::nD;
-  const int32_t g = node_block_rev(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
   const int32_t sub = static_cast<int32_t>(threadIdx.x) / kBlock, tid = static_cast<int32_t>(threadIdx.x) % kBlock;
-  const int32_t beg = g * per_wg;
-  const int32_t end = beg + per_wg < n_items ? beg + per_wg : n_items;
-  for (int32_t base = beg; base < end; base += NS) {
-    const int32_t it = base + sub;
-    if (it >= end) continue;
-    const uint32_t item = items[it];
+  const int32_t np = batch_positions<NS>(n_items);
+  for (int32_t pos = static_cast<int32_t>(blockIdx.x); pos < np; pos += static_cast<int32_t>(gridDim.x)) {
+    const int32_t it = batch_item<NS>(np - 1 - pos, sub);  // from the end, where pass 1 ended
+    if (it >= n_items) continue;
+    const uint32_t item = wave_item(items, it);
     const BatchSolve& s = solves[item >> kItemShift];
     if (!s.live) continue;  // stopped at an earlier check of this launch sequence
     const int32_t lb = static_cast<int32_t>(item & kItemMask);
@@ -676,8 +671,8 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg(const BatchSolve* __re
 #pragma unroll
     for (int d = 0; d < D; ++d) F[d] = s.a.F[d];
     const WallPhi wp{nullptr, s.phi_w};
-    cg_node<L, false, false, true>(static_cast<const double*>(s.f[p]), static_cast<double*>(s.f[p ^ 1]), ad, i, s.NP, a,
-                             static_cast<const double*>(s.phi), wp, F, nullptr, nullptr);
+    cg_node<L, false, false, true>(static_cast<const double*>(device_ptr(s.f[p])), static_cast<double*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, a,
+                             static_cast<const double*>(device_ptr(s.phi)), wp, F, nullptr, nullptr);
   }
 }
 
@@ -975,32 +970,32 @@ hipError_t prestream_f64(int lattice, const RowWin& ad, const double* r0, int32_
 }
 
 hipError_t batch_cg_f64(int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                        int32_t n_items, int32_t grid, int32_t per_wg, int32_t parity, int ns, hipStream_t s) {
+                        int32_t n_items, int32_t grid, int32_t parity, int ns, hipStream_t s) {
   LB_DISPATCH_LATTICE(lattice, L, {
     const dim3 g(grid), b(kBlock), b2(2 * kBlock);
     if (ns == 2) {
-      if (reduce) k_batch_cg_phi<L, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity);
-      else k_batch_cg_phi<L, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity);
-      k_batch_cg<L, 2><<<g, b2, 0, s>>>(solves, items, n_items, per_wg, parity);
+      if (reduce) k_batch_cg_phi<L, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
+      else k_batch_cg_phi<L, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
+      k_batch_cg<L, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
     } else {
-      if (reduce) k_batch_cg_phi<L, true, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity);
-      else k_batch_cg_phi<L, false, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity);
-      k_batch_cg<L, 1><<<g, b, 0, s>>>(solves, items, n_items, per_wg, parity);
+      if (reduce) k_batch_cg_phi<L, true, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      else k_batch_cg_phi<L, false, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      k_batch_cg<L, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
     }
   });
   return hipGetLastError();
 }
 
 hipError_t batch_bgk_f64(int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                         int32_t n_items, int32_t grid, int32_t per_wg, int32_t parity, int ns, bool accum, hipStream_t s) {
+                         int32_t n_items, int32_t grid, int32_t parity, int ns, bool accum, hipStream_t s) {
   LB_DISPATCH_LATTICE(lattice, L, {
     const dim3 b(kBlock * (ns == 2 ? 2 : 1));
     if (ns == 2) {
-      if (reduce) k_batch_bgk<L, true, 2><<<dim3(grid), b, 0, s>>>(solves, items, n_items, per_wg, parity, accum ? 1 : 0);
-      else k_batch_bgk<L, false, 2><<<dim3(grid), b, 0, s>>>(solves, items, n_items, per_wg, parity, accum ? 1 : 0);
+      if (reduce) k_batch_bgk<L, true, 2><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
+      else k_batch_bgk<L, false, 2><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
     } else {
-      if (reduce) k_batch_bgk<L, true, 1><<<dim3(grid), b, 0, s>>>(solves, items, n_items, per_wg, parity, accum ? 1 : 0);
-      else k_batch_bgk<L, false, 1><<<dim3(grid), b, 0, s>>>(solves, items, n_items, per_wg, parity, accum ? 1 : 0);
+      if (reduce) k_batch_bgk<L, true, 1><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
+      else k_batch_bgk<L, false, 1><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
     }
   });
   return hipGetLastError();
