@@ -595,27 +595,35 @@ __device__ __forceinline__ void cg_collide(const double (&t)[L::nQ], const doubl
   const double omt = 1.0 - ti;
   const double r45 = 4.5 * rho, r3 = 3.0 * rho;
   Pair<S>* __restrict__ out = elem_ptr<O>(reinterpret_cast<Pair<S>*>(gout), pidx<Q>(0, i));
-#pragma unroll
-  for (int q = 0; q < Q; ++q) {
+  // Directions in pairs: the terms even in c_q are the same for both, the odd
+  // ones (3 rho cu, 3 cF, the recolouring) change their sign, exactly (192^3
+  // pack: FP16S 151 us per step for 155, FP32S 222 for 223).
+  auto put = [&](int q, double geq, double dF, double st, double rc) {
     const double w = L::w(q);
-    const double cu = cdot<L>(q, u);
-    const double cF = cdot<L>(q, F);
-    const double cg = cdot<L>(q, g);
-    const double geq = w * (a0 + r45 * cu * cu + r3 * cu);
-    const double dF = (w * tf) * (9.0 * cF * cu + m3uF + 3.0 * cF);
-    double st, rc;
-    if (q < Q - 1) {
-      st = af * (w * cg * cg - L::B(q));
-      rc = rfb * w * cg * (1.0 / L::cNorm(q));
-    } else {
-      st = -af * L::B(q);
-      rc = 0.0;
-    }
     const double bs = omt * t[q] + ti * geq + dF + st;
     const float bt = static_cast<float>(bs);
     const float bd = static_cast<float>(phi_n * (w + bs) + 2.0 * rc);
     const Pair<S> v{Store<S>::put_sr(bt, sr_bits(hn, q)), Store<S>::put_sr(bd, sr_bits(hn, q + 32))};
     st_elem<NT>(v, out + (q << kPLog));
+  };
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int rq = L::rev(q);
+    if (rq < q) continue;
+    const double w = L::w(q), wt = w * tf;
+    const double cu = cdot<L>(q, u);
+    const double cF = cdot<L>(q, F);
+    const double ev = a0 + r45 * cu * cu;
+    const double fev = 9.0 * cF * cu + m3uF;
+    if (rq == q) {  // rest
+      put(q, w * (ev + r3 * cu), wt * (fev + 3.0 * cF), -af * L::B(q), 0.0);
+      continue;
+    }
+    const double cg = cdot<L>(q, g);
+    const double st = af * (w * cg * cg - L::B(q));
+    const double rc = rfb * w * cg * (1.0 / L::cNorm(q));
+    put(q, w * (ev + r3 * cu), wt * (fev + 3.0 * cF), st, rc);
+    put(rq, w * (ev - r3 * cu), wt * (fev - 3.0 * cF), st, -rc);
   }
 }
 
