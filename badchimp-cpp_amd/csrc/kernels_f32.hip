@@ -175,7 +175,7 @@ __device__ __forceinline__ void load_g(const S* __restrict__ gin, const A& ad, i
 template <class L>
 __device__ __forceinline__ float rheology_visc_lp(const float (&g)[L::nQ], float a0, float r45, float r3,
                                                   const float* u, const float (&F)[3], const float* __restrict__ sr,
-                                                  const float* __restrict__ nu, int n) {
+                                                  const float* __restrict__ nu, int n, const float* lds) {
   constexpr int Q = L::nQ, D = L::nD;
   float E[D][D];
 #pragma unroll
@@ -209,8 +209,11 @@ __device__ __forceinline__ float rheology_visc_lp(const float (&g)[L::nQ], float
       sq += 2.0f * E[i][j] * E[i][j];
     }
   }
-  const int k = table_index(sr, n, sq);
-  return (nu[k + 1] - nu[k]) * (sq - sr[k]) / (sr[k + 1] - sr[k]) + nu[k];
+  auto visc = [&](auto s, auto v) {
+    const int k = table_index(s, n, sq);
+    return (v[k + 1] - v[k]) * (sq - s[k]) / (s[k + 1] - s[k]) + v[k];
+  };
+  return n <= kTableLds ? visc(lds_ptr(lds), lds_ptr(lds) + kTableLds) : visc(sr, nu);
 }
 
 // One node of the BGK + Guo step on shifted populations; returns j_x (FP64)
@@ -226,7 +229,7 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
                                               double* __restrict__ vel_o, float tauA_inv = 0.0f,
                                               float tauA_factor = 0.0f, const float* __restrict__ sr = nullptr,
                                               const float* __restrict__ nu = nullptr, int tab_n = 0,
-                                              uint32_t step = 0) {
+                                              uint32_t step = 0, const float* table = nullptr) {
   constexpr int Q = L::nQ, D = L::nD;
   const SrSeed hn = sr_node(i, step);  // unused (removed) for float storage
   float g[Q];
@@ -256,7 +259,7 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
   const float m3uF = -3.0f * dot<L>(u, F);
   const float r45 = 4.5f * rho, r3 = 3.0f * rho;
   if constexpr (MODE == kRheology) {
-    const float visc = rheology_visc_lp<L>(g, a0, r45, r3, u, F, sr, nu, tab_n);
+    const float visc = rheology_visc_lp<L>(g, a0, r45, r3, u, F, sr, nu, tab_n, table);
     const float tau = visc * 3.0f / rho + 0.5f;
     tau_inv = 1.0f / tau;
     tau_factor = 1.0f - 0.5f / tau;
@@ -332,11 +335,13 @@ __global__ __launch_bounds__(kBlock) void k_bgk_lp(const S* __restrict__ gin, S*
   const int32_t i = b * kBlock + threadIdx.x;
   // the block's running sum, read before the node work (latency overlapped)
   const double prev = REDUCE && accum && threadIdx.x == 0 ? partial[b] : 0.0;
+  __shared__ float table[MODE == kRheology ? 2 * kTableLds : 1];
+  if (MODE == kRheology && tab_n <= kTableLds) table_to_lds(sr, nu, tab_n, table);
   double jx = 0.0;
   if (i < n) {
     const float F[3] = {F0, F1, F2};
     jx = bgk_node_lp<L, S, A, FIRST, STORE, REDUCE, MODE, NT>(gin, gout, ad, i, NP, tau_inv, tau_factor, F, rho_o,
-                                                          vel_o, tauA_inv, tauA_factor, sr, nu, tab_n, step);
+                                                          vel_o, tauA_inv, tauA_factor, sr, nu, tab_n, step, table);
   }
   if (REDUCE) {
     const double s = block_sum(jx);

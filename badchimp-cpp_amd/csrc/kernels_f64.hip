@@ -117,7 +117,7 @@ __device__ __forceinline__ double strided_sum(const double* __restrict__ partial
 // out: a sum that starts at +0 never holds -0, so adding +-0 never changes it.
 template <class L>
 __device__ __forceinline__ double rheology_visc(const double (&f)[L::nQ], double rho, const double* u,
-                                                double c2u2, const BgkArgs& a) {
+                                                double c2u2, const BgkArgs& a, const double* lds) {
   constexpr int Q = L::nQ, D = L::nD;
   double S[D][D];
 #pragma unroll
@@ -152,10 +152,11 @@ __device__ __forceinline__ double rheology_visc(const double (&f)[L::nQ], double
       sq += (2 * S[i][j]) * S[i][j];
     }
   }
-  const double* __restrict__ sr = a.tab_sr;
-  const double* __restrict__ nu = a.tab_nu;
-  const int k = table_index(sr, a.tab_n, sq);
-  return ((nu[k + 1] - nu[k]) * (sq - sr[k])) / (sr[k + 1] - sr[k]) + nu[k];
+  auto visc = [&](auto sr, auto nu) {
+    const int k = table_index(sr, a.tab_n, sq);
+    return ((nu[k + 1] - nu[k]) * (sq - sr[k])) / (sr[k + 1] - sr[k]) + nu[k];
+  };
+  return a.tab_n <= kTableLds ? visc(lds_ptr(lds), lds_ptr(lds) + kTableLds) : visc(a.tab_sr, a.tab_nu);
 }
 
 // One node of the std_case loop body (std_case/main.cpp:110-145); returns the
@@ -168,7 +169,7 @@ __device__ __forceinline__ double rheology_visc(const double (&f)[L::nQ], double
 template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
 __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, double* __restrict__ fout, const A& ad,
                                            int32_t i, int64_t NP, const BgkArgs& a, double* __restrict__ rho_o,
-                                           double* __restrict__ vel_o) {
+                                           double* __restrict__ vel_o, const double* table = nullptr) {
   constexpr int Q = L::nQ, D = L::nD;
   double jx = 0.0;
   double f[1][Q];
@@ -197,21 +198,28 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
   // per wave instead of 640 (64^3 pack: 7.8 us for 8.0), the two-phase collision
   // 1237 instead of 1402 (FP64 64^3 21.2 us for 21.8, 192^3 436 for 438).
   if constexpr (MODE == kRheology) {
-    const double visc = rheology_visc<L>(f[0], rho, u, c2u2, a);
+    const double visc = rheology_visc<L>(f[0], rho, u, c2u2, a, table);
     // tau_ = visc_ * c2Inv / rho + 0.5 (LBrheology.h:463); calcDeltaOmegaF's
     // tau_factor at that tau (LBcollision.h:206)
     const double tau = (visc * L::c2Inv) / rho + 0.5;
     const double tau_inv = 1.0 / tau;
     const double tau_factor = 1 - 0.5 / tau;
     if (STORE) rho_o[NP + i] = visc;
+    auto put = [&](int q, double feq, double dF) {
+      const double om = (-tau_inv) * (f[0][q] - feq);
+      st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
+    };
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
+      const int r = L::rev(q);
+      if (r < q) continue;
       const double cu = cdot<L>(q, u);
       const double cF = cdot<L>(q, a.F);
-      const double feq = (L::w(q) * rho) * ((1 + L::c2Inv * cu) + L::c4Inv0_5 * (cu * cu - c2u2));
-      const double om = (-tau_inv) * (f[0][q] - feq);
-      const double dF = (L::w(q) * tau_factor) * (L::c2Inv * cF + L::c4Inv * (cF * cu - c2uF));
-      st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
+      const double wr = L::w(q) * rho, wt = L::w(q) * tau_factor;
+      const double odd = L::c2Inv * cu, even = L::c4Inv0_5 * (cu * cu - c2u2);
+      const double oddF = L::c2Inv * cF, evenF = L::c4Inv * (cF * cu - c2uF);
+      put(q, wr * ((1 + odd) + even), wt * (oddF + evenF));
+      if (r != q) put(r, wr * ((1 - odd) + even), wt * (evenF - oddF));
     }
     return jx;
   }
@@ -267,8 +275,10 @@ __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
   const int32_t i = b * kBlock + threadIdx.x;
   // the block's running sum, read before the node work (latency overlapped)
   const double prev = REDUCE && accum && threadIdx.x == 0 ? partial[b] : 0.0;
+  __shared__ double table[MODE == kRheology ? 2 * kTableLds : 1];
+  if (MODE == kRheology && a.tab_n <= kTableLds) table_to_lds(a.tab_sr, a.tab_nu, a.tab_n, table);
   double jx = 0.0;
-  if (i < n) jx = bgk_node<L, A, FIRST, STORE, REDUCE, MODE, NT>(fin, fout, ad, i, NP, a, rho_o, vel_o);
+  if (i < n) jx = bgk_node<L, A, FIRST, STORE, REDUCE, MODE, NT>(fin, fout, ad, i, NP, a, rho_o, vel_o, table);
   if (REDUCE) {
     const double s = block_sum(jx);
     if (threadIdx.x == 0) partial[b] = accum ? prev + s : s;
