@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <string>
 #include <utility>
@@ -10,6 +11,7 @@
 
 #include "../../include/badchimp_amd.h"
 #include "addressing.hpp"
+#include "host_threads.hpp"
 #include "lattice.hpp"
 
 namespace lbamd {
@@ -144,11 +146,12 @@ inline bool build_windows(const RowBuild& rb, bool allow_periodic, WinBuild& wb,
   wb.win.assign(static_cast<size_t>(PX) * wb.PY * wb.W, 0u);
   wb.count.assign(pz ? static_cast<size_t>(PX) * wb.PY : 0u, 0u);
   wb.plane.assign(planes || rb.coord.size() >= kMax ? static_cast<size_t>(PX) : 0u, 0u);
-  for (int32_t px = 0; px < PX; ++px) {
+  // the nodes of a plane are consecutive (one plane per tile along X)
+  static_assert(kTileLogX == 0, "x planes are not consecutive in the compact order");
+  std::atomic<bool> fits{true};
+  auto plane = [&](int32_t px) {
     int32_t X = px - 1;
-    if (!RowGeom::wrap(X, g.E[0], g.periodic & 1)) continue;
-    // the nodes of a plane are consecutive (one plane per tile along X)
-    static_assert(kTileLogX == 0, "x planes are not consecutive in the compact order");
+    if (!RowGeom::wrap(X, g.E[0], g.periodic & 1)) return;
     const uint32_t base = wb.plane.empty() ? 0u : rb.rows[static_cast<size_t>(g.row(X, 0)) * g.W].x;
     if (!wb.plane.empty()) wb.plane[px] = base;
     for (int32_t py = 0; py < wb.PY; ++py) {
@@ -156,35 +159,36 @@ inline bool build_windows(const RowBuild& rb, bool allow_periodic, WinBuild& wb,
       if (!RowGeom::wrap(Y, g.E[1], g.periodic & 2)) continue;
       const uint2* words = &rb.rows[static_cast<size_t>(g.row(X, Y)) * g.W];  // 32 cells each, no bits beyond E_Z
       const size_t pr = static_cast<size_t>(px) * wb.PY + py;
-      auto cell = [&](int32_t z) -> uint32_t {
-        if (pz) z = z < 0 ? z + EZ : (z >= EZ ? z - EZ : z);
-        return z < 0 || z >= EZ ? 0u : (words[z >> 5].y >> (z & 31)) & 1u;
-      };
-      for (int32_t w = 0; w < wb.W; ++w) {
-        const int32_t z0 = w << kWinLog, h = z0 & 31;
-        const uint2 e = words[z0 >> 5];
-        const uint32_t first = e.x + static_cast<uint32_t>(__builtin_popcount(e.y & ((1u << h) - 1u))) - base;
-        if (first >= kMax) {
-          why = "x plane above 2^22 nodes";
-          return false;
+      uint32_t* out = &wb.win[pr * wb.W];
+      const uint32_t row0 = words[0].y & 1u, rowN = (words[g.W - 1].y >> ((EZ - 1) & 31)) & 1u;
+      uint32_t before = pz ? rowN : 0u;  // the cell before the word
+      for (int32_t k = 0; k < g.W; ++k) {
+        const uint32_t y = words[k].y, next = k + 1 < g.W ? words[k + 1].y & 1u : 0u;
+        uint32_t first = words[k].x - base;
+        for (int32_t w = 4 * k; w < std::min(4 * k + 4, wb.W); ++w) {
+          const int32_t h = (w & 3) << kWinLog;
+          const uint32_t cells = (y >> h) & 0xffu;
+          const uint32_t after = h < 24 ? (y >> (h + 8)) & 1u : next;
+          uint32_t bits = before | (cells << 1) | (after << 9);
+          // the cell after the row's last one is its first
+          if (pz && w == wb.W - 1) bits |= row0 << (EZ - (w << kWinLog) + 1);
+          if (first >= kMax) fits = false;
+          out[w] = (bits << kWinBase) | (first & (kMax - 1u));
+          first += static_cast<uint32_t>(__builtin_popcount(cells));
+          before = cells >> 7;
         }
-        // cells 8w .. 8w+7 lie in one 32-cell word; the two beside them by cell
-        uint32_t bits = ((e.y >> h) & ((1u << kWinCells) - 1u)) << 1;
-        bits |= cell(z0 - 1);
-        const int32_t end = z0 + static_cast<int32_t>(kWinCells);
-        if (end <= EZ) {
-          bits |= cell(end) << (kWinCells + 1);
-        } else {
-          // the row ends inside the word: the cell after the last one wraps
-          bits |= cell(EZ) << (EZ - z0 + 1);
-        }
-        wb.win[pr * wb.W + w] = (bits << kWinBase) | first;
       }
-      if (pz) {
-        const uint2 last = words[g.W - 1];
-        wb.count[pr] = last.x + static_cast<uint32_t>(__builtin_popcount(last.y)) - words[0].x;
-      }
+      if (pz) wb.count[pr] = words[g.W - 1].x + static_cast<uint32_t>(__builtin_popcount(words[g.W - 1].y)) - words[0].x;
     }
+  };
+  // (parallel_ranges counts items of about a cell's work)
+  const int64_t per = static_cast<int64_t>(wb.PY) * wb.W;
+  parallel_ranges(PX * per, [&](int64_t b, int64_t e, int) {
+    for (int64_t px = (b + per - 1) / per; px * per < e; ++px) plane(static_cast<int32_t>(px));
+  });
+  if (!fits) {
+    why = "x plane above 2^22 nodes";
+    return false;
   }
   return true;
 }
@@ -229,8 +233,8 @@ inline std::vector<uint8_t> block_xcd(const std::vector<uint32_t>& coord) {
   const int64_t n = static_cast<int64_t>(coord.size()), nb = (n + kBlock - 1) / kBlock;
   std::vector<uint8_t> xcd(static_cast<size_t>(nb));
   std::vector<int64_t> start;  // first node of each plane
-  for (int64_t i = 0; i < n; ++i)
-    if (i == 0 || (coord[i] >> 22) != (coord[i - 1] >> 22)) start.push_back(i);
+  for (auto it = coord.begin(); it != coord.end(); it = std::upper_bound(it, coord.end(), *it | 0x3fffffu))
+    start.push_back(it - coord.begin());
   if (nb < 2 * static_cast<int64_t>(start.size())) {
     const int64_t run = std::min<int64_t>(32, (nb + 7) / 8);
     for (int64_t b = 0; b < nb; ++b) xcd[b] = static_cast<uint8_t>((b / run) % 8);
