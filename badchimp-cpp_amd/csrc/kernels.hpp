@@ -54,6 +54,12 @@ hipError_t unstage_f64(int lattice, int nf, const double* g, double* f, int32_t 
 hipError_t init_eq_f64(int lattice, double* f, int nf, int field, int32_t n, int64_t NP,
                        const double* rho, const double* vel, hipStream_t s);
 
+// nc components (src[c stride + i], float or double) of the nodes at positions
+// [p0, p0 + m) of the ascending node order to pinned host memory, interleaved;
+// node[p]: compact index at position p, null where it is p.
+hipError_t nodes_out(const void* src, bool is_float, int64_t stride, int nc, const int32_t* node, int64_t p0,
+                     int64_t m, double* out, hipStream_t s);
+
 // ---- tagged boundaries (std_one_phase/main.cpp:27-204, 513-575) -------------
 // One step with the tag-derived pull table ad, the anti-bounce-back
 // direction masks abb, the domain labels/mass-source flags info, the force

@@ -833,6 +833,22 @@ __global__ __launch_bounds__(kBlock) void k_finish_momx(const double* __restrict
   }
 }
 
+// Node fields for the host: the nc components src[c stride + i] of the nodes at
+// the positions [p0, p0 + m) of the ascending node order, component after
+// component per node, as doubles.  node[p]: compact index at position p (null:
+// the same).  out is pinned host memory, written across the link in full lines;
+// it takes the same time as a copy of those bytes, and the reorder nothing.
+template <typename T, int NC>
+__global__ __launch_bounds__(kBlock) void k_nodes_out(const T* __restrict__ src, int64_t stride,
+                                                      const int32_t* __restrict__ node, int64_t p0, int64_t m,
+                                                      double* __restrict__ out) {
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (e >= m * NC) return;
+  const int64_t p = p0 + e / NC;
+  const int64_t i = node ? node[p] : p;
+  out[e] = static_cast<double>(src[(e % NC) * stride + i]);
+}
+
 inline dim3 grid_for(int32_t n) { return dim3(static_cast<unsigned>((n + kBlock - 1) / kBlock)); }
 
 }  // namespace
@@ -1058,6 +1074,23 @@ hipError_t batch_rest_f64(int lattice, double* f, int64_t NP, hipStream_t s) {
     const int64_t n = static_cast<int64_t>(L::nQ) * NP;
     k_batch_rest<L><<<dim3(static_cast<unsigned>((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s>>>(f, NP);
   });
+  return hipGetLastError();
+}
+
+hipError_t nodes_out(const void* src, bool is_float, int64_t stride, int nc, const int32_t* node, int64_t p0,
+                     int64_t m, double* out, hipStream_t s) {
+  if (m <= 0) return hipSuccess;
+  const dim3 g(static_cast<unsigned>((m * nc + kBlock - 1) / kBlock)), b(kBlock);
+  if (is_float) {
+    if (nc != 1) return hipErrorInvalidValue;
+    k_nodes_out<float, 1><<<g, b, 0, s>>>(static_cast<const float*>(src), stride, node, p0, m, out);
+  } else {
+    const double* d = static_cast<const double*>(src);
+    if (nc == 1) k_nodes_out<double, 1><<<g, b, 0, s>>>(d, stride, node, p0, m, out);
+    else if (nc == 2) k_nodes_out<double, 2><<<g, b, 0, s>>>(d, stride, node, p0, m, out);
+    else if (nc == 3) k_nodes_out<double, 3><<<g, b, 0, s>>>(d, stride, node, p0, m, out);
+    else return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
