@@ -53,6 +53,7 @@ struct lb_ctx {
     uint32_t* d_send_nodes = nullptr;
     uint32_t* d_recv_nodes = nullptr;
     double* d_buf = nullptr;
+    double* h_buf = nullptr;  // the same in pinned host memory
   };
   std::vector<Halo> halos;
   std::vector<int16_t> node_type;
