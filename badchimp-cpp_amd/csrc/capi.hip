@@ -205,6 +205,9 @@ int pre_state(lb_ctx* c, const void** out) {
   return LB_OK;
 }
 
+// nodes per host thread of the set-up passes that look at every link of a node
+constexpr int64_t kMinNodes = 8192;
+
 // Row layout of a node list (positions and neighbour index).  Returns false
 // with a reason when the node list is not a set of cells of one box that the
 // layout can address.
@@ -248,7 +251,7 @@ bool build_rows(int lattice, int32_t n_nodes, const int32_t* nb, const int32_t* 
         }
       }
     }
-  });
+  }, kMinNodes);
   int32_t lo[3], hi[3], period[3] = {0, 0, 0};
   for (int a = 0; a < 3; ++a) { lo[a] = tlo[0][a]; hi[a] = thi[0][a]; }
   for (int t = 0; t < kMaxHostThreads; ++t) {
@@ -484,7 +487,7 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
       }
       wall_dirs[i] = wd;
     }
-  });
+  }, kMinNodes);
   // the first refused link in (compact node, direction) order, as one pass
   // over the nodes would find it
   const LinkError* first = std::min_element(err, err + kMaxHostThreads,
@@ -530,7 +533,7 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
             break;
           }
         }
-    });
+    }, kMinNodes);
     return std::none_of(bad, bad + kMaxHostThreads, [](bool x) { return x; });
   };
   if (rows_ok && !agrees([&](int q, int32_t i) { return row_source(c->lattice, rb, q, i); })) {
