@@ -244,7 +244,10 @@ struct RowWinT : WinWrap<PZ> {
   // vector offset plus a per-direction uniform base.
   template <class L>
   __device__ __forceinline__ void rows(int32_t i, Rows<L>& r) const {
-    const uint32_t c = coord[i];
+    cell_rows<L>(coord[i], r);
+  }
+  template <class L>
+  __device__ __forceinline__ void cell_rows(uint32_t c, Rows<L>& r) const {
     const uint32_t X = c >> 22, Y = (c >> 12) & 1023u, Z = c & 4095u;
     r.t = kWinBase + (Z & (kWinCells - 1u));
     const uint32_t pr = (X + 1u) * static_cast<uint32_t>(PY) + (Y + 1u);
@@ -285,6 +288,10 @@ struct RowWinT : WinWrap<PZ> {
   __device__ __forceinline__ void sources(int32_t i, uint32_t (&src)[L::nQ - 1]) const {
     Rows<L> r;
     rows<L>(i, r);
+    row_sources<L>(i, r, src);
+  }
+  template <class L>
+  __device__ __forceinline__ static void row_sources(int32_t i, const Rows<L>& r, uint32_t (&src)[L::nQ - 1]) {
 #pragma unroll
     for (int q = 0; q < L::nQ - 1; ++q) {
       // both candidates, combined by a mask: a per-lane select, not a branch

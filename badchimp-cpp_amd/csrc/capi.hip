@@ -604,6 +604,7 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
         LB_HIP(c, hipMemcpy(c->d_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice));
       }
       c->addr.layout = nc ? kLayWinZ : kLayWin;
+      c->tile_box = TileBox{rb.g.E[0], rb.g.E[2], rb.g.periodic & 1};
       if (nc) {
         set(c->addr.winz);
         c->addr.winz.count = c->d_win + nw + np;
@@ -1086,11 +1087,27 @@ hipError_t launch_single(lb_ctx* c, const BgkArgs& a, int from, bool first, bool
 constexpr int32_t kGraphSteps = 128;
 constexpr int32_t kGraphMinSteps = 2 * kGraphSteps;
 
+// Small D2Q9 lists take kTileSteps steps per launch (tile2d.hpp): the box of
+// the row windows in at most kTileMaxTiles tiles, an operator without a table.
+bool tiled(const lb_ctx* c, const BgkArgs& a) {
+  return c->lattice == LB_D2Q9 && c->precision != LB_FP16S && c->addr.layout == kLayWin && a.mode != kRheology &&
+         c->tile_box.tiles() <= kTileMaxTiles;
+}
+
+hipError_t launch_tile(lb_ctx* c, const BgkArgs& a, int from) {
+  if (c->precision == LB_FP64)
+    return bgk_tile_f64(static_cast<const double*>(c->d_f[from]), static_cast<double*>(c->d_f[1 - from]), c->addr.win,
+                        c->tile_box, a, c->stream);
+  return bgk_tile_f32s(static_cast<const float*>(c->d_f[from]), static_cast<float*>(c->d_f[1 - from]), c->addr.win,
+                       c->tile_box, a, c->stream);
+}
+
 int step_single(lb_ctx* c, int32_t nsteps, const BgkArgs& a) {
   hipSetDevice(c->device);
   Timer t(c);
-  auto advance = [c](int32_t n) {
-    if (n & 1) c->cur = 1 - c->cur;
+  // n steps in some launches, each of which changes the buffer
+  auto advance = [c](int32_t n, int32_t launches) {
+    if (launches & 1) c->cur = 1 - c->cur;
     c->post = true;
     c->step_count += static_cast<uint32_t>(n);
     c->cg_colour_done = false;
@@ -1102,16 +1119,22 @@ int step_single(lb_ctx* c, int32_t nsteps, const BgkArgs& a) {
     if (!c->post) {
       hipError_t e = launch_single(c, a, c->cur, true, false);
       if (e != hipSuccess) return fail(c, LB_ERR_HIP, "bgk launch: %s", hipGetErrorString(e));
-      advance(1);
+      advance(1, 1);
       ++s;
     }
-    const int32_t replays = (nsteps - s - 1) / kGraphSteps;
+    // launches of `per` steps each; an even number of them returns to the
+    // buffer it started from
+    const int32_t per = tiled(c, a) ? kTileSteps : 1;
+    const int32_t launches = per == 1 ? kGraphSteps : kGraphSteps / (2 * per) * 2;
+    const int32_t replays = (nsteps - s - 1) / (per * launches);
     if (replays > 0) {
       hipGraph_t graph = nullptr;
       hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
       if (e != hipSuccess) return fail(c, LB_ERR_HIP, "graph capture: %s", hipGetErrorString(e));
-      for (int32_t k = 0; k < kGraphSteps && e == hipSuccess; ++k)
-        e = launch_single(c, a, (k & 1) ? 1 - c->cur : c->cur, false, false);
+      for (int32_t k = 0; k < launches && e == hipSuccess; ++k) {
+        const int from = (k & 1) ? 1 - c->cur : c->cur;
+        e = per == 1 ? launch_single(c, a, from, false, false) : launch_tile(c, a, from);
+      }
       const hipError_t e2 = hipStreamEndCapture(c->stream, &graph);
       if (e == hipSuccess) e = e2;
       if (e == hipSuccess) e = hipGraphInstantiate(&run, graph, nullptr, nullptr, 0);
@@ -1124,12 +1147,15 @@ int step_single(lb_ctx* c, int32_t nsteps, const BgkArgs& a) {
         }
         return fail(c, LB_ERR_HIP, "step graph: %s", hipGetErrorString(e));
       }
-      advance(kGraphSteps * replays);
-      s += kGraphSteps * replays;
+      advance(per * launches * replays, launches * replays);
+      s += per * launches * replays;
     }
   }
-  for (; s < nsteps; ++s) {
-    hipError_t e = launch_single(c, a, c->cur, !c->post, s == nsteps - 1);
+  const bool tiles = tiled(c, a);
+  while (s < nsteps) {
+    // tiles for what is left before the last step (it stores rho and u)
+    const bool tile = tiles && c->post && s + kTileSteps < nsteps;
+    hipError_t e = tile ? launch_tile(c, a, c->cur) : launch_single(c, a, c->cur, !c->post, s == nsteps - 1);
     if (e != hipSuccess) {
       if (run) {
         hipStreamSynchronize(c->stream);
@@ -1137,7 +1163,8 @@ int step_single(lb_ctx* c, int32_t nsteps, const BgkArgs& a) {
       }
       return fail(c, LB_ERR_HIP, "bgk launch: %s", hipGetErrorString(e));
     }
-    advance(1);
+    advance(tile ? kTileSteps : 1, 1);
+    s += tile ? kTileSteps : 1;
   }
   const int rc = t.stop(nsteps);
   if (run) hipGraphExecDestroy(run);  // the stream has drained (t.stop waits for it)

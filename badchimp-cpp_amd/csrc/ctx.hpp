@@ -61,6 +61,7 @@ struct lb_ctx {
   uint32_t* d_coord = nullptr;      // row layout: packed cell coordinates
   uint2* d_rows = nullptr;          // row layout: {base, mask} per (row, word)
   uint32_t* d_win = nullptr;        // row windows: words, first nodes of the x planes, row counts (WinBuild)
+  lbamd::TileBox tile_box{0, 0, 0}; // D2Q9 row windows: the box
   int32_t* d_order = nullptr;       // row windows: block order, or null
   lbamd::Addr addr;                 // layout used by the single-phase kernels
   std::string layout_note;          // "rows", or why the table layout is used

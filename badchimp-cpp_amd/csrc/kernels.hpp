@@ -7,6 +7,7 @@
 #include "addressing.hpp"
 #include "context.hpp"
 #include "layout_select.hpp"
+#include "tile2d.hpp"
 
 namespace lbamd {
 
@@ -28,6 +29,13 @@ struct Addr {
 hipError_t bgk_f64(int lattice, bool first, bool store, bool reduce, const double* fin,
                    double* fout, const Addr& ad, int32_t n, int64_t NP, const BgkArgs& a,
                    double* rho, double* vel, double* partial, hipStream_t s, bool accum = false);
+
+// kTileSteps BGK or TRT steps of a D2Q9 list over row windows in one launch, from
+// and to post-collision populations (tile2d.hpp).
+hipError_t bgk_tile_f64(const double* fin, double* fout, const RowWin& ad, const TileBox& box, const BgkArgs& a,
+                        hipStream_t s);
+hipError_t bgk_tile_f32s(const float* gin, float* gout, const RowWin& ad, const TileBox& box, const BgkArgs& a,
+                         hipStream_t s);
 
 // Two-phase pass 1 (+ pass 2 partial sums): phi = (rho0-rho1)/(rho0+rho1)
 // and sum_q (f0+f1) c_x per block (main_TWOPHASE.cpp:238-298).  layout: row

@@ -17,6 +17,7 @@
 #include "kernels_f32.hpp"
 #include "lattice.hpp"
 #include "table.hpp"
+#include "tile2d.hpp"
 
 namespace lbamd {
 namespace {
@@ -222,18 +223,15 @@ __device__ __forceinline__ float rheology_visc_lp(const float (&g)[L::nQ], float
 // tauAnti_factor = tauA_factor; tau_inv, tau_factor are then the symmetric
 // ones.  MODE kRheology: tau_inv, tau_factor from the node's viscosity
 // (table sr/nu of n rows), stored beside rho (rho_o[NP + i]) when STORE.
-template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
-__device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __restrict__ gout, const A& ad,
-                                              int32_t i, int64_t NP, float tau_inv, float tau_factor,
-                                              const float (&F)[3], double* __restrict__ rho_o,
-                                              double* __restrict__ vel_o, float tauA_inv = 0.0f,
-                                              float tauA_factor = 0.0f, const float* __restrict__ sr = nullptr,
-                                              const float* __restrict__ nu = nullptr, int tab_n = 0,
-                                              uint32_t step = 0, const float* table = nullptr) {
+// g: the pre-collision populations; put(q, v) takes the post-collision ones.
+template <class L, typename S, bool STORE, bool REDUCE, int MODE, class Put>
+__device__ __forceinline__ double bgk_collide_lp(const float (&g)[L::nQ], int32_t i, int64_t NP, float tau_inv,
+                                                 float tau_factor, const float (&F)[3], double* __restrict__ rho_o,
+                                                 double* __restrict__ vel_o, float tauA_inv, float tauA_factor,
+                                                 const float* __restrict__ sr, const float* __restrict__ nu, int tab_n,
+                                                 uint32_t step, const float* table, Put&& put) {
   constexpr int Q = L::nQ, D = L::nD;
   const SrSeed hn = sr_node(i, step);  // unused (removed) for float storage
-  float g[Q];
-  load_g<L, S, FIRST>(gin, ad, i, NP, g);
   float drho = 0.0f;
 #pragma unroll
   for (int q = 0; q < Q; ++q) drho += g[q];
@@ -266,8 +264,6 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
     if (STORE) rho_o[NP + i] = static_cast<double>(visc);
   }
   const float omt = 1.0f - tau_inv;
-  // one 64-bit address per node; the direction offsets fold into the stores
-  S* __restrict__ out = elem_ptr<A::kOff32>(gout, pidx<Q>(0, i));
   if constexpr (MODE == kTrt) {
     // Each pair relaxes its even part (gs = (g_q + g_r)/2 = f_sym - w, towards
     // w(a0 + 4.5 rho cu^2)) with 1/tauSym and its odd part (ga = (g_q - g_r)/2,
@@ -284,14 +280,14 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
       const float ga = 0.5f * (g[q] - g[rq]);
       const float sym = omt * gs + (w * tau_inv) * (a0 + r45 * cu * cu) + (w * tau_factor) * (9.0f * cF * cu + m3uF);
       const float anti = oma * ga + (w * tauA_inv) * (r3 * cu) + (w * tauA_factor) * (3.0f * cF);
-      st_elem<NT>(Store<S>::put_sr(sym + anti, sr_bits(hn, q)), out + (q << kPLog));
-      st_elem<NT>(Store<S>::put_sr(sym - anti, sr_bits(hn, rq)), out + (rq << kPLog));
+      put(q, Store<S>::put_sr(sym + anti, sr_bits(hn, q)));
+      put(rq, Store<S>::put_sr(sym - anti, sr_bits(hn, rq)));
     }
     {
       constexpr int q = Q - 1;  // rest: even only
       const float w = float(L::w(q));
       const float gq = omt * g[q] + (w * tau_inv) * a0 + (w * tau_factor) * m3uF;
-      st_elem<NT>(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
+      put(q, Store<S>::put_sr(gq, sr_bits(hn, q)));
     }
     return REDUCE ? static_cast<double>(jd[0]) : 0.0;
   }
@@ -309,16 +305,51 @@ __device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __re
     const float fod = 3.0f * cF;
     const float gq = omt * g[q] + wt * (ev + od) + wf * (fev + fod);
     const float gr = omt * g[rq] + wt * (ev - od) + wf * (fev - fod);
-    st_elem<NT>(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
-    st_elem<NT>(Store<S>::put_sr(gr, sr_bits(hn, rq)), out + (rq << kPLog));
+    put(q, Store<S>::put_sr(gq, sr_bits(hn, q)));
+    put(rq, Store<S>::put_sr(gr, sr_bits(hn, rq)));
   }
   {
     constexpr int q = Q - 1;  // rest: c = 0
     const float w = float(L::w(q));
     const float gq = omt * g[q] + (w * tau_inv) * a0 + (w * tau_factor) * m3uF;
-    st_elem<NT>(Store<S>::put_sr(gq, sr_bits(hn, q)), out + (q << kPLog));
+    put(q, Store<S>::put_sr(gq, sr_bits(hn, q)));
   }
   return REDUCE ? static_cast<double>(jd[0]) : 0.0;
+}
+
+template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
+__device__ __forceinline__ double bgk_node_lp(const S* __restrict__ gin, S* __restrict__ gout, const A& ad,
+                                              int32_t i, int64_t NP, float tau_inv, float tau_factor,
+                                              const float (&F)[3], double* __restrict__ rho_o,
+                                              double* __restrict__ vel_o, float tauA_inv = 0.0f,
+                                              float tauA_factor = 0.0f, const float* __restrict__ sr = nullptr,
+                                              const float* __restrict__ nu = nullptr, int tab_n = 0,
+                                              uint32_t step = 0, const float* table = nullptr) {
+  float g[L::nQ];
+  load_g<L, S, FIRST>(gin, ad, i, NP, g);
+  // one 64-bit address per node; the direction offsets fold into the stores
+  S* __restrict__ out = elem_ptr<A::kOff32>(gout, pidx<L::nQ>(0, i));
+  return bgk_collide_lp<L, S, STORE, REDUCE, MODE>(g, i, NP, tau_inv, tau_factor, F, rho_o, vel_o, tauA_inv,
+                                                   tauA_factor, sr, nu, tab_n, step, table,
+                                                   [&](int q, S v) { st_elem<NT>(v, out + (q << kPLog)); });
+}
+
+// kTileSteps steps of a small D2Q9 list in float storage (tile2d.hpp).
+template <int MODE>
+__global__ __launch_bounds__(kTileEdge * kTileEdge) void k_bgk_tile_lp(const float* __restrict__ gin,
+                                                                       float* __restrict__ gout, RowWin ad,
+                                                                       TileBox box, float tau_inv, float tau_factor,
+                                                                       float F0, float F1, float tauA_inv,
+                                                                       float tauA_factor) {
+  const float F[3] = {F0, F1, 0.0f};
+  tile_steps(gin, gout, ad, box, [&](float (&g)[D2Q9::nQ], int32_t i) {
+    float v[D2Q9::nQ];
+    bgk_collide_lp<D2Q9, float, false, false, MODE>(g, i, 0, tau_inv, tau_factor, F, nullptr, nullptr, tauA_inv,
+                                                    tauA_factor, nullptr, nullptr, 0, 0u, nullptr,
+                                                    [&](int q, float x) { v[q] = x; });
+#pragma unroll
+    for (int q = 0; q < D2Q9::nQ; ++q) g[q] = v[q];
+  });
 }
 
 template <class L, typename S, class A, bool FIRST, bool STORE, bool REDUCE, int MODE, bool NT>
@@ -945,6 +976,18 @@ hipError_t bgk_lowp(int precision, int lattice, bool first, bool store, bool red
     }
     keys(std::false_type{});
   });
+}
+
+hipError_t bgk_tile_f32s(const float* gin, float* gout, const RowWin& ad, const TileBox& box, const BgkArgs& a,
+                         hipStream_t s) {
+  const dim3 g(static_cast<unsigned>(box.tiles())), b(kTileEdge * kTileEdge);
+  const float ti = static_cast<float>(a.tau_inv), tf = static_cast<float>(a.tau_factor);
+  const float F0 = static_cast<float>(a.F[0]), F1 = static_cast<float>(a.F[1]);
+  const float tai = static_cast<float>(a.tauA_inv), taf = static_cast<float>(a.tauA_factor);
+  if (a.mode == kTrt) k_bgk_tile_lp<kTrt><<<g, b, 0, s>>>(gin, gout, ad, box, ti, tf, F0, F1, tai, taf);
+  else if (a.mode == kBgk) k_bgk_tile_lp<kBgk><<<g, b, 0, s>>>(gin, gout, ad, box, ti, tf, F0, F1, tai, taf);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
 }
 
 hipError_t flux_lowp(int precision, int lattice, int nf, bool first, const void* gin,

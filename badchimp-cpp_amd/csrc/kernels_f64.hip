@@ -18,6 +18,7 @@
 #include "lattice.hpp"
 #include "layout_select.hpp"
 #include "table.hpp"
+#include "tile2d.hpp"
 
 namespace lbamd {
 namespace {
@@ -166,30 +167,28 @@ __device__ __forceinline__ double rheology_visc(const double (&f)[L::nQ], double
 // kRheology: polymer_viscosity_tabulation/main.cpp:105-155, the relaxation
 // time from the node's strain rate and the viscosity table; the viscosity
 // is stored beside rho (rho_o[NP + i]) when STORE.
-template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
-__device__ __forceinline__ double bgk_node(const double* __restrict__ fin, double* __restrict__ fout, const A& ad,
-                                           int32_t i, int64_t NP, const BgkArgs& a, double* __restrict__ rho_o,
-                                           double* __restrict__ vel_o, const double* table = nullptr) {
+// f: the pre-collision populations; put_out(q, v) takes the post-collision ones.
+template <class L, bool STORE, bool REDUCE, int MODE, class Put>
+__device__ __forceinline__ double bgk_collide(const double (&f)[L::nQ], int32_t i, int64_t NP, const BgkArgs& a,
+                                              double* __restrict__ rho_o, double* __restrict__ vel_o,
+                                              const double* table, Put&& put_out) {
   constexpr int Q = L::nQ, D = L::nD;
   double jx = 0.0;
-  double f[1][Q];
-  load_node<L, 1, FIRST>(fin, ad, i, NP, f);
   // calcRho, calcVel (LBmacroscopic.h:11-45)
-  const double rho = qsum<L>(f[0]);
+  const double rho = qsum<L>(f);
   double u[D];
 #pragma unroll
-  for (int d = 0; d < D; ++d) u[d] = (qsumc<L>(f[0], d) + 0.5 * a.F[d]) / rho;
+  for (int d = 0; d < D; ++d) u[d] = (qsumc<L>(f, d) + 0.5 * a.F[d]) / rho;
   if (STORE) {
     rho_o[i] = rho;
 #pragma unroll
     for (int d = 0; d < D; ++d) vel_o[d * NP + i] = u[d];
   }
-  if (REDUCE) jx = qsumc<L>(f[0], 0) + 0.5 * a.F[0];
+  if (REDUCE) jx = qsumc<L>(f, 0) + 0.5 * a.F[0];
   const double u2 = dot<L>(u, u);
   const double uF = dot<L>(u, a.F);
   const double c2u2 = L::c2 * u2;
   const double c2uF = L::c2 * uF;
-  double* __restrict__ out = elem_ptr<A::kOff32>(fout, pidx<Q>(0, i));
   // Directions q and rev q share every term that is even in c_q, and the odd
   // ones up to the sign: c_q . v of the reverse direction is the negative,
   // exactly (IEEE sums and products of negated operands), so each pair forms
@@ -198,7 +197,7 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
   // per wave instead of 640 (64^3 pack: 7.8 us for 8.0), the two-phase collision
   // 1237 instead of 1402 (FP64 64^3 21.2 us for 21.8, 192^3 436 for 438).
   if constexpr (MODE == kRheology) {
-    const double visc = rheology_visc<L>(f[0], rho, u, c2u2, a, table);
+    const double visc = rheology_visc<L>(f, rho, u, c2u2, a, table);
     // tau_ = visc_ * c2Inv / rho + 0.5 (LBrheology.h:463); calcDeltaOmegaF's
     // tau_factor at that tau (LBcollision.h:206)
     const double tau = (visc * L::c2Inv) / rho + 0.5;
@@ -206,8 +205,8 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
     const double tau_factor = 1 - 0.5 / tau;
     if (STORE) rho_o[NP + i] = visc;
     auto put = [&](int q, double feq, double dF) {
-      const double om = (-tau_inv) * (f[0][q] - feq);
-      st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
+      const double om = (-tau_inv) * (f[q] - feq);
+      put_out(q, (f[q] + om) + dF);
     };
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -231,21 +230,21 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
       const double cu = cdot<L>(q, u);
       const double cF = cdot<L>(q, a.F);
       // calcOmegaBGKTRT (LBcollision.h:66-70)
-      const double fqSym = 0.5 * (f[0][q] + f[0][r]);
-      const double fqAnti = 0.5 * (f[0][q] - f[0][r]);
+      const double fqSym = 0.5 * (f[q] + f[r]);
+      const double fqAnti = 0.5 * (f[q] - f[r]);
       const double rw = rho * L::w(q);
       const double sym = (-a.tau_inv) * (fqSym - rw * (1.0 + L::c4Inv0_5 * (cu * cu - c2u2)));
       const double anti = a.tauA_inv * (fqAnti - (rw * L::c2Inv) * cu);
       // calcDeltaOmegaFTRT, phi = 1 (LBcollision.h:229): w * 1.0 == w
       const double oddF = (a.tauA_factor * L::c2Inv) * cF, evenF = (a.tau_factor * L::c4Inv) * (cF * cu - c2uF);
-      st_elem<NT>((f[0][q] + (sym - anti)) + L::w(q) * (oddF + evenF), out + (q << kPLog));
-      if (r != q) st_elem<NT>((f[0][r] + (sym + anti)) + L::w(q) * (evenF - oddF), out + (r << kPLog));
+      put_out(q, (f[q] + (sym - anti)) + L::w(q) * (oddF + evenF));
+      if (r != q) put_out(r, (f[r] + (sym + anti)) + L::w(q) * (evenF - oddF));
     }
     return jx;
   }
   auto put = [&](int q, double feq, double dF) {
-    const double om = (-a.tau_inv) * (f[0][q] - feq);
-    st_elem<NT>((f[0][q] + om) + dF, out + (q << kPLog));
+    const double om = (-a.tau_inv) * (f[q] - feq);
+    put_out(q, (f[q] + om) + dF);
   };
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
@@ -261,6 +260,30 @@ __device__ __forceinline__ double bgk_node(const double* __restrict__ fin, doubl
     if (r != q) put(r, rw * ((1.0 - odd) + even), wt * (evenF - oddF));
   }
   return jx;
+}
+
+template <class L, class A, bool FIRST, bool STORE, bool REDUCE, int MODE = kBgk, bool NT = true>
+__device__ __forceinline__ double bgk_node(const double* __restrict__ fin, double* __restrict__ fout, const A& ad,
+                                           int32_t i, int64_t NP, const BgkArgs& a, double* __restrict__ rho_o,
+                                           double* __restrict__ vel_o, const double* table = nullptr) {
+  double f[1][L::nQ];
+  load_node<L, 1, FIRST>(fin, ad, i, NP, f);
+  double* __restrict__ out = elem_ptr<A::kOff32>(fout, pidx<L::nQ>(0, i));
+  return bgk_collide<L, STORE, REDUCE, MODE>(f[0], i, NP, a, rho_o, vel_o, table,
+                                             [&](int q, double v) { st_elem<NT>(v, out + (q << kPLog)); });
+}
+
+// kTileSteps steps of a small D2Q9 list (tile2d.hpp).
+template <int MODE>
+__global__ __launch_bounds__(kTileEdge * kTileEdge) void k_bgk_tile(const double* __restrict__ fin,
+                                                                    double* __restrict__ fout, RowWin ad, TileBox box,
+                                                                    BgkArgs a) {
+  tile_steps(fin, fout, ad, box, [&](double (&f)[D2Q9::nQ], int32_t i) {
+    double v[D2Q9::nQ];
+    bgk_collide<D2Q9, false, false, MODE>(f, i, 0, a, nullptr, nullptr, nullptr, [&](int q, double x) { v[q] = x; });
+#pragma unroll
+    for (int q = 0; q < D2Q9::nQ; ++q) f[q] = v[q];
+  });
 }
 
 // REDUCE: the block's sum of j_x goes to partial[b], or is added to it
@@ -910,6 +933,15 @@ hipError_t bgk_f64(int lattice, bool first, bool store, bool reduce, const doubl
       keys(std::false_type{});
     });
   });
+  return hipGetLastError();
+}
+
+hipError_t bgk_tile_f64(const double* fin, double* fout, const RowWin& ad, const TileBox& box, const BgkArgs& a,
+                        hipStream_t s) {
+  const dim3 g(static_cast<unsigned>(box.tiles())), b(kTileEdge * kTileEdge);
+  if (a.mode == kTrt) k_bgk_tile<kTrt><<<g, b, 0, s>>>(fin, fout, ad, box, a);
+  else if (a.mode == kBgk) k_bgk_tile<kBgk><<<g, b, 0, s>>>(fin, fout, ad, box, a);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
