@@ -206,7 +206,7 @@ int pre_state(lb_ctx* c, const void** out) {
 }
 
 // nodes per host thread of the set-up passes that look at every link of a node
-constexpr int64_t kMinNodes = 8192;
+constexpr int64_t kMinNodes = 16384;
 
 // Row layout of a node list (positions and neighbour index).  Returns false
 // with a reason when the node list is not a set of cells of one box that the
