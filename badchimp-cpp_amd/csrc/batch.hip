@@ -42,6 +42,7 @@
 #include "kernels.hpp"
 #include "kernels_f32.hpp"
 #include "lattice.hpp"
+#include "layout_select.hpp"
 #include "rowbuild.hpp"
 
 using namespace lbamd;
@@ -198,6 +199,7 @@ struct lb_batch {
   int32_t shape = 4;
   int32_t ns = 1;           // 256-thread slices per workgroup (workgroups of 256 ns threads)
   int64_t tuned_nodes = -1;
+  bool nt = true;           // streaming stores (all active solves' populations; stream_stores)
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   // results and counters
   std::vector<Result> done;
@@ -245,20 +247,21 @@ hipError_t launch_step(lb_batch* b, bool reduce, int32_t shape, int32_t ns, int3
     const int32_t n = b->n_items_bgk;
     const int32_t grid = shape_grid(b, shape, ns, n);
     if (b->prec[0] == LB_FP64)
-      e = batch_bgk_f64(b->lattice, true, b->d_solves, b->d_items, n, grid, parity, ns, koff > 0, b->stream);
+      e = batch_bgk_f64(b->lattice, true, b->d_solves, b->d_items, n, grid, parity, ns, b->nt, koff > 0,
+                        b->stream);
     else
       e = batch_bgk_lowp(b->prec[0], b->lattice, true, b->d_solves, b->d_items, n, grid, parity,
-                         b->d_step, koff, ns, koff > 0, b->stream);
+                         b->d_step, koff, ns, b->nt, koff > 0, b->stream);
   }
   if (e == hipSuccess && b->n_items_cg > 0) {
     const int32_t n = b->n_items_cg;
     const uint32_t* it = b->d_items + b->n_items_bgk;
     const int32_t grid = shape_grid(b, shape, ns, n);
     if (b->prec[1] == LB_FP64)
-      e = batch_cg_f64(b->lattice, reduce, b->d_solves, it, n, grid, parity, ns, b->stream);
+      e = batch_cg_f64(b->lattice, reduce, b->d_solves, it, n, grid, parity, ns, b->nt, b->stream);
     else
       e = batch_cg_lowp(b->prec[1], b->lattice, reduce, b->d_solves, it, n, grid, parity, b->d_step, koff,
-                        ns, b->stream);
+                        ns, b->nt, b->stream);
   }
   return e;
 }
@@ -269,6 +272,7 @@ int refresh(lb_batch* b) {
   b->items.clear();
   b->active.clear();
   b->resident_nodes = 0;
+  int64_t bytes = 0;
   for (int kind = 0; kind < 2; ++kind) {
     std::vector<uint32_t> items;
     std::vector<uint8_t> xcd;
@@ -277,6 +281,7 @@ int refresh(lb_batch* b) {
       if (!sl.used || sl.kind != kind) continue;
       b->active.push_back(s);
       b->resident_nodes += sl.fp.n;
+      bytes += 2 * (kind + 1) * b->Q * sl.fp.NP * static_cast<int64_t>(elem_bytes(b->prec[kind]));
       for (int64_t k = 0; k < sl.fp.nblk; ++k)
         items.push_back((static_cast<uint32_t>(s) << kItemShift) | static_cast<uint32_t>(k));
       xcd.insert(xcd.end(), sl.xcd.begin(), sl.xcd.end());
@@ -286,6 +291,7 @@ int refresh(lb_batch* b) {
     if (kind == 0) b->n_items_bgk = static_cast<int32_t>(b->items.size());
   }
   b->n_items_cg = static_cast<int32_t>(b->items.size()) - b->n_items_bgk;
+  b->nt = stream_stores(bytes);
   if (static_cast<int64_t>(b->items.size()) > b->items_cap) {
     if (b->d_items) hipFree(b->d_items);
     b->d_items = nullptr;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "addressing.hpp"
 #include "context.hpp"
@@ -82,10 +83,11 @@ hipError_t tag_mass_f64(int lattice, bool first, const double* fin, const TableA
 
 // ---- batched form -----------------------------------------------------------
 // One FP64 step of every solve listed in items (see k_batch_bgk): grid
-// workgroups of 256 ns threads (ns = 1 or 2 items at a time); reduce writes each solve's block partials of j_x (accum:
-// adds to them).
+// workgroups of 256 ns threads (ns = 1 or 2 items at a time), nt: streaming
+// stores (stream_stores); reduce writes each solve's block partials of j_x
+// (accum: adds to them).
 hipError_t batch_bgk_f64(int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                         int32_t n_items, int32_t grid, int32_t parity, int ns, bool accum,
+                         int32_t n_items, int32_t grid, int32_t parity, int ns, bool nt, bool accum,
                          hipStream_t s);
 // Two-phase rest state (phase-0 density r0 per compact node) placed where the
 // first pull through ad reads it (FP64 form).
@@ -94,7 +96,7 @@ hipError_t prestream_f64(int lattice, const RowWin& ad, const double* r0, int32_
 // Both passes of one FP64 colour-gradient step of every two-phase solve listed
 // in items (as batch_bgk_f64); reduce writes each solve's three flux partials.
 hipError_t batch_cg_f64(int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                        int32_t n_items, int32_t grid, int32_t parity, int ns, hipStream_t s);
+                        int32_t n_items, int32_t grid, int32_t parity, int ns, bool nt, hipStream_t s);
 // out[slot] = sum of the solve's block partials, for each slot listed.
 hipError_t batch_sum(const BatchSolve* solves, const int32_t* slots, int32_t n_slots, double* out,
                      hipStream_t s);
@@ -105,6 +107,16 @@ hipError_t batch_check(BatchSolve* solves, SolveCheck* chk, const int32_t* slots
                        int32_t M, uint32_t* step, hipStream_t s);
 // Rest state (f = w) of one FP64 buffer of Q * NP elements.
 hipError_t batch_rest_f64(int lattice, double* f, int64_t NP, hipStream_t s);
+
+// f(256-thread slices per workgroup, streaming stores) as constants.
+template <class F>
+void batch_dispatch(int ns, bool nt, F&& f) {
+  using std::integral_constant;
+  if (ns == 2 && nt) f(integral_constant<int, 2>{}, std::true_type{});
+  else if (ns == 2) f(integral_constant<int, 2>{}, std::false_type{});
+  else if (nt) f(integral_constant<int, 1>{}, std::true_type{});
+  else f(integral_constant<int, 1>{}, std::false_type{});
+}
 
 // ---- shared ---------------------------------------------------------------
 // out[c] = sum over blocks of partial[c*nblocks + b], c < ncomp (fixed order).

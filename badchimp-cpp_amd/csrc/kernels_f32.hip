@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void k_bgk_lp(const S* __restrict__ gin, S*
 
 // Batched form (see k_batch_bgk in the FP64 kernels): the parameters are
 // rounded to float exactly as the single-solve launcher rounds them.
-template <class L, typename S, bool REDUCE, int NS>
+template <class L, typename S, bool REDUCE, int NS, bool NT>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk_lp(const BatchSolve* __restrict__ solves,
                                                               const uint32_t* __restrict__ items, int32_t n_items,
                                                               int32_t parity,
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk_lp(const BatchSolve* 
     double jx = 0.0;
     if (act && i < s.n) {
       const float F[3] = {static_cast<float>(s.a.F[0]), static_cast<float>(s.a.F[1]), static_cast<float>(s.a.F[2])};
-      jx = bgk_node_lp<L, S, RowWin, false, false, REDUCE>(
+      jx = bgk_node_lp<L, S, RowWin, false, false, REDUCE, kBgk, NT>(
           static_cast<const S*>(device_ptr(s.f[p])), static_cast<S*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, static_cast<float>(s.a.tau_inv),
           static_cast<float>(s.a.tau_factor), F, nullptr, nullptr, 0.0f, 0.0f, nullptr, nullptr, 0,
           gstep - s.step_base);
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi_lp(const BatchSolv
 // At least 4 waves per SIMD (at most 128 VGPRs, no spills): left to
 // itself the compiler takes 132 VGPRs (3 waves) for the FP64 two-phase
 // arithmetic, and the pass ran 6 % slower (192^3 pack, FP32S).
-template <class L, typename S, int NS>
+template <class L, typename S, int NS, bool NT>
 __global__ __launch_bounds__(kBlock * NS, 4) void k_batch_cg_lp(const BatchSolve* __restrict__ solves,
                                                              const uint32_t* __restrict__ items, int32_t n_items,
                                                              int32_t parity,
@@ -784,7 +784,7 @@ __global__ __launch_bounds__(kBlock * NS, 4) void k_batch_cg_lp(const BatchSolve
       pn[qq] = f ? v : pw;
     }
     const double F[3] = {s.a.F[0], s.a.F[1], s.a.F[2]};
-    cg_collide<L, S, true, false, true>(t, dd, pn, F, s.nu0Inv, s.nu1Inv, s.sigma, s.beta, static_cast<S*>(device_ptr(s.f[p ^ 1])),
+    cg_collide<L, S, true, false, NT>(t, dd, pn, F, s.nu0Inv, s.nu1Inv, s.sigma, s.beta, static_cast<S*>(device_ptr(s.f[p ^ 1])),
                                   i, s.NP, nullptr, nullptr, gstep - s.step_base);
   }
 }
@@ -1015,40 +1015,37 @@ hipError_t flux_lowp(int precision, int lattice, int nf, bool first, const void*
 }
 
 hipError_t batch_bgk_lowp(int precision, int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                          int32_t n_items, int32_t grid, int32_t parity, const uint32_t* step0,
-                          int32_t koff, int ns, bool accum, hipStream_t s) {
+                          int32_t n_items, int32_t grid, int32_t parity, const uint32_t* step0, int32_t koff, int ns,
+                          bool nt, bool accum, hipStream_t s) {
   return dispatch(precision, lattice, Addr{}, [&](auto l, auto st, auto) {
     using L = decltype(l);
     using S = decltype(st);
-    const dim3 g(grid), b(kBlock);
-    if (ns == 2) {
-      const dim3 b2(2 * kBlock);
-      if (reduce) k_batch_bgk_lp<L, S, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
-      else k_batch_bgk_lp<L, S, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
-    } else {
-      if (reduce) k_batch_bgk_lp<L, S, true, 1><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
-      else k_batch_bgk_lp<L, S, false, 1><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
-    }
+    auto go = [&](auto slices, auto str) {
+      constexpr int NS = decltype(slices)::value;
+      constexpr bool NT = decltype(str)::value;
+      const dim3 g(grid), b(NS * kBlock);
+      if (reduce) k_batch_bgk_lp<L, S, true, NS, NT><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
+      else k_batch_bgk_lp<L, S, false, NS, NT><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff, accum ? 1 : 0);
+    };
+    batch_dispatch(ns, nt, go);
   });
 }
 
 hipError_t batch_cg_lowp(int precision, int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                         int32_t n_items, int32_t grid, int32_t parity, const uint32_t* step0,
-                         int32_t koff, int ns, hipStream_t s) {
+                         int32_t n_items, int32_t grid, int32_t parity, const uint32_t* step0, int32_t koff, int ns,
+                         bool nt, hipStream_t s) {
   return dispatch(precision, lattice, Addr{}, [&](auto l, auto st, auto) {
     using L = decltype(l);
     using S = decltype(st);
-    const dim3 g(grid), b(kBlock);
-    if (ns == 2) {
-      const dim3 b2(2 * kBlock);
-      if (reduce) k_batch_cg_phi_lp<L, S, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
-      else k_batch_cg_phi_lp<L, S, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
-      k_batch_cg_lp<L, S, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity, step0, koff);
-    } else {
-      if (reduce) k_batch_cg_phi_lp<L, S, true, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
-      else k_batch_cg_phi_lp<L, S, false, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
-      k_batch_cg_lp<L, S, 1><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff);
-    }
+    auto go = [&](auto slices, auto str) {
+      constexpr int NS = decltype(slices)::value;
+      constexpr bool NT = decltype(str)::value;
+      const dim3 g(grid), b(NS * kBlock);
+      if (reduce) k_batch_cg_phi_lp<L, S, true, NS><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      else k_batch_cg_phi_lp<L, S, false, NS><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      k_batch_cg_lp<L, S, NS, NT><<<g, b, 0, s>>>(solves, items, n_items, parity, step0, koff);
+    };
+    batch_dispatch(ns, nt, go);
   });
 }
 

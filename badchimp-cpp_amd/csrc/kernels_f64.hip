@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kBlock) void k_bgk(const double* __restrict__ fin,
 // solve's (bgk_node), so a solve gets the same bits alone or in any mix.
 // NS: items a workgroup works on at a time, one per 256-thread slice; every
 // slice reduces its item exactly as a 256-thread workgroup would.
-template <class L, bool REDUCE, int NS>
+template <class L, bool REDUCE, int NS, bool NT>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk(const BatchSolve* __restrict__ solves,
                                                            const uint32_t* __restrict__ items, int32_t n_items,
                                                            int32_t parity, int32_t accum) {
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_bgk(const BatchSolve* __r
     const double prev = REDUCE && accum && tid == 0 && act ? device_ptr(s.partial)[lb] : 0.0;
     double jx = 0.0;
     if (act && i < s.n)
-      jx = bgk_node<L, RowWin, false, false, REDUCE>(static_cast<const double*>(device_ptr(s.f[p])),
+      jx = bgk_node<L, RowWin, false, false, REDUCE, kBgk, NT>(static_cast<const double*>(device_ptr(s.f[p])),
                                                      static_cast<double*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, s.a,
                                                      nullptr, nullptr);
     if (REDUCE) {
@@ -716,7 +716,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg_phi(const BatchSolve* 
   }
 }
 
-template <class L, int NS>
+template <class L, int NS, bool NT>
 __global__ __launch_bounds__(kBlock * NS) void k_batch_cg(const BatchSolve* __restrict__ solves,
                                                           const uint32_t* __restrict__ items, int32_t n_items,
                                                           int32_t parity) {
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(kBlock * NS) void k_batch_cg(const BatchSolve* __re
 #pragma unroll
     for (int d = 0; d < D; ++d) F[d] = s.a.F[d];
     const WallPhi wp{nullptr, s.phi_w};
-    cg_node<L, false, false, true>(static_cast<const double*>(device_ptr(s.f[p])), static_cast<double*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, a,
+    cg_node<L, false, false, NT>(static_cast<const double*>(device_ptr(s.f[p])), static_cast<double*>(device_ptr(s.f[p ^ 1])), ad, i, s.NP, a,
                              static_cast<const double*>(device_ptr(s.phi)), wp, F, nullptr, nullptr);
   }
 }
@@ -1063,33 +1063,32 @@ hipError_t prestream_f64(int lattice, const RowWin& ad, const double* r0, int32_
 }
 
 hipError_t batch_cg_f64(int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                        int32_t n_items, int32_t grid, int32_t parity, int ns, hipStream_t s) {
+                        int32_t n_items, int32_t grid, int32_t parity, int ns, bool nt, hipStream_t s) {
   LB_DISPATCH_LATTICE(lattice, L, {
-    const dim3 g(grid), b(kBlock), b2(2 * kBlock);
-    if (ns == 2) {
-      if (reduce) k_batch_cg_phi<L, true, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
-      else k_batch_cg_phi<L, false, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
-      k_batch_cg<L, 2><<<g, b2, 0, s>>>(solves, items, n_items, parity);
-    } else {
-      if (reduce) k_batch_cg_phi<L, true, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
-      else k_batch_cg_phi<L, false, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
-      k_batch_cg<L, 1><<<g, b, 0, s>>>(solves, items, n_items, parity);
-    }
+    auto go = [&](auto slices, auto str) {
+      constexpr int NS = decltype(slices)::value;
+      constexpr bool NT = decltype(str)::value;
+      const dim3 g(grid), b(NS * kBlock);
+      if (reduce) k_batch_cg_phi<L, true, NS><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      else k_batch_cg_phi<L, false, NS><<<g, b, 0, s>>>(solves, items, n_items, parity);
+      k_batch_cg<L, NS, NT><<<g, b, 0, s>>>(solves, items, n_items, parity);
+    };
+    batch_dispatch(ns, nt, go);
   });
   return hipGetLastError();
 }
 
 hipError_t batch_bgk_f64(int lattice, bool reduce, const BatchSolve* solves, const uint32_t* items,
-                         int32_t n_items, int32_t grid, int32_t parity, int ns, bool accum, hipStream_t s) {
+                         int32_t n_items, int32_t grid, int32_t parity, int ns, bool nt, bool accum, hipStream_t s) {
   LB_DISPATCH_LATTICE(lattice, L, {
-    const dim3 b(kBlock * (ns == 2 ? 2 : 1));
-    if (ns == 2) {
-      if (reduce) k_batch_bgk<L, true, 2><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
-      else k_batch_bgk<L, false, 2><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
-    } else {
-      if (reduce) k_batch_bgk<L, true, 1><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
-      else k_batch_bgk<L, false, 1><<<dim3(grid), b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
-    }
+    auto go = [&](auto slices, auto str) {
+      constexpr int NS = decltype(slices)::value;
+      constexpr bool NT = decltype(str)::value;
+      const dim3 g(grid), b(NS * kBlock);
+      if (reduce) k_batch_bgk<L, true, NS, NT><<<g, b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
+      else k_batch_bgk<L, false, NS, NT><<<g, b, 0, s>>>(solves, items, n_items, parity, accum ? 1 : 0);
+    };
+    batch_dispatch(ns, nt, go);
   });
   return hipGetLastError();
 }
