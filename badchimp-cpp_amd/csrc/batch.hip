@@ -7,9 +7,9 @@
 // table and the block partials, carved from one pre-allocated device region by
 // a first-fit allocator.  Every step is one launch over all resident solves
 // (k_batch_bgk / k_batch_bgk_lp); every check_every steps the last launch also
-// writes block partials of j_x, one small launch sums them per solve, the host
-// reads one double per solve, evaluates k = nu <j_x> / F_x and retires the
-// solves whose |dk| <= tol |k| (the stop of lb_solve_permeability).  Retired
+// writes block partials of j_x, one small launch sums them per solve, another
+// evaluates k = nu <j_x> / F_x and decides the solves whose |dk| <= tol |k| (the
+// stop of lb_solve_permeability); the host reads the stop states.  Retired
 // solves free their memory; waiting requests can then be admitted, at a check
 // boundary, so every solve sees whole check intervals.
 //
@@ -106,34 +106,36 @@ struct RangeAlloc {
 
 // Sizes of one solve's device region (nf = 1 single-phase, 2 two-phase).
 struct Footprint {
-  int64_t n = 0, NP = 0, nblk = 0, nwin = 0;
+  int64_t n = 0, NP = 0, nblk = 0;
   int nf = 1;
   int64_t off_f0 = 0, off_f1 = 0, off_coord = 0, off_win = 0, off_part = 0, off_phi = 0, bytes = 0;
 };
 
-Footprint footprint_of(int Q, size_t esz, int64_t n, int64_t nwin, int nf) {
+Footprint footprint_of(int Q, size_t esz, int64_t n, int64_t window_bytes, int nf) {
   Footprint fp;
   fp.n = n;
   fp.nf = nf;
   fp.NP = std::max<int64_t>((n + kBlock - 1) / kBlock, 1) * kBlock;
   fp.nblk = std::max<int64_t>((n + kBlock - 1) / kBlock, 1);
-  fp.nwin = nwin;
   const int64_t fb = align_up(static_cast<int64_t>(nf) * Q * fp.NP * static_cast<int64_t>(esz));
   fp.off_f0 = 0;
   fp.off_f1 = fb;
   fp.off_coord = 2 * fb;
   fp.off_win = fp.off_coord + align_up(fp.NP * 4);
-  fp.off_part = fp.off_win + align_up(nwin * static_cast<int64_t>(sizeof(uint32_t)));
+  fp.off_part = fp.off_win + align_up(window_bytes);
   fp.off_phi = fp.off_part + align_up((nf == 2 ? 3 : 1) * fp.nblk * 8);
   // colour field: double in FP64, float otherwise
   fp.bytes = fp.off_phi + (nf == 2 ? align_up(fp.NP * (esz == 8 ? 8 : 4)) : 0);
   return fp;
 }
 
-// 32-bit words of a solve's window table and its first nodes of the x planes
-int64_t window_words(const RowBuild& rb) {
-  const int64_t px = rb.g.E[0] + 2;
-  return px * (rb.g.E[1] + 2) * win_words(rb.g.E[2]) + (rb.coord.size() >> kWinBase ? px : 0);
+// Bytes reserved for a solve's window table and its first nodes of the x planes:
+// 16 per row and 32 cells, what pools are sized by, or what the table takes where
+// that is more (the x planes of lists beyond 2^kWinBase nodes).
+int64_t window_bytes(const RowBuild& rb) {
+  const int64_t px = rb.g.E[0] + 2, rows = px * (rb.g.E[1] + 2);
+  const int64_t words = rows * win_words(rb.g.E[2]) + (rb.coord.size() >> kWinBase ? px : 0);
+  return std::max(rows * ((rb.g.E[2] + 31) / 32) * 16, words * 4);
 }
 
 struct Slot {
@@ -583,9 +585,8 @@ int lb_batch_footprint(int lattice, int precision, int32_t n_fields, int32_t nd,
   std::string why;
   if (!rows_from_geometry(lattice, dims, geo, periodic_mask, rb, why))
     return fail_global(LB_ERR_UNSUPPORTED, "lb_batch_footprint: %s", why.c_str());
-  const int64_t nwin = window_words(rb);
   const Footprint fp = footprint_of(lattice == LB_D2Q9 ? 9 : 19, elem_bytes(precision),
-                                    static_cast<int64_t>(rb.coord.size()), nwin, n_fields);
+                                    static_cast<int64_t>(rb.coord.size()), window_bytes(rb), n_fields);
   if (bytes) *bytes = fp.bytes;
   if (n_fluid) *n_fluid = fp.n;
   return LB_OK;
@@ -662,7 +663,7 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
   const int nf = p.kind == 1 ? 2 : 1;
   const int prec = b->prec[p.kind];
   const size_t esz = elem_bytes(prec);
-  const Footprint fp = footprint_of(b->Q, esz, n, window_words(rb), nf);
+  const Footprint fp = footprint_of(b->Q, esz, n, window_bytes(rb), nf);
   if (static_cast<uint64_t>(nf) * b->Q * static_cast<uint64_t>(fp.NP) * esz >= (1ull << 32) ||
       fp.nblk > static_cast<int64_t>(kItemMask) + 1)
     return bfail(b, LB_ERR_UNSUPPORTED, "lb_batch_add: %lld fluid nodes exceed one solve", (long long)n);
