@@ -1075,10 +1075,11 @@ hipError_t launch_single(lb_ctx* c, const BgkArgs& a, int from, bool first, bool
 
 // Long runs replay a captured graph of kGraphSteps steps (an even count, so
 // a replay returns to the buffer it started from): on small node lists the
-// launches, not the kernels, set the step time.  On the 256 x 128 D2Q9
-// channel (32 k nodes) a plain launch costs 3.8 us per step, a step inside a
-// graph 3.1 us, and each graph launch about 12 us more: graphs of 2 steps
-// ran at 8.1 us per step, of 8 at 3.9, of 32 at 3.4, of 128 at 3.2.  The
+// launches, not the kernels, set the step time.  With one step per launch the
+// 256 x 128 D2Q9 channel (32 k nodes) takes 3.8 us per step by plain launches,
+// 3.1 us inside a graph, and each graph launch costs about 12 us more: graphs of
+// 2 steps ran at 8.1 us per step, of 8 at 3.9, of 32 at 3.4, of 128 at 3.2 (2.1
+// with the tiles of tile2d.hpp, which that list takes now).  The
 // first step after an upload and the last one (it stores rho and u) are
 // launched on their own, and so are the steps left over.  FP16S steps pass
 // the step count as their rounding seed and are always launched one by one.
@@ -1659,9 +1660,16 @@ int lb_reduce_flux(lb_ctx* c, int32_t dir, double* sum_fc, double* sum_phi0_fc, 
 
 namespace {
 // Steps per graph of a permeability solve: with a check every 100 steps, two
-// replays and four launches (48^3 pack, FP32S: 5.0 us per step for 5.5 with a
-// launch per step; FP64 48^3 5.95 for 6.4).
+// replays and four launches.  Capturing costs 0.11-0.15 ms per solve, so only
+// solves whose steps are bound by their launches and that may run long enough to
+// gain it back take graphs.  1000 steps, checked every 100, graph / launches, ms:
+// FP32S 32^3 4.59 / 5.15, 48^3 5.06 / 5.44, 56^3 5.2 / 5.6, 64^3 (16 MB of
+// populations) 5.98 / 6.17, FP64 48^3 5.87 / 6.09; beyond: FP32S 72^3 (23 MB)
+// 8.04 / 8.08, 96^3 12.30 / 12.17, FP64 64^3 8.58 / 8.55.  48^3 FP32S by the
+// number of steps: 200 1.16 / 1.11, 300 1.65 / 1.62, 500 2.64 / 2.74.
 constexpr int32_t kSolveGraphSteps = 48;
+constexpr int64_t kSolveGraphBytes = 20000000;  // both population buffers
+constexpr int64_t kSolveGraphMinSteps = 500;
 
 int solve_permeability(lb_ctx* c, const char* name, double tau, double tau_anti, const double* force,
                        int32_t check_every, double tol, int64_t max_steps, double n_box, double* k_out,
@@ -1705,7 +1713,8 @@ int solve_permeability(lb_ctx* c, const char* name, double tau, double tau_anti,
         if (x) hipGraphExecDestroy(x);
     }
   } graphs{c};
-  const bool graphed = c->precision != LB_FP16S && c->n_bulk > 0;
+  const bool graphed = c->precision != LB_FP16S && c->n_bulk > 0 && max_steps >= kSolveGraphMinSteps &&
+                       2 * c->Q * c->NP * static_cast<int64_t>(elem_size(c->precision)) < kSolveGraphBytes;
   Timer t(c);
   int64_t launches = 0;
   while (steps < max_steps) {

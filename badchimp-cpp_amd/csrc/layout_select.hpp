@@ -21,17 +21,18 @@ inline bool rowwin_fits(int Q, int64_t NP, int n_fields, int64_t elem_bytes) {
 }
 
 // Whether the step kernels write populations with streaming stores, for both
-// buffers of a context, or of all active solves of a batch, together.  Up to the MALL's 256 MiB a plain store leaves
-// the values where the next step reads them; above it a plain store only
-// displaces lines that are still to be read.  Below 20 MB, where the buffers fit
-// the L2s, a plain store is written back when the kernel ends, after its last
-// node.  Plain / streaming, us per step: FP32S 64^3 pack (16 MB) 5.55 / 5.23,
-// D2Q9 1021x509 (22 MB) 5.6 / 6.0, FP32S 80^3 (30 MB) 7.4 / 8.9, FP64 96^3
-// (107 MB) 19.3 / 23.7, FP16S 161x143x150 (100 MB) 22.2 / 26.8, FP64 128^3
-// (255 MB) 40.4 / 47.6; two-phase FP64 64^3 (62 MB) 22.0 / 22.0, 100^3 (245 MB)
-// 59.1 / 62.4; beyond: FP32S 165^3 (273 MB) 52.9 / 50.9, FP64 256^3 366 / 351.  A batch of 4
-// packs of 64^3, FP32S (64 MB) 13.5 / 15.6, FP64 (128 MB) 22.6 / 26.8; 3 of 96^3,
-// FP16S 20.6 / 24.7; 4 of 128^3, FP16S 56.1 / 67.4.
+// buffers of a context, or of all active solves of a batch, together.  Up to the
+// MALL's 256 MiB a plain store leaves the values where the next step reads them;
+// above it a plain store only displaces lines that are still to be read.  Below
+// 20 MB, where the buffers fit the L2s, a plain store is written back when the
+// kernel ends, after its last node.  Plain / streaming, us per step:
+// FP32S 64^3 pack (16 MB) 5.55 / 5.23, D2Q9 1021x509 (22 MB) 5.6 / 6.0, FP32S
+// 80^3 (30 MB) 7.4 / 8.9, FP64 96^3 (107 MB) 19.3 / 23.7, FP16S 161x143x150
+// (100 MB) 22.2 / 26.8, FP64 128^3 (255 MB) 40.4 / 47.6; two-phase FP64 64^3
+// (62 MB) 22.0 / 22.0, 100^3 (245 MB) 59.1 / 62.4; beyond: FP32S 165^3 (273 MB)
+// 52.9 / 50.9, FP64 256^3 366 / 351.  A batch of 4 packs of 64^3, FP32S (64 MB)
+// 13.5 / 15.6, FP64 (128 MB) 22.6 / 26.8; 3 of 96^3, FP16S 20.6 / 24.7; 4 of
+// 128^3, FP16S 56.1 / 67.4.
 inline bool stream_stores(int64_t both_buffers) {
   return both_buffers < 20000000 || both_buffers > (int64_t{256} << 20);
 }
