@@ -536,16 +536,18 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
     }, kMinNodes);
     return std::none_of(bad, bad + kMaxHostThreads, [](bool x) { return x; });
   };
-  if (rows_ok && !agrees([&](int q, int32_t i) { return row_source(c->lattice, rb, q, i); })) {
-    rows_ok = false;
-    why = "row layout disagrees with the neighbour index";
-  }
-  // row windows, checked link by link
+  // row windows; the rows are looked at where they may be used, that is without
+  // windows or for two fields that the windows cannot address (launch_layout)
   WinBuild wb;
   bool win_ok = rows_ok && win_allowed && build_windows(rb, true, wb, why);
   if (win_ok && !agrees([&](int q, int32_t i) { return win_source(c->lattice, rb, wb, q, i); })) {
     win_ok = false;
     why = "row windows disagree with the neighbour index";
+  }
+  if (rows_ok && !(win_ok && rowwin_fits(Q, NP, 2, static_cast<int64_t>(elem_size(c->precision)))) &&
+      !agrees([&](int q, int32_t i) { return row_source(c->lattice, rb, q, i); })) {
+    rows_ok = win_ok = false;
+    why = "row layout disagrees with the neighbour index";
   }
   // device allocation: the context holds no topology until every buffer
   // below is in place, so a failure leaves no pointer to freed memory
