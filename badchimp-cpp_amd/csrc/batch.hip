@@ -848,7 +848,9 @@ int lb_batch_add_many(lb_batch* b, int32_t count, int32_t nd, const int32_t* dim
       prepare(b->lattice, dims + static_cast<size_t>(k) * nd, geos[k], periodic_mask, *pre[k]);
   };
   std::vector<std::thread> pool;
-  for (int t = 1; t < nthr; ++t) pool.emplace_back(work);
+  pool.reserve(nthr);
+  for (int t = 1; t < nthr && start_thread(pool, work); ++t) {
+  }
   work();
   for (auto& t : pool) t.join();
   AddArgs p;

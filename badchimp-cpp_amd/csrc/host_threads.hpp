@@ -3,7 +3,9 @@
 #pragma once
 #include <algorithm>
 #include <cstdint>
+#include <exception>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace lbamd {
@@ -17,10 +19,23 @@ inline int host_threads() {
   return std::max(1, std::min(kMaxHostThreads, static_cast<int>(hw ? hw : 1)));
 }
 
+// Starts f on a thread of its own in the pool; false where the system has none
+// to give (a process or container limit), which the callers, C entry points
+// among them, take as having fewer threads.
+template <class F>
+bool start_thread(std::vector<std::thread>& pool, F&& f) {
+  try {
+    pool.emplace_back(std::forward<F>(f));
+  } catch (const std::exception&) {
+    return false;
+  }
+  return true;
+}
+
 // f(begin, end, t) over contiguous chunks of [0, n), chunk t on thread t
-// (t < host_threads()), at least min_items each: a thread costs about 25 us, an
-// item of a light pass (some loads and stores) a nanosecond or less.  f must not
-// throw.
+// (t < host_threads()) or on the caller's, at least min_items each: a thread
+// costs about 25 us, an item of a light pass (some loads and stores) a
+// nanosecond or less.  f must not throw.
 template <class F>
 void parallel_ranges(int64_t n, F&& f, int64_t min_items = int64_t{1} << 16) {
   const int T = static_cast<int>(std::min<int64_t>(host_threads(), std::max<int64_t>(1, n / min_items)));
@@ -29,13 +44,16 @@ void parallel_ranges(int64_t n, F&& f, int64_t min_items = int64_t{1} << 16) {
     return;
   }
   const int64_t chunk = (n + T - 1) / T;
+  auto run = [&f, n, chunk](int t) {
+    const int64_t b = std::min(n, t * chunk);
+    f(b, std::min(n, b + chunk), t);
+  };
   std::vector<std::thread> pool;
   pool.reserve(T - 1);
-  for (int t = 1; t < T; ++t) {
-    const int64_t b = std::min(n, t * chunk), e = std::min(n, b + chunk);
-    pool.emplace_back([&f, b, e, t] { f(b, e, t); });
-  }
-  f(int64_t{0}, std::min(n, chunk), 0);
+  int next = 1;
+  while (next < T && start_thread(pool, [&run, next] { run(next); })) ++next;
+  run(0);
+  for (; next < T; ++next) run(next);
   for (auto& th : pool) th.join();
 }
 
