@@ -618,9 +618,10 @@ struct Prepared {
   std::string why;
 };
 
-void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t periodic_mask, Prepared& pr) {
+// (threads: the row windows on threads of their own, build_windows)
+void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t periodic_mask, bool threads, Prepared& pr) {
   if (!rows_from_geometry(lattice, dims, geo, periodic_mask, pr.rb, pr.why) ||
-      !build_windows(pr.rb, false, pr.wb, pr.why)) {
+      !build_windows(pr.rb, false, pr.wb, pr.why, false, threads)) {
     pr.code = LB_ERR_UNSUPPORTED;
     return;
   }
@@ -654,7 +655,7 @@ int add_solve(lb_batch* b, int32_t nd, const int32_t* dims, const int32_t* geo, 
   hipSetDevice(b->device);
   if (!pre) {
     pre = std::make_shared<Prepared>();
-    prepare(b->lattice, dims, geo, periodic_mask, *pre);
+    prepare(b->lattice, dims, geo, periodic_mask, true, *pre);
   }
   if (pre->code != LB_OK) return bfail(b, pre->code, "lb_batch_add: %s", pre->why.c_str());
   const RowBuild& rb = pre->rb;
@@ -845,7 +846,7 @@ int lb_batch_add_many(lb_batch* b, int32_t count, int32_t nd, const int32_t* dim
   const int nthr = std::max(1, std::min<int>(16, std::min<int>(count, static_cast<int>(std::thread::hardware_concurrency()))));
   auto work = [&]() {
     for (int32_t k; (k = next.fetch_add(1)) < count;)
-      prepare(b->lattice, dims + static_cast<size_t>(k) * nd, geos[k], periodic_mask, *pre[k]);
+      prepare(b->lattice, dims + static_cast<size_t>(k) * nd, geos[k], periodic_mask, nthr == 1, *pre[k]);
   };
   std::vector<std::thread> pool;
   pool.reserve(nthr);

@@ -129,9 +129,10 @@ struct WinBuild {
 };
 
 // planes: bases from the first node of the x plane also where the node list
-// fits without (for tests).
+// fits without (for tests).  threads: large tables are filled on host threads;
+// false for a caller that is one of several threads with a geometry each.
 inline bool build_windows(const RowBuild& rb, bool allow_periodic, WinBuild& wb, std::string& why,
-                          bool planes = false) {
+                          bool planes = false, bool threads = true) {
   const RowGeom& g = rb.g;
   const bool pz = (g.periodic & 4) != 0;
   if (pz && !allow_periodic) {
@@ -183,9 +184,11 @@ inline bool build_windows(const RowBuild& rb, bool allow_periodic, WinBuild& wb,
   };
   // (parallel_ranges counts items of about a cell's work)
   const int64_t per = static_cast<int64_t>(wb.PY) * wb.W;
-  parallel_ranges(PX * per, [&](int64_t b, int64_t e, int) {
+  auto fill = [&](int64_t b, int64_t e, int) {
     for (int64_t px = (b + per - 1) / per; px * per < e; ++px) plane(static_cast<int32_t>(px));
-  });
+  };
+  if (threads) parallel_ranges(PX * per, fill);
+  else fill(0, PX * per, 0);
   if (!fits) {
     why = "x plane above 2^22 nodes";
     return false;
