@@ -377,21 +377,24 @@ std::pair<bool, int64_t> row_source(int lattice, const RowBuild& rb, int q, int3
 // 1.8 M nodes); the two-phase fields of the 192^3 pack 4 ms for 33.
 constexpr size_t kFieldStage = size_t{32} << 20;
 
-// The stage of a context of n nodes: a vector per node, at most kFieldStage.
-int alloc_stage(lb_ctx* c, int64_t n) {
-  const size_t want = std::max<size_t>(std::min(kFieldStage, static_cast<size_t>(n) * 3 * sizeof(double)), 64);
-  if (want > c->stage_bytes) {
-    if (c->field_stage) hipHostFree(c->field_stage);
-    c->field_stage = nullptr;
-    c->stage_bytes = 0;
-    const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&c->field_stage), want, hipHostMallocDefault);
-    if (e != hipSuccess)
-      return fail(c, LB_ERR_NOMEM, "hipHostMalloc(%zu bytes) for fields: %s", want, hipGetErrorString(e));
-    c->stage_bytes = want;
-  }
+// The stage of a context: a vector per node, at most kFieldStage.  Made at the
+// first field download of a topology, so that a context that downloads none pins
+// nothing; false where it cannot be pinned.
+bool have_stage(lb_ctx* c) {
+  const size_t want = std::max<size_t>(std::min(kFieldStage, static_cast<size_t>(c->n_bulk) * 3 * sizeof(double)), 64);
+  bool ok = c->field_stage || hipHostMalloc(reinterpret_cast<void**>(&c->field_stage), want, hipHostMallocDefault) == hipSuccess;
+  if (ok) c->stage_bytes = want;
+  else c->field_stage = nullptr;
   for (hipEvent_t& ev : c->stage_ev)
-    if (!ev) LB_HIP(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  return LB_OK;
+    ok = ok && (ev || hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess);
+  if (!ok) (void)hipGetLastError();  // not the next launch's error
+  return ok;
+}
+
+void free_stage(lb_ctx* c) {
+  if (c->field_stage) hipHostFree(c->field_stage);
+  c->field_stage = nullptr;
+  c->stage_bytes = 0;
 }
 
 int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const int16_t* node_type,
@@ -564,6 +567,7 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
   free_fields(c);
   free_tags(c);
   free_halos(c);
+  free_stage(c);
   c->n_ghost = 0;
   c->slot_of.clear();
   for (void* p : {static_cast<void*>(c->d_coord), static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win),
@@ -666,7 +670,6 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
     if ((rc = dev_alloc(c, &c->d_rank, rank.size())) != LB_OK) return rc;
     LB_HIP(c, hipMemcpy(c->d_rank, rank.data(), rank.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   }
-  if ((rc = alloc_stage(c, n_bulk)) != LB_OK) return rc;
   c->wall_nodes = walls;
   c->node_type.assign(node_type, node_type + n_nodes);
   c->n_ghost = n_ghost;
@@ -725,7 +728,7 @@ int lb_ctx_destroy(lb_ctx* c) {
                   static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win), static_cast<void*>(c->d_table),
                   static_cast<void*>(c->d_rank), static_cast<void*>(c->d_order), static_cast<void*>(c->d_node)})
     if (p) hipFree(p);
-  if (c->field_stage) hipHostFree(c->field_stage);
+  free_stage(c);
   for (hipEvent_t e : c->stage_ev)
     if (e) hipEventDestroy(e);
   hipEventDestroy(c->ev0);
@@ -946,9 +949,28 @@ int lb_init_equilibrium(lb_ctx* c, int32_t n_fields, int32_t field, int32_t rho_
 }  // extern "C"
 
 namespace {
+// Without pinned memory: the components copied to pageable memory as they lie
+// on the device, and reordered from there.
+int download_nodes_pageable(lb_ctx* c, const void* src, bool is_float, int nc, double* out) {
+  const size_t bytes = static_cast<size_t>(nc) * c->NP * (is_float ? sizeof(float) : sizeof(double));
+  std::unique_ptr<char[]> h(new (std::nothrow) char[bytes]);
+  if (!h) return fail(c, LB_ERR_NOMEM, "field download: no host memory");
+  LB_HIP(c, hipMemcpyAsync(h.get(), src, bytes, hipMemcpyDeviceToHost, c->stream));
+  LB_HIP(c, hipStreamSynchronize(c->stream));
+  auto copy = [&](const auto* in) {
+    for (int64_t i = 0; i < c->n_bulk; ++i)
+      for (int d = 0; d < nc; ++d)
+        out[static_cast<size_t>(c->node_of[i]) * nc + d] = static_cast<double>(in[d * c->NP + i]);
+  };
+  if (is_float) copy(reinterpret_cast<const float*>(h.get()));
+  else copy(reinterpret_cast<const double*>(h.get()));
+  return LB_OK;
+}
+
 int download_nodes(lb_ctx* c, const void* src, bool is_float, int nc, double* out) {
   const int64_t n = c->n_bulk;
   if (n == 0) return LB_OK;
+  if (!have_stage(c)) return download_nodes_pageable(c, src, is_float, nc, out);
   const size_t rec = static_cast<size_t>(nc) * sizeof(double);
   // one slab if it fits the whole stage, else slabs of half of it in turn
   const bool whole = static_cast<size_t>(n) * rec <= c->stage_bytes;

@@ -30,8 +30,8 @@ struct lb_ctx {
   int32_t* d_rank = nullptr;
   std::vector<std::array<int32_t, 3>> bulk_runs;
   int32_t* d_node = nullptr;    // compact node at each position, null where it is the position itself
-  // pinned staging of the node fields (lb_download_scalar / _vector), made with
-  // the topology, at most kFieldStage bytes
+  // pinned staging of the node fields (lb_download_scalar / _vector), made at a
+  // topology's first field download, at most kFieldStage bytes
   double* field_stage = nullptr;
   size_t stage_bytes = 0;
   hipEvent_t stage_ev[2] = {nullptr, nullptr};

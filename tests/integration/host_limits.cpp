@@ -1,0 +1,106 @@
+// Contexts where pinned host memory is short.  The program's own hipHostMalloc
+// stands before the runtime's: it counts the calls and, with "nopin", refuses
+// them.  argv: pin | nopin, output file (every downloaded value, as doubles).
+#include <dlfcn.h>
+
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "badchimp_amd.h"
+
+static int pins = 0;
+static bool refuse = false;
+extern "C" int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
+  using Malloc = int (*)(void**, size_t, unsigned);
+  static const Malloc next = reinterpret_cast<Malloc>(dlsym(RTLD_NEXT, "hipHostMalloc"));
+  ++pins;
+  return refuse ? 2 /* hipErrorOutOfMemory */ : next(p, bytes, flags);
+}
+
+static lb_ctx* ctx = nullptr;
+static void ok(int rc, const char* what) {
+  if (rc == LB_OK) return;
+  std::printf("%s: %d %s\n", what, rc, lb_last_error(ctx));
+  std::exit(1);
+}
+static std::vector<double> all;
+static void keep(const std::vector<double>& v) { all.insert(all.end(), v.begin(), v.end()); }
+
+struct Lists {
+  int32_t n = 0;
+  std::vector<int32_t> nb, pos, bulk;
+  std::vector<int16_t> types;
+};
+static Lists lists(const int32_t* dims, const std::vector<int32_t>& geo, int rank) {
+  lb_topo* t = nullptr;
+  ok(lb_topo_from_geometry(LB_D3Q19, 3, dims, geo.data(), 1, rank, &t), "geometry");
+  Lists l;
+  l.n = lb_topo_num_nodes(t);
+  l.nb.resize(static_cast<size_t>(l.n) * 19);
+  l.pos.resize(static_cast<size_t>(l.n) * 3);
+  l.types.resize(l.n);
+  l.bulk.resize(lb_topo_num_bulk(t));
+  ok(lb_topo_neighbors(t, l.nb.data()), "neighbours");
+  ok(lb_topo_positions(t, l.pos.data()), "positions");
+  ok(lb_topo_node_types(t, l.types.data()), "types");
+  ok(lb_topo_bulk(t, l.bulk.data()), "bulk");
+  lb_topo_destroy(t);
+  return l;
+}
+static void set(const Lists& l, int precision) {
+  ok(lb_ctx_create(LB_D3Q19, precision, 0, &ctx), "context");
+  ok(lb_set_topology_grid(ctx, l.n, l.nb.data(), l.types.data(), l.bulk.data(), static_cast<int32_t>(l.bulk.size()),
+                          l.pos.data(), 0),
+     "topology");
+}
+static void fields(int n, int nf) {
+  std::vector<double> rho(static_cast<size_t>(n) * nf), vel(static_cast<size_t>(n) * 3), phi(n);
+  ok(lb_download_scalar(ctx, LB_RHO, nf, rho.data()), "density");
+  ok(lb_download_vector(ctx, LB_VEL, 1, vel.data()), "velocity");
+  keep(rho);
+  keep(vel);
+  if (nf == 2) {
+    ok(lb_download_scalar(ctx, LB_PHI, 1, phi.data()), "colour");
+    keep(phi);
+  }
+}
+
+int main(int argc, char** argv) {
+  if (argc != 3) return 2;
+  refuse = !std::strcmp(argv[1], "nopin");
+  const int32_t dims[3] = {20, 18, 33};
+  std::vector<int32_t> geo(20 * 18 * 33), split;
+  uint32_t r = 7;
+  for (size_t k = 0; k < geo.size(); ++k) {
+    const size_t y = k / 33 % 18, z = k % 33;
+    r = r * 1664525u + 1013904223u;
+    geo[k] = y != 0 && y != 17 && z != 0 && z != 32 && r >> 30 != 0;
+  }
+  const double force[3] = {1e-4, 2e-5, 0.0};
+  const Lists whole = lists(dims, geo, 1);
+  std::vector<double> rho(static_cast<size_t>(whole.n) * 2), rest(static_cast<size_t>(whole.n) * 3, 0.0);
+  for (int32_t k = 0; k < whole.n; ++k) {
+    rho[2 * k] = 0.2 + 0.01 * (k % 60);
+    rho[2 * k + 1] = 1.0 - rho[2 * k];
+  }
+  // one field in FP64, two in float storage
+  set(whole, LB_FP64);
+  ok(lb_init_equilibrium(ctx, 1, 0, 2, 0, rho.data(), rest.data()), "initial state");
+  ok(lb_step_bgk(ctx, 7, 0.9, force), "steps");
+  std::printf("pinned before a download %d\n", pins);
+  fields(whole.n, 1);
+  lb_ctx_destroy(ctx);
+  set(whole, LB_FP32S);
+  ok(lb_set_wall_densities(ctx, rho.data()), "wall densities");
+  for (int k = 0; k < 2; ++k) ok(lb_init_equilibrium(ctx, 2, k, 2, k, rho.data(), rest.data()), "initial state");
+  ok(lb_step_cg(ctx, 5, 0.9, 1.1, 0.01, 0.7, LB_FORCE_FIXED, force), "two-phase steps");
+  fields(whole.n, 2);
+  lb_ctx_destroy(ctx);
+  std::FILE* f = std::fopen(argv[2], "wb");
+  if (!f || std::fwrite(all.data(), sizeof(double), all.size(), f) != all.size() || std::fclose(f)) return 1;
+  std::printf("pinned %d, %zu values\n", pins, all.size());
+  return 0;
+}

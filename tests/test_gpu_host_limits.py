@@ -1,0 +1,47 @@
+"""Calls that stage values in pinned host memory, where that memory cannot be
+had (tests/integration/host_limits.cpp refuses hipHostMalloc): the same values
+through ordinary memory.  Set-up and steps pin none."""
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import lbamd
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "badchimp-cpp_amd", "lib")
+
+
+@pytest.fixture(scope="module")
+def limits(tmp_path_factory):
+    """run(mode): (stdout, values) of the program."""
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    lbamd.lib()  # built
+    tmp = tmp_path_factory.mktemp("limits")
+    exe = str(tmp / "host_limits")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "integration", "host_limits.cpp"), "-o", exe, "-L", LIB,
+                    "-lbadchimp_amd", "-Wl,-rpath," + LIB, "-L/opt/rocm/lib", "-Wl,-rpath-link,/opt/rocm/lib",
+                    "-Wl,-rpath,/opt/rocm/lib", "-ldl"], check=True, capture_output=True, timeout=100)
+
+    def run(mode):
+        out = str(tmp / mode)
+        r = subprocess.run([exe, mode, out], capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, (r.returncode, r.stdout, r.stderr[-2000:])
+        return r.stdout, np.fromfile(out)
+    return run
+
+
+def test_fields_without_pinned_memory(gpu_available, limits):
+    text, pinned = limits("pin")
+    assert "pinned before a download 0\n" in text and int(re.search(r"pinned (\d+),", text).group(1)) >= 2, text
+    text, plain = limits("nopin")
+    assert int(re.search(r"pinned (\d+),", text).group(1)) >= 2, text
+    assert pinned.size > 20000 and np.abs(pinned).max() > 0.1
+    assert np.array_equal(pinned, plain)
