@@ -148,12 +148,8 @@ int alloc_fields(lb_ctx* c, int nf) {
     c->bytes += static_cast<int64_t>(bytes);
   }
   c->n_fields = nf;
-  // Block order of the row windows.  Measured (order against node_block, us per
-  // step): FP32S 128^3 26.1 / 27.3, 165^3 50.9 / 52.9, 256^3 187 / 188; FP64
-  // 64^3 9.7 / 10.4, 128^3 47.6 / 49.0, 256^3 358 / 351 (1.0 GB per buffer,
-  // bound by the HBM, which the wider front serves less well); two-phase
-  // FP64 192^3 439 / 453 (0.8 GB per buffer), FP32S 222 / 239.
-  c->addr.win.order = c->addr.winz.order = nf == 1 && bytes > (size_t{900} << 20) ? nullptr : c->d_order;
+  c->addr.win.order = c->addr.winz.order =
+      plane_order(nf, static_cast<int64_t>(elem_size(c->precision)), static_cast<int64_t>(bytes)) ? c->d_order : nullptr;
   c->addr.nt = stream_stores(2 * static_cast<int64_t>(bytes));
   c->cur = 0;
   c->post = false;

@@ -37,6 +37,28 @@ inline bool stream_stores(int64_t both_buffers) {
   return both_buffers < 20000000 || both_buffers > (int64_t{256} << 20);
 }
 
+// Whether the blocks of the row windows go to the XCDs plane by plane
+// (block_order in rowbuild.hpp) or in runs of 4 (node_block), by the bytes of one
+// population buffer and the storage form.  The plane order reads neighbouring rows
+// from the XCD's own L2; its front is wider, eight runs of a plane, and from some
+// size of the buffers on that costs more at the HBM than the L2 saves.  Plane
+// order / runs, us per step, sphere packs of porosity 0.4 by MB per buffer:
+// FP64    122 40.8 / 45.1, 291 105.2 / 106.8, 552 199.6 / 201.3, 635 226.1 /
+//         229.2, 689 245.8 / 246.4; 725 263.2 / 260.3, 889 323.8 / 314.9, 1462
+//         536.6 / 514.8, 2158 791.2 / 760.6; porosity 0.8, 817 281.7 / 279.8
+// FP32S   276 105.6 / 107.6, 538 203.2 / 204.5, 602 230.0 / 231.6, 644 246.1 /
+//         245.9; 731 279.4 / 274.1, 1079 415.0 / 404.8, 2073 828.2 / 783.7
+// FP16S   644 342.3 / 342.2, 761 397.7 / 401.6; 892 466.5 / 463.3, 1036 548.6 / 535.0
+// two fields, both of them counted:
+// FP64    852 439 / 453, 1451 788.6 / 791.9, 2150 1171 / 1173; 3233 1802 / 1769,
+//         3858 2160 / 2114
+// FP32S   1075 627.4 / 635.9; 1462 857.7 / 854.2, 2158 1298 / 1272
+// FP16S   1288 1033 / 1051, 1784 1421 / 1441 (larger ones not timed)
+inline bool plane_order(int n_fields, int64_t elem_bytes, int64_t buffer) {
+  if (n_fields == 1) return buffer <= (elem_bytes == 2 ? 820000000 : 700000000);
+  return buffer <= (elem_bytes == 8 ? 2300000000 : elem_bytes == 4 ? 1350000000 : int64_t{1} << 32);
+}
+
 // Layout of a launch over n_fields fields: the context's layout, with the row
 // windows replaced by the rows
 // (64-bit addresses, same sources) when the fields do not fit below 4 GiB.

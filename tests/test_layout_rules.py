@@ -1,0 +1,37 @@
+"""The rules that choose between two forms of a step (csrc/layout_select.hpp)
+take the faster one at the sizes where both were timed (MI355X; us per step,
+as the comments of the rules give them; differences under 1 % are left out)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# fields, bytes per element, MB of one population buffer: plane order, runs of 4
+ORDER = [
+    (1, 8, 122, 40.83, 45.08), (1, 8, 291, 105.22, 106.80), (1, 8, 635, 226.09, 229.17), (1, 8, 725, 263.24, 260.32),
+    (1, 8, 801, 289.94, 285.54), (1, 8, 889, 323.77, 314.89), (1, 8, 1462, 536.63, 514.82),
+    (1, 8, 2158, 791.23, 760.64), (1, 4, 276, 105.57, 107.62), (1, 4, 731, 279.40, 274.13),
+    (1, 4, 1079, 414.97, 404.83), (1, 4, 1522, 585.29, 577.75), (1, 4, 2073, 828.17, 783.68),
+    (1, 2, 1036, 548.56, 535.02), (2, 8, 852, 439.0, 453.0), (2, 8, 3233, 1801.54, 1769.08),
+    (2, 8, 3858, 2160.10, 2113.84), (2, 4, 1075, 627.38, 635.91), (2, 4, 2158, 1298.15, 1272.02),
+    (2, 2, 1288, 1032.99, 1050.91), (2, 2, 1784, 1420.92, 1441.10),
+]
+
+
+def rules(tmp_path, lines):
+    """The values of C++ expressions over csrc/layout_select.hpp."""
+    src, exe = tmp_path / "r.cpp", str(tmp_path / "r")
+    src.write_text("#include <cstdio>\n#include \"layout_select.hpp\"\nint main() {\n  using namespace lbamd;\n"
+                   + "".join('  std::printf("%%d\\n", int(%s));\n' % x for x in lines) + "}\n")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "badchimp-cpp_amd", "csrc"), str(src), "-o",
+                    exe], check=True, capture_output=True)
+    return list(map(int, subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split()))
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_block_order_is_the_faster_one(tmp_path):
+    got = rules(tmp_path, ["plane_order(%d, %d, %d000000LL)" % r[:3] for r in ORDER])
+    assert got == [int(r[3] < r[4]) for r in ORDER]
