@@ -228,17 +228,24 @@ inline std::pair<bool, int64_t> win_source(int lattice, const RowBuild& rb, cons
 // every plane goes to XCD k: the rows that a gather reaches, and the node's own
 // lines that its bounce-back reads, were read or will be by the same XCD.  On
 // the 256^3 pack in FP32S the L2s then fetch 1.11x the populations instead of
-// 1.55x (node_block: runs of 4 blocks round-robin).  Planes of fewer than 2
-// blocks on average (two dimensions) have their neighbours in the blocks before
-// and after: there an XCD takes runs of blocks, long ones (n / 8 blocks, at
-// most 32).
+// 1.55x (node_block: runs of 4 blocks round-robin).  Planes of fewer than 8 blocks
+// on average have runs shorter than a block, so that a block reaches into several
+// of them: there an XCD takes runs of consecutive blocks, long ones (n / 8 blocks,
+// at most 32), which hold several planes.  Runs of 32 / plane by plane / runs of 4,
+// us per step by blocks per plane: D2Q9 channel FP64 258x620 (2.4) 5.36 / 8.18 /
+// 6.51, 177x900 (3.5) 5.42 / 8.14 / 7.44, 106x1500 (5.9) 5.51 / 5.91 / 8.02; FP32S
+// 258x620 4.06 / 4.91 / 4.60, 1000x1900 (7.4) 23.2 / 24.8 / 24.4; packs FP64
+// 90x28x28 open (2.6) 4.92 / 6.48 / 5.29, 48^3 (3.6) 5.00 / 5.18 / 5.32, 64^3 (6)
+// 7.2 / 7.9 / 8.8, 74^3 (8) 11.20 / 11.25 / 11.86; FP32S 900x56x56 (4.6) 27.1 / 31.6
+// / 32.9; from 8 on 80^3 (9.3) FP32S 7.71 / 7.70, FP16S 6.57 / 6.49, 32x64x64 open
+// (15) FP64 8.4 / 7.9.
 inline std::vector<uint8_t> block_xcd(const std::vector<uint32_t>& coord) {
   const int64_t n = static_cast<int64_t>(coord.size()), nb = (n + kBlock - 1) / kBlock;
   std::vector<uint8_t> xcd(static_cast<size_t>(nb));
   std::vector<int64_t> start;  // first node of each plane
   for (auto it = coord.begin(); it != coord.end(); it = std::upper_bound(it, coord.end(), *it | 0x3fffffu))
     start.push_back(it - coord.begin());
-  if (nb < 2 * static_cast<int64_t>(start.size())) {
+  if (nb < 8 * static_cast<int64_t>(start.size())) {
     const int64_t run = std::min<int64_t>(32, (nb + 7) / 8);
     for (int64_t b = 0; b < nb; ++b) xcd[b] = static_cast<uint8_t>((b / run) % 8);
     return xcd;

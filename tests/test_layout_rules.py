@@ -35,3 +35,42 @@ def rules(tmp_path, lines):
 def test_block_order_is_the_faster_one(tmp_path):
     got = rules(tmp_path, ["plane_order(%d, %d, %d000000LL)" % r[:3] for r in ORDER])
     assert got == [int(r[3] < r[4]) for r in ORDER]
+
+
+XCDS = r'''
+#include "rowbuild.hpp"
+#include <cstdio>
+using namespace lbamd;
+// box of x planes of ny x nz fluid cells: 1 where consecutive blocks share an XCD
+// in long runs, 2 where every plane's blocks go to the XCDs in order, else 0
+static int form(int nx, int ny, int nz) {
+  std::vector<uint32_t> coord;
+  for (int x = 0; x < nx; ++x)
+    for (int y = 0; y < ny; ++y)
+      for (int z = 0; z < nz; ++z) coord.push_back(uint32_t(x) << 22 | uint32_t(y) << 12 | uint32_t(z));
+  const std::vector<uint8_t> xcd = block_xcd(coord);
+  int64_t changes = 0, mids = 0;
+  for (size_t b = 1; b < xcd.size(); ++b) changes += xcd[b] != xcd[b - 1];
+  for (size_t b = 0; b < xcd.size(); ++b) {
+    const int64_t mid = std::min<int64_t>(coord.size() - 1, 256 * b + 128), n = ny * nz;
+    mids += xcd[b] == mid % n * 8 / n;
+  }
+  const int64_t nb = xcd.size(), run = std::min<int64_t>(32, (nb + 7) / 8);
+  return changes == (nb - 1) / run ? 1 : mids == nb ? 2 : 0;
+}
+int main() {
+  std::printf("%d %d %d %d %d %d %d\n", form(300, 1, 300), form(258, 1, 620), form(177, 1, 900), form(60, 30, 40),
+              form(90, 37, 55), form(40, 32, 64), form(70, 60, 60));
+}
+'''
+
+
+def test_blocks_of_thin_planes_go_to_the_xcds_in_long_runs(tmp_path):
+    """Planes of 1.2, 2.4, 3.5, 4.7 and 7.9 blocks in runs of blocks, of 8 and 14 plane by plane."""
+    src, exe = tmp_path / "x.hip", str(tmp_path / "x")
+    src.write_text(XCDS)
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-arch=gfx950", "-std=c++17", "-O1", "-I",
+                    os.path.join(ROOT, "badchimp-cpp_amd", "csrc"), str(src), "-o", exe], check=True,
+                   capture_output=True)
+    out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout
+    assert out.split() == ["1", "1", "1", "1", "1", "2", "2"], out
