@@ -373,24 +373,65 @@ std::pair<bool, int64_t> row_source(int lattice, const RowBuild& rb, int q, int3
 // 1.8 M nodes); the two-phase fields of the 192^3 pack 4 ms for 33.
 constexpr size_t kFieldStage = size_t{32} << 20;
 
-// The stage of a context: a vector per node, at most kFieldStage.  Made at the
-// first field download of a topology, so that a context that downloads none pins
-// nothing; false where it cannot be pinned.
-bool have_stage(lb_ctx* c) {
-  const size_t want = std::max<size_t>(std::min(kFieldStage, static_cast<size_t>(c->n_bulk) * 3 * sizeof(double)), 64);
-  bool ok = c->field_stage || hipHostMalloc(reinterpret_cast<void**>(&c->field_stage), want, hipHostMallocDefault) == hipSuccess;
-  if (ok) c->stage_bytes = want;
-  else c->field_stage = nullptr;
-  for (hipEvent_t& ev : c->stage_ev)
-    ok = ok && (ev || hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess);
-  if (!ok) (void)hipGetLastError();  // not the next launch's error
-  return ok;
+// Stages are lent to one download at a time and kept for the next one, of any
+// context: pinning 32 MiB takes 1.5 ms with its first use, as long as a small
+// context's download.  At most kIdleStages wait in the process; the last context
+// that is destroyed frees them.
+struct FieldStage {
+  double* p = nullptr;
+  size_t bytes = 0;
+};
+constexpr size_t kIdleStages = 4;
+std::mutex g_stage_mu;
+std::vector<FieldStage> g_idle_stages;
+int g_contexts = 0;
+
+// A stage of at least `want` bytes; none where it cannot be pinned.
+FieldStage take_stage(size_t want) {
+  FieldStage s;
+  {
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    if (!g_idle_stages.empty()) {  // the largest one, or in place of it
+      auto it = std::max_element(g_idle_stages.begin(), g_idle_stages.end(),
+                                 [](const FieldStage& x, const FieldStage& y) { return x.bytes < y.bytes; });
+      s = *it;
+      g_idle_stages.erase(it);
+    }
+  }
+  if (s.bytes >= want) return s;
+  if (s.p) hipHostFree(s.p);
+  s = FieldStage{};
+  size_t bytes = size_t{1} << 20;
+  while (bytes < want) bytes *= 2;
+  if (hipHostMalloc(reinterpret_cast<void**>(&s.p), bytes, hipHostMallocPortable) == hipSuccess) {
+    s.bytes = bytes;
+  } else {
+    s.p = nullptr;
+    (void)hipGetLastError();  // not the next launch's error
+  }
+  return s;
 }
 
-void free_stage(lb_ctx* c) {
-  if (c->field_stage) hipHostFree(c->field_stage);
-  c->field_stage = nullptr;
-  c->stage_bytes = 0;
+void give_stage(FieldStage s) {
+  if (!s.p) return;
+  {
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    if (g_contexts > 0 && g_idle_stages.size() < kIdleStages) {
+      g_idle_stages.push_back(s);
+      return;
+    }
+  }
+  hipHostFree(s.p);
+}
+
+void count_context(int d) {
+  std::vector<FieldStage> gone;
+  {
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    g_contexts += d;
+    if (g_contexts == 0) gone.swap(g_idle_stages);
+  }
+  for (const FieldStage& s : gone) hipHostFree(s.p);
 }
 
 int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const int16_t* node_type,
@@ -563,7 +604,6 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
   free_fields(c);
   free_tags(c);
   free_halos(c);
-  free_stage(c);
   c->n_ghost = 0;
   c->slot_of.clear();
   for (void* p : {static_cast<void*>(c->d_coord), static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win),
@@ -707,6 +747,7 @@ int lb_ctx_create(int lattice, int precision, int device, lb_ctx** out) {
     return fail_global(LB_ERR_HIP, "stream/event creation failed");
   }
   scratch_setup(device);
+  count_context(1);
   *out = c;
   return LB_OK;
 }
@@ -724,13 +765,13 @@ int lb_ctx_destroy(lb_ctx* c) {
                   static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win), static_cast<void*>(c->d_table),
                   static_cast<void*>(c->d_rank), static_cast<void*>(c->d_order), static_cast<void*>(c->d_node)})
     if (p) hipFree(p);
-  free_stage(c);
   for (hipEvent_t e : c->stage_ev)
     if (e) hipEventDestroy(e);
   hipEventDestroy(c->ev0);
   hipEventDestroy(c->ev1);
   hipStreamDestroy(c->stream);
   delete c;
+  count_context(-1);
   return LB_OK;
 }
 
@@ -966,12 +1007,19 @@ int download_nodes_pageable(lb_ctx* c, const void* src, bool is_float, int nc, d
 int download_nodes(lb_ctx* c, const void* src, bool is_float, int nc, double* out) {
   const int64_t n = c->n_bulk;
   if (n == 0) return LB_OK;
-  if (!have_stage(c)) return download_nodes_pageable(c, src, is_float, nc, out);
+  struct Lease {
+    FieldStage s;
+    ~Lease() { give_stage(s); }
+  } stage{take_stage(std::min(kFieldStage, static_cast<size_t>(n) * 3 * sizeof(double)))};
+  bool ready = stage.s.p != nullptr;
+  for (hipEvent_t& ev : c->stage_ev)
+    ready = ready && (ev || hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess);
+  if (!ready) return download_nodes_pageable(c, src, is_float, nc, out);
   const size_t rec = static_cast<size_t>(nc) * sizeof(double);
   // one slab if it fits the whole stage, else slabs of half of it in turn
-  const bool whole = static_cast<size_t>(n) * rec <= c->stage_bytes;
-  const int64_t slab = whole ? n : static_cast<int64_t>(c->stage_bytes / 2 / rec);
-  double* half[2] = {c->field_stage, c->field_stage + (whole ? 0 : slab * nc)};
+  const bool whole = static_cast<size_t>(n) * rec <= stage.s.bytes;
+  const int64_t slab = whole ? n : static_cast<int64_t>(stage.s.bytes / 2 / rec);
+  double* half[2] = {stage.s.p, stage.s.p + (whole ? 0 : slab * nc)};
   const int64_t slabs = (n + slab - 1) / slab;
   auto enqueue = [&](int64_t k) -> hipError_t {
     hipError_t e = nodes_out(src, is_float, c->NP, nc, c->d_node, k * slab, std::min(slab, n - k * slab), half[k & 1],

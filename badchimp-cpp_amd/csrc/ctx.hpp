@@ -30,11 +30,7 @@ struct lb_ctx {
   int32_t* d_rank = nullptr;
   std::vector<std::array<int32_t, 3>> bulk_runs;
   int32_t* d_node = nullptr;    // compact node at each position, null where it is the position itself
-  // pinned staging of the node fields (lb_download_scalar / _vector), made at a
-  // topology's first field download, at most kFieldStage bytes
-  double* field_stage = nullptr;
-  size_t stage_bytes = 0;
-  hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};  // of a field download's two slabs
   std::vector<int32_t> wall_nodes;  // wall slot -> node number
   // other-rank fluid nodes (type 4, the halo): population slots after the
   // bulk nodes in compact order; slot_of[node] = compact index (bulk, then

@@ -92,12 +92,15 @@ int main(int argc, char** argv) {
   ok(lb_step_bgk(ctx, 7, 0.9, force), "steps");
   std::printf("pinned before a download %d\n", pins);
   fields(whole.n, 1);
-  lb_ctx_destroy(ctx);
+  lb_ctx* const one = ctx;
   set(whole, LB_FP32S);
   ok(lb_set_wall_densities(ctx, rho.data()), "wall densities");
   for (int k = 0; k < 2; ++k) ok(lb_init_equilibrium(ctx, 2, k, 2, k, rho.data(), rest.data()), "initial state");
   ok(lb_step_cg(ctx, 5, 0.9, 1.1, 0.01, 0.7, LB_FORCE_FIXED, force), "two-phase steps");
   fields(whole.n, 2);
+  lb_ctx_destroy(ctx);
+  ctx = one;
+  fields(whole.n, 1);
   lb_ctx_destroy(ctx);
   std::FILE* f = std::fopen(argv[2], "wb");
   if (!f || std::fwrite(all.data(), sizeof(double), all.size(), f) != all.size() || std::fclose(f)) return 1;

@@ -1,6 +1,7 @@
 """Calls that stage values in pinned host memory, where that memory cannot be
 had (tests/integration/host_limits.cpp refuses hipHostMalloc): the same values
-through ordinary memory.  Set-up and steps pin none."""
+through ordinary memory.  Set-up and steps pin none, and the downloads of two
+contexts in turn share one piece."""
 import os
 import re
 import shutil
@@ -40,7 +41,7 @@ def limits(tmp_path_factory):
 
 def test_fields_without_pinned_memory(gpu_available, limits):
     text, pinned = limits("pin")
-    assert "pinned before a download 0\n" in text and int(re.search(r"pinned (\d+),", text).group(1)) >= 2, text
+    assert "pinned before a download 0\n" in text and "pinned 1," in text, text
     text, plain = limits("nopin")
     assert int(re.search(r"pinned (\d+),", text).group(1)) >= 2, text
     assert pinned.size > 20000 and np.abs(pinned).max() > 0.1
