@@ -2029,14 +2029,15 @@ int lb_halo_add(lb_ctx* c, int32_t neighbor_rank, int32_t n_send, const int32_t*
   if (e == hipSuccess) e = upload(&h.d_send_nodes, ns);
   if (e == hipSuccess) e = upload(&h.d_recv_nodes, nr);
   if (e == hipSuccess) e = hipMalloc(&h.d_buf, nbuf * sizeof(double));
-  if (e == hipSuccess)
-    e = hipHostMalloc(reinterpret_cast<void**>(&h.h_buf), nbuf * sizeof(double), hipHostMallocDefault);
   if (e != hipSuccess) {
-    if (h.h_buf) hipHostFree(h.h_buf);
     for (void* p : {static_cast<void*>(h.d_send), static_cast<void*>(h.d_recv), static_cast<void*>(h.d_send_nodes),
                     static_cast<void*>(h.d_recv_nodes), static_cast<void*>(h.d_buf)})
       if (p) hipFree(p);
     return fail(c, LB_ERR_NOMEM, "lb_halo_add: %s", hipGetErrorString(e));
+  }
+  if (hipHostMalloc(reinterpret_cast<void**>(&h.h_buf), nbuf * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    h.h_buf = nullptr;  // the copies to and from d_buf serve all buffers then
+    (void)hipGetLastError();
   }
   c->halos.push_back(h);
   *index = static_cast<int32_t>(c->halos.size()) - 1;
@@ -2073,7 +2074,7 @@ bool plain_host(const void* p) {
 template <class F>
 hipError_t halo_out(lb_ctx* c, const lb_ctx::Halo& h, int64_t n, double* to, F&& pack) {
   if (n <= 0) return hipStreamSynchronize(c->stream);
-  const bool host = plain_host(to);
+  const bool host = h.h_buf && plain_host(to);
   hipError_t e = pack(host ? h.h_buf : h.d_buf);
   if (e == hipSuccess && !host) e = hipMemcpyAsync(to, h.d_buf, n * sizeof(double), hipMemcpyDefault, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -2085,7 +2086,7 @@ hipError_t halo_out(lb_ctx* c, const lb_ctx::Halo& h, int64_t n, double* to, F&&
 template <class F>
 hipError_t halo_in(lb_ctx* c, const lb_ctx::Halo& h, int64_t n, const double* from, F&& unpack) {
   if (n <= 0) return hipStreamSynchronize(c->stream);
-  const bool host = plain_host(from);
+  const bool host = h.h_buf && plain_host(from);
   hipError_t e = hipSuccess;
   if (host) std::memcpy(h.h_buf, from, static_cast<size_t>(n) * sizeof(double));
   else e = hipMemcpyAsync(h.d_buf, from, n * sizeof(double), hipMemcpyDefault, c->stream);

@@ -49,7 +49,7 @@ struct lb_ctx {
     uint32_t* d_send_nodes = nullptr;
     uint32_t* d_recv_nodes = nullptr;
     double* d_buf = nullptr;
-    double* h_buf = nullptr;  // the same in pinned host memory
+    double* h_buf = nullptr;  // the same in pinned host memory, or null where none could be had
   };
   std::vector<Halo> halos;
   std::vector<int16_t> node_type;

@@ -1,6 +1,7 @@
 // Contexts where pinned host memory is short.  The program's own hipHostMalloc
 // stands before the runtime's: it counts the calls and, with "nopin", refuses
-// them.  argv: pin | nopin, output file (every downloaded value, as doubles).
+// them.  argv: pin | nopin, output file (every downloaded value, as doubles), and
+// the memory of the halo buffers: pageable | pinned | device | managed.
 #include <dlfcn.h>
 
 #include <cstdint>
@@ -20,6 +21,14 @@ extern "C" int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
   return refuse ? 2 /* hipErrorOutOfMemory */ : next(p, bytes, flags);
 }
 
+extern "C" {
+int hipMalloc(void**, size_t);
+int hipMallocManaged(void**, size_t, unsigned);
+int hipMemcpy(void*, const void*, size_t, int);
+int hipFree(void*);
+int hipHostFree(void*);
+}
+
 static lb_ctx* ctx = nullptr;
 static void ok(int rc, const char* what) {
   if (rc == LB_OK) return;
@@ -28,6 +37,33 @@ static void ok(int rc, const char* what) {
 }
 static std::vector<double> all;
 static void keep(const std::vector<double>& v) { all.insert(all.end(), v.begin(), v.end()); }
+
+// a halo buffer of n doubles in the memory asked for
+struct Buffer {
+  char kind;  // second letter: a(geable), i(nned), e(vice), managed as M
+  size_t n;
+  double* p = nullptr;
+  Buffer(const char* name, size_t count) : kind(*name == 'm' ? 'M' : name[1]), n(count) {
+    void** q = reinterpret_cast<void**>(&p);
+    const int e = kind == 'e' ? hipMalloc(q, n * 8) : kind == 'M' ? hipMallocManaged(q, n * 8, 1)
+                  : kind == 'i' ? hipHostMalloc(q, n * 8, 0) : (*q = std::calloc(n, 8)) == nullptr;
+    if (e != 0) {
+      std::printf("%s buffer: %d\n", name, e);
+      std::exit(1);
+    }
+  }
+  ~Buffer() {
+    if (kind == 'e' || kind == 'M') (void)hipFree(p);
+    else if (kind == 'i') (void)hipHostFree(p);
+    else std::free(p);
+  }
+  void set(const std::vector<double>& v) { ok(hipMemcpy(p, v.data(), v.size() * 8, 4), "copy in"); }
+  std::vector<double> get(size_t count) const {
+    std::vector<double> v(count);
+    ok(hipMemcpy(v.data(), p, count * 8, 4), "copy out");
+    return v;
+  }
+};
 
 struct Lists {
   int32_t n = 0;
@@ -69,7 +105,7 @@ static void fields(int n, int nf) {
 }
 
 int main(int argc, char** argv) {
-  if (argc != 3) return 2;
+  if (argc != 4) return 2;
   refuse = !std::strcmp(argv[1], "nopin");
   const int32_t dims[3] = {20, 18, 33};
   std::vector<int32_t> geo(20 * 18 * 33), split;
@@ -102,6 +138,47 @@ int main(int argc, char** argv) {
   ctx = one;
   fields(whole.n, 1);
   lb_ctx_destroy(ctx);
+  std::printf("pinned for fields %d\n", pins);
+  // a rank of a split domain with one exchange: what it packs, and its fields
+  // and colour after an unpack
+  split = geo;
+  for (size_t k = split.size() / 2; k < split.size(); ++k) split[k] *= 2;
+  const Lists part = lists(dims, split, 1);
+  std::vector<int32_t> send(part.bulk.begin(), part.bulk.begin() + 50), recv;
+  for (int32_t k = 1; k < part.n; ++k)
+    if (part.types[k] == 4) recv.push_back(k);
+  const int32_t ns = static_cast<int32_t>(send.size()), nr = static_cast<int32_t>(recv.size());
+  const std::vector<int32_t> two(send.size(), 2), one_dir(recv.size(), 1), dir(recv.size(), 3);
+  std::vector<int32_t> dirs;
+  for (int32_t k = 0; k < ns; ++k) dirs.insert(dirs.end(), {0, 4});
+  Buffer out(argv[3], 4 * send.size()), in(argv[3], 2 * recv.size());
+  std::vector<double> got(2 * recv.size());
+  for (size_t k = 0; k < got.size(); ++k) got[k] = 0.01 + 1e-4 * static_cast<double>(k % 17);
+  in.set(got);
+  for (int nf = 1; nf <= 2; ++nf) {
+    int32_t x = -1;
+    set(part, LB_FP64);
+    ok(lb_set_wall_densities(ctx, rho.data()), "wall densities");
+    ok(lb_halo_add(ctx, 1, ns, send.data(), two.data(), dirs.data(), nr, recv.data(), one_dir.data(), dir.data(), &x),
+       "exchange");
+    for (int k = 0; k < nf; ++k) ok(lb_init_equilibrium(ctx, nf, k, 2, k, rho.data(), rest.data()), "initial state");
+    for (int s = 0; s < 3; ++s) {
+      if (nf == 1) {
+        ok(lb_step_bgk(ctx, 1, 0.9, force), "step");
+      } else {
+        ok(lb_step_cg_colour(ctx, nullptr), "colour");
+        ok(lb_halo_pack_colour(ctx, x, out.p), "pack colour");
+        keep(out.get(ns));
+        ok(lb_halo_unpack_colour(ctx, x, in.p), "unpack colour");
+        ok(lb_step_cg_collide(ctx, 0.9, 1.1, 0.01, 0.7, LB_FORCE_FIXED, force, 0.0), "collision");
+      }
+      ok(lb_halo_pack(ctx, x, nf, out.p), "pack");
+      keep(out.get(2 * ns * nf));
+      ok(lb_halo_unpack(ctx, x, nf, in.p), "unpack");
+    }
+    fields(part.n, nf);
+    lb_ctx_destroy(ctx);
+  }
   std::FILE* f = std::fopen(argv[2], "wb");
   if (!f || std::fwrite(all.data(), sizeof(double), all.size(), f) != all.size() || std::fclose(f)) return 1;
   std::printf("pinned %d, %zu values\n", pins, all.size());

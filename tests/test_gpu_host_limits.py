@@ -20,7 +20,7 @@ LIB = os.path.join(ROOT, "badchimp-cpp_amd", "lib")
 
 @pytest.fixture(scope="module")
 def limits(tmp_path_factory):
-    """run(mode): (stdout, values) of the program."""
+    """run(mode, buffers): (stdout, values) of the program."""
     if shutil.which("g++") is None:
         pytest.skip("g++ not available")
     lbamd.lib()  # built
@@ -29,20 +29,27 @@ def limits(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "include"),
                     os.path.join(ROOT, "tests", "integration", "host_limits.cpp"), "-o", exe, "-L", LIB,
                     "-lbadchimp_amd", "-Wl,-rpath," + LIB, "-L/opt/rocm/lib", "-Wl,-rpath-link,/opt/rocm/lib",
-                    "-Wl,-rpath,/opt/rocm/lib", "-ldl"], check=True, capture_output=True, timeout=100)
+                    "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64", "-ldl"], check=True, capture_output=True, timeout=100)
 
-    def run(mode):
-        out = str(tmp / mode)
-        r = subprocess.run([exe, mode, out], capture_output=True, text=True, timeout=100)
+    def run(mode, buffers="pageable"):
+        out = str(tmp / (mode + buffers))
+        r = subprocess.run([exe, mode, out, buffers], capture_output=True, text=True, timeout=100)
         assert r.returncode == 0, (r.returncode, r.stdout, r.stderr[-2000:])
         return r.stdout, np.fromfile(out)
     return run
 
 
-def test_fields_without_pinned_memory(gpu_available, limits):
+def test_values_without_pinned_memory(gpu_available, limits):
+    """Fields of one and two phases, and packed and unpacked halos and colours."""
     text, pinned = limits("pin")
-    assert "pinned before a download 0\n" in text and "pinned 1," in text, text
+    assert "pinned before a download 0\n" in text and "pinned for fields 1\n" in text, text
     text, plain = limits("nopin")
-    assert int(re.search(r"pinned (\d+),", text).group(1)) >= 2, text
-    assert pinned.size > 20000 and np.abs(pinned).max() > 0.1
+    assert int(re.search(r"pinned (\d+),", text).group(1)) >= 5, text
+    assert pinned.size > 20000 and np.abs(pinned).max() > 0.1 and np.isfinite(pinned).all()
     assert np.array_equal(pinned, plain)
+
+
+@pytest.mark.parametrize("buffers", ["pinned", "device", "managed"])
+def test_halo_buffers_in_any_memory(gpu_available, limits, buffers):
+    """Packs and unpacks in the caller's pinned, device and managed memory."""
+    assert np.array_equal(limits("pin", buffers)[1], limits("pin")[1])
