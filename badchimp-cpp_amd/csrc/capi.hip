@@ -1784,30 +1784,37 @@ int solve_permeability(lb_ctx* c, const char* name, double tau, double tau_anti,
         if (x) hipGraphExecDestroy(x);
     }
   } graphs{c};
-  const bool graphed = c->precision != LB_FP16S && c->n_bulk > 0 && max_steps >= kSolveGraphMinSteps &&
-                       2 * c->Q * c->NP * static_cast<int64_t>(elem_size(c->precision)) < kSolveGraphBytes;
+  bool graphed = c->precision != LB_FP16S && c->n_bulk > 0 && max_steps >= kSolveGraphMinSteps &&
+                 2 * c->Q * c->NP * static_cast<int64_t>(elem_size(c->precision)) < kSolveGraphBytes;
+  // the graph of kSolveGraphSteps steps from buffer `from`; null where it cannot be made
+  auto graph_from = [&](int from) -> hipGraphExec_t {
+    hipGraphExec_t& g = graphs.g[from];
+    if (g) return g;
+    hipGraph_t graph = nullptr;
+    hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) {
+      for (int32_t k = 0; k < kSolveGraphSteps && e == hipSuccess; ++k) e = step((k & 1) ? 1 - from : from, false, false, true);
+      const hipError_t e2 = hipStreamEndCapture(c->stream, &graph);
+      if (e == hipSuccess) e = e2;
+    }
+    if (e == hipSuccess) e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
+    if (graph) hipGraphDestroy(graph);
+    if (e == hipSuccess) return g;
+    (void)hipGetLastError();  // the steps are launched one by one then
+    return g = nullptr;
+  };
   Timer t(c);
   int64_t launches = 0;
   while (steps < max_steps) {
     const int64_t chunk = std::min<int64_t>(check_every, max_steps - steps);
     for (int64_t s = 0; s < chunk;) {
-      hipError_t e = hipSuccess;
+      hipError_t e;
       int32_t n = 1;
-      if (graphed && s > 0 && chunk - 1 - s >= kSolveGraphSteps) {
+      hipGraphExec_t g = nullptr;
+      if (graphed && s > 0 && chunk - 1 - s >= kSolveGraphSteps) graphed = (g = graph_from(c->cur)) != nullptr;
+      if (g) {
         n = kSolveGraphSteps;
-        hipGraphExec_t& g = graphs.g[c->cur];
-        if (!g) {
-          hipGraph_t graph = nullptr;
-          e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
-          if (e == hipSuccess) {
-            for (int32_t k = 0; k < n && e == hipSuccess; ++k) e = step((k & 1) ? 1 - c->cur : c->cur, false, false, true);
-            const hipError_t e2 = hipStreamEndCapture(c->stream, &graph);
-            if (e == hipSuccess) e = e2;
-          }
-          if (e == hipSuccess) e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
-          if (graph) hipGraphDestroy(graph);
-        }
-        if (e == hipSuccess) e = hipGraphLaunch(g, c->stream);
+        e = hipGraphLaunch(g, c->stream);
       } else {
         e = step(c->cur, !c->post, s == chunk - 1, s > 0);
         if (e == hipSuccess) c->cur = 1 - c->cur;

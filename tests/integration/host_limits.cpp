@@ -1,7 +1,8 @@
-// Contexts where pinned host memory is short.  The program's own hipHostMalloc
-// stands before the runtime's: it counts the calls and, with "nopin", refuses
-// them.  argv: pin | nopin, output file (every downloaded value, as doubles), and
-// the memory of the halo buffers: pageable | pinned | device | managed.
+// Contexts where pinned host memory is short, or graphs cannot be made.  The
+// program's own hipHostMalloc and hipGraphInstantiate stand before the runtime's:
+// they count the calls and, with "nopin" or "nograph", refuse them.  argv: pin |
+// nopin | nograph, output file (every downloaded value and solve, as doubles),
+// and the memory of the halo buffers: pageable | pinned | device | managed.
 #include <dlfcn.h>
 
 #include <cstdint>
@@ -12,13 +13,20 @@
 
 #include "badchimp_amd.h"
 
-static int pins = 0;
-static bool refuse = false;
+static int pins = 0, graphs = 0;
+static bool refuse = false, refuse_graphs = false;
 extern "C" int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
   using Malloc = int (*)(void**, size_t, unsigned);
   static const Malloc next = reinterpret_cast<Malloc>(dlsym(RTLD_NEXT, "hipHostMalloc"));
   ++pins;
   return refuse ? 2 /* hipErrorOutOfMemory */ : next(p, bytes, flags);
+}
+
+extern "C" int hipGraphInstantiate(void** exec, void* graph, void** node, char* log, size_t bytes) {
+  using Instantiate = int (*)(void**, void*, void**, char*, size_t);
+  static const Instantiate next = reinterpret_cast<Instantiate>(dlsym(RTLD_NEXT, "hipGraphInstantiate"));
+  ++graphs;
+  return refuse_graphs ? 2 : next(exec, graph, node, log, bytes);
 }
 
 extern "C" {
@@ -107,6 +115,7 @@ static void fields(int n, int nf) {
 int main(int argc, char** argv) {
   if (argc != 4) return 2;
   refuse = !std::strcmp(argv[1], "nopin");
+  refuse_graphs = !std::strcmp(argv[1], "nograph");
   const int32_t dims[3] = {20, 18, 33};
   std::vector<int32_t> geo(20 * 18 * 33), split;
   uint32_t r = 7;
@@ -179,6 +188,17 @@ int main(int argc, char** argv) {
     fields(part.n, nf);
     lb_ctx_destroy(ctx);
   }
+  // a solve whose steps replay graphs
+  set(whole, LB_FP32S);
+  ok(lb_init_equilibrium(ctx, 1, 0, 2, 0, rho.data(), rest.data()), "initial state");
+  double k = 0.0;
+  int64_t steps = 0;
+  graphs = 0;
+  ok(lb_solve_permeability(ctx, 0.9, force, 101, 1e-30, 606, 20.0 * 18 * 33, &k, &steps), "solve");
+  keep({k, static_cast<double>(steps)});
+  std::printf("graphs %d\n", graphs);
+  fields(whole.n, 1);
+  lb_ctx_destroy(ctx);
   std::FILE* f = std::fopen(argv[2], "wb");
   if (!f || std::fwrite(all.data(), sizeof(double), all.size(), f) != all.size() || std::fclose(f)) return 1;
   std::printf("pinned %d, %zu values\n", pins, all.size());

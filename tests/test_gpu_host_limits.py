@@ -1,7 +1,8 @@
 """Calls that stage values in pinned host memory, where that memory cannot be
 had (tests/integration/host_limits.cpp refuses hipHostMalloc): the same values
 through ordinary memory.  Set-up and steps pin none, and the downloads of two
-contexts in turn share one piece."""
+contexts in turn share one piece.  A permeability solve whose steps replay a
+graph gives the same k where no graph can be made."""
 import os
 import re
 import shutil
@@ -53,3 +54,11 @@ def test_values_without_pinned_memory(gpu_available, limits):
 def test_halo_buffers_in_any_memory(gpu_available, limits, buffers):
     """Packs and unpacks in the caller's pinned, device and managed memory."""
     assert np.array_equal(limits("pin", buffers)[1], limits("pin")[1])
+
+
+def test_solve_without_graphs(gpu_available, limits):
+    text, graphed = limits("pin")
+    assert int(re.search(r"graphs (\d+)", text).group(1)) == 2, text  # one per starting buffer
+    text, plain = limits("nograph")
+    assert int(re.search(r"graphs (\d+)", text).group(1)) == 1, text
+    assert np.array_equal(graphed, plain)
