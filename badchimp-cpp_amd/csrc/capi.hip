@@ -1160,10 +1160,10 @@ constexpr int32_t kGraphSteps = 128;
 constexpr int32_t kGraphMinSteps = 2 * kGraphSteps;
 
 // Small D2Q9 lists take kTileSteps steps per launch (tile2d.hpp): the box of
-// the row windows in at most kTileMaxTiles tiles, an operator without a table.
+// the row windows in few enough tiles (tiles_pay), an operator without a table.
 bool tiled(const lb_ctx* c, const BgkArgs& a) {
   return c->lattice == LB_D2Q9 && c->precision != LB_FP16S && c->addr.layout == kLayWin && a.mode != kRheology &&
-         c->tile_box.tiles() <= kTileMaxTiles;
+         tiles_pay(static_cast<int64_t>(elem_size(c->precision)), c->tile_box.tiles(), c->n_bulk);
 }
 
 hipError_t launch_tile(lb_ctx* c, const BgkArgs& a, int from) {

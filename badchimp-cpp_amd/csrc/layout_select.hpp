@@ -59,6 +59,27 @@ inline bool plane_order(int n_fields, int64_t elem_bytes, int64_t buffer) {
   return buffer <= (elem_bytes == 8 ? 2300000000 : elem_bytes == 4 ? 1350000000 : int64_t{1} << 32);
 }
 
+// Whether a D2Q9 list of n nodes takes kTileSteps steps per launch in tiles
+// (tile2d.hpp) or one.  A tiled launch goes by its tiles, solid cells included, and
+// costs another round of 256 workgroups (one more per CU) at a time: FP64 2.1 us per
+// step up to 256 tiles, 2.9 up to 512, 3.65 up to 768, 4.4 up to 1024, 5.2 beyond.
+// A plain step goes by its nodes: 3.2-3.6 us up to 256 blocks of 256 nodes, 4.0-4.5
+// up to 512, 5.1 beyond.  So FP64 lists take tiles up to two rounds more than full
+// rounds of blocks (less a few: 65 k nodes are 256 blocks).  Tiled / plain, BGK and
+// TRT, us per step: 425 tiles, 29 k to 59 k nodes 2.80-3.20 / 3.40-3.66; 616 tiles,
+// 66 k 3.65 / 3.96 and 3.79 / 3.99; 570, 62 k 3.72 / 3.67 and 3.80 / 3.68; 616, 42 k
+// 3.70 / 3.48 and 3.89 / 3.50; 946, 130 k 4.44 / 4.72; 840, 94 k 4.51 / 4.26; 880,
+// 60 k 4.38 / 3.67 and 4.59 / 3.70; 1100, 152 k 5.27 / 5.21.  Float storage, with half
+// the LDS, pays up to 1000 tiles at every porosity from 0.5 on: 425 tiles 1.91-2.22
+// / 3.08-3.20, 840 tiles, 59 k to 120 k nodes 2.96-3.22 / 3.12-3.54; beyond it depends
+// on the solids: 1428 tiles, 198 k 3.71 / 4.57, 118 k 3.63 / 3.58, 2278 tiles, 190 k
+// 4.96 / 4.33.
+inline bool tiles_pay(int64_t elem_bytes, int64_t tiles, int64_t n) {
+  if (elem_bytes == 4) return tiles <= 1000;
+  const int64_t blocks = (n + 255) / 256;
+  return (tiles + 255) / 256 <= 2 + (blocks + 8) / 256;
+}
+
 // Layout of a launch over n_fields fields: the context's layout, with the row
 // windows replaced by the rows
 // (64-bit addresses, same sources) when the fields do not fit below 4 GiB.

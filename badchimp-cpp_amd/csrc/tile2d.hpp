@@ -13,8 +13,8 @@
 // workgroups per CU) measured best of 2 to 8 steps and edges of 16 to 30.  us per
 // step, tiled / plain: FP64 channel 64x48 1.54 / 2.95, 256x128 (32 k nodes) 2.1 /
 // 3.3, 384x190 2.95 / 4.0, 512x256 (946 tiles) 4.4 / 4.6; FP32S 256x128 1.6 / 2.9,
-// 512x256 2.9 / 3.5.  Larger boxes pay more for the halos' work than a launch
-// costs: 1021x509 has 3 698 tiles.
+// 512x256 2.9 / 3.5.  Larger boxes, and those with many solids, pay more for the
+// halos' work than a launch costs (tiles_pay in layout_select.hpp).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,7 +26,6 @@ namespace lbamd {
 constexpr int kTileSteps = 6;
 constexpr int kTileEdge = 22;                           // threads along each axis
 constexpr int kTileCells = kTileEdge - 2 * (kTileSteps - 1);  // own cells along each axis
-constexpr int kTileMaxTiles = 1000;
 
 // The box of a tiled launch: cells along x and along the rows, and whether x is
 // periodic.

@@ -37,6 +37,26 @@ def test_block_order_is_the_faster_one(tmp_path):
     assert got == [int(r[3] < r[4]) for r in ORDER]
 
 
+# bytes per element, tiles, nodes: tiled, plain
+TILES = [
+    (8, 242, 18818, 1.88, 3.25), (8, 425, 29114, 2.80, 3.40), (8, 425, 59400, 3.20, 3.66),
+    (8, 500, 35950, 2.97, 3.92), (8, 570, 78480, 3.62, 4.16), (8, 570, 62438, 3.80, 3.68),
+    (8, 616, 66138, 3.79, 3.99), (8, 616, 49486, 3.70, 3.55), (8, 680, 72634, 3.59, 4.17),
+    (8, 680, 44844, 3.62, 3.46), (8, 748, 101600, 3.69, 4.33), (8, 792, 109220, 4.56, 4.40),
+    (8, 792, 65222, 4.29, 3.65), (8, 840, 94144, 4.51, 4.26), (8, 880, 72278, 4.39, 4.19),
+    (8, 946, 130048, 4.44, 4.72), (8, 946, 77314, 4.43, 4.22), (8, 1034, 142240, 5.25, 5.12),
+    (8, 1100, 91040, 5.18, 4.31), (8, 1620, 229120, 6.96, 6.60), (8, 2278, 190280, 8.60, 5.62),
+    (4, 242, 18818, 1.45, 3.06), (4, 616, 41610, 2.62, 3.13), (4, 840, 58664, 2.96, 3.12),
+    (4, 946, 130048, 2.94, 3.61), (4, 2278, 190280, 4.96, 4.33),
+]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_tiles_are_taken_where_they_are_faster(tmp_path):
+    got = rules(tmp_path, ["tiles_pay(%d, %d, %d)" % r[:3] for r in TILES])
+    assert got == [int(r[3] < r[4]) for r in TILES]
+
+
 XCDS = r'''
 #include "rowbuild.hpp"
 #include <cstdio>
