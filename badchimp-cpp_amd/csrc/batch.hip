@@ -630,7 +630,7 @@ void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t perio
   pr.xcd = block_xcd(rb.coord);
   // every node's own window must name it (a cheap check of the construction)
   for (int64_t i = 0; i < n; ++i) {
-    const auto own = win_cell(rb, pr.wb, static_cast<int32_t>(i), 0, 0, 0);
+    const auto own = WinNode(rb, pr.wb, i).cell(0, 0, 0);
     if (!own.first || own.second != i) {
       pr.code = LB_ERR_STATE;
       pr.why = "row windows inconsistent at node " + std::to_string(i);

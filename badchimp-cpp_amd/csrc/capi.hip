@@ -202,8 +202,8 @@ int pre_state(lb_ctx* c, const void** out) {
 }
 
 // Nodes per host thread of the set-up passes that look at every link of a node.
-// Starting the threads of a pass costs up to a millisecond: D2Q9 421x201 (84 k
-// nodes) took 21.8 ms in all with 16 k nodes per thread for 16.4 on one, D3Q19
+// Starting and joining the 16 threads of a pass takes 0.4 ms and more: D2Q9 421x201
+// (84 k nodes) took 21.8 ms in all with 16 k nodes per thread for 16.4 on one, D3Q19
 // with 140 k nodes 85 ms for 94.
 constexpr int64_t min_nodes(int Q) { return Q == D2Q9::nQ ? 1 << 16 : 1 << 14; }
 
@@ -563,32 +563,44 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
     }
   // a layout is used only when every link it yields is the table's (checked
   // over chunks of the compact nodes on host threads)
-  auto agrees = [&](auto&& source) {
+  auto agrees = [&](auto&& node_agrees) {
     bool bad[kMaxHostThreads] = {};
     parallel_ranges(n_bulk, [&](int64_t b, int64_t e, int t) {
-      for (int64_t i = b; i < e && !bad[t]; ++i)
-        for (int q = 0; q < Q - 1; ++q) {
-          const uint32_t l = link[static_cast<size_t>(q) * NP + i];
-          const auto r = source(q, static_cast<int32_t>(i));
-          const bool stream = (l >> 30) == kLinkStream;
-          if (r.first != stream || (stream && r.second != static_cast<int64_t>(l & kLinkIndexMask))) {
-            bad[t] = true;
-            break;
-          }
-        }
+      while (b < e && node_agrees(b)) ++b;
+      bad[t] = b < e;
     }, min_nodes(Q));
     return std::none_of(bad, bad + kMaxHostThreads, [](bool x) { return x; });
+  };
+  auto link_is = [&](int q, int64_t i, const std::pair<bool, int64_t>& source) {
+    const uint32_t l = link[static_cast<size_t>(q) * NP + i];
+    const bool stream = (l >> 30) == kLinkStream;
+    return source.first == stream && (!stream || source.second == static_cast<int64_t>(l & kLinkIndexMask));
+  };
+  // (directions as constants: a set-up of 36 k nodes took 0.5 ms longer without)
+  auto windows_agree = [&](auto lat, const WinBuild& w) {
+    using L = decltype(lat);
+    return agrees([&](int64_t i) {
+      const WinNode n(rb, w, i);
+      bool ok = true;
+#pragma unroll
+      for (int q = 0; q < L::nQ - 1; ++q) ok = link_is(q, i, n.cell(-cx<L>(q), -cy<L>(q), -cz<L>(q))) && ok;
+      return ok;
+    });
   };
   // row windows; the rows are looked at where they may be used, that is without
   // windows or for two fields that the windows cannot address (launch_layout)
   WinBuild wb;
   bool win_ok = rows_ok && win_allowed && build_windows(rb, true, wb, why);
-  if (win_ok && !agrees([&](int q, int32_t i) { return win_source(c->lattice, rb, wb, q, i); })) {
+  if (win_ok && !(c->lattice == LB_D2Q9 ? windows_agree(D2Q9{}, wb) : windows_agree(D3Q19{}, wb))) {
     win_ok = false;
     why = "row windows disagree with the neighbour index";
   }
   if (rows_ok && !(win_ok && rowwin_fits(Q, NP, 2, static_cast<int64_t>(elem_size(c->precision)))) &&
-      !agrees([&](int q, int32_t i) { return row_source(c->lattice, rb, q, i); })) {
+      !agrees([&](int64_t i) {
+        for (int q = 0; q < Q - 1; ++q)
+          if (!link_is(q, i, row_source(c->lattice, rb, q, static_cast<int32_t>(i)))) return false;
+        return true;
+      })) {
     rows_ok = win_ok = false;
     why = "row layout disagrees with the neighbour index";
   }

@@ -196,29 +196,37 @@ inline bool build_windows(const RowBuild& rb, bool allow_periodic, WinBuild& wb,
   return true;
 }
 
-// The cell (dx, dy, dz) off compact node i's under the row windows, as RowWin
-// and RowWinZ find it on the device: {fluid, compact index}, or {false, i}.
-inline std::pair<bool, int64_t> win_cell(const RowBuild& rb, const WinBuild& wb, int32_t i, int dx, int dy, int dz) {
-  const uint32_t cc = rb.coord[i];
-  const int32_t X = static_cast<int32_t>(cc >> 22), Y = static_cast<int32_t>((cc >> 12) & 1023u),
-                Z = static_cast<int32_t>(cc & 4095u);
-  const uint32_t t = kWinBase + (static_cast<uint32_t>(Z) & (kWinCells - 1u));
-  const size_t pr = static_cast<size_t>(X + 1 + dx) * wb.PY + (Y + 1 + dy);
-  const uint32_t m = wb.win[pr * wb.W + (Z >> kWinLog)];
-  const uint32_t below = (2u << t) - (2u << kWinBase);
-  const uint32_t b0 = (m & ((1u << kWinBase) - 1u)) + static_cast<uint32_t>(__builtin_popcount(m & below)) +
-                      (wb.plane.empty() ? 0u : wb.plane[X + 1 + dx]);
-  if (!((m >> (t + 1 + dz)) & 1u)) return {false, i};
-  const uint32_t n = wb.count.empty() ? 0u : wb.count[pr];
-  if (dz == 0) return {true, static_cast<int64_t>(b0)};
-  if (dz < 0) return {true, static_cast<int64_t>(b0 - 1u + (Z == 0 ? n : 0u))};
-  return {true, static_cast<int64_t>(b0 + ((m >> (t + 1u)) & 1u) - (Z == wb.EZ - 1 ? n : 0u))};
-}
+// The cells around compact node i as RowWin and RowWinZ find them on the device.
+struct WinNode {
+  const WinBuild& wb;
+  const int64_t i;
+  const int32_t X, Z;
+  const size_t pr;    // padded row
+  const uint32_t t;   // bit of cell z - 1 in a word
+  WinNode(const RowBuild& rb, const WinBuild& w, int64_t n)
+      : wb(w), i(n), X(static_cast<int32_t>(rb.coord[n] >> 22)), Z(static_cast<int32_t>(rb.coord[n] & 4095u)),
+        pr(static_cast<size_t>(X + 1) * w.PY + (((rb.coord[n] >> 12) & 1023u) + 1)),
+        t(kWinBase + (static_cast<uint32_t>(Z) & (kWinCells - 1u))) {}
+  // the cell (dx, dy, dz) off the node's: {fluid, compact index}, or {false, i}
+  std::pair<bool, int64_t> cell(int dx, int dy, int dz) const {
+    const size_t row = pr + static_cast<int64_t>(dx) * wb.PY + dy;
+    const uint32_t m = wb.win[row * wb.W + (Z >> kWinLog)];
+    if (!((m >> (t + 1 + dz)) & 1u)) return {false, i};
+    const uint32_t below = (2u << t) - (2u << kWinBase);
+    const uint32_t b0 = (m & ((1u << kWinBase) - 1u)) + static_cast<uint32_t>(__builtin_popcount(m & below)) +
+                        (wb.plane.empty() ? 0u : wb.plane[X + 1 + dx]);
+    if (dz == 0) return {true, static_cast<int64_t>(b0)};
+    const uint32_t n = !wb.count.empty() && Z == (dz < 0 ? 0 : wb.EZ - 1) ? wb.count[row] : 0u;
+    if (dz < 0) return {true, static_cast<int64_t>(b0 - 1u + n)};
+    return {true, static_cast<int64_t>(b0 + ((m >> (t + 1u)) & 1u) - n)};
+  }
+};
 
 // Source of direction q for compact node i under the row windows.
 inline std::pair<bool, int64_t> win_source(int lattice, const RowBuild& rb, const WinBuild& wb, int q, int32_t i) {
-  if (lattice == LB_D2Q9) return win_cell(rb, wb, i, -D2Q9::c(q, 0), 0, -D2Q9::c(q, 1));
-  return win_cell(rb, wb, i, -D3Q19::c(q, 0), -D3Q19::c(q, 1), -D3Q19::c(q, 2));
+  const WinNode n(rb, wb, i);
+  if (lattice == LB_D2Q9) return n.cell(-D2Q9::c(q, 0), 0, -D2Q9::c(q, 1));
+  return n.cell(-D3Q19::c(q, 0), -D3Q19::c(q, 1), -D3Q19::c(q, 2));
 }
 
 // XCD of each 256-node block of a node list in row order, for dispatch (the
