@@ -293,7 +293,7 @@ int refresh(lb_batch* b) {
     if (kind == 0) b->n_items_bgk = static_cast<int32_t>(b->items.size());
   }
   b->n_items_cg = static_cast<int32_t>(b->items.size()) - b->n_items_bgk;
-  b->nt = stream_stores(bytes);
+  b->nt = stream_stores(bytes, b->n_items_bgk == 0 ? 2 : 1);  // two-phase solves alone: two fields
   if (static_cast<int64_t>(b->items.size()) > b->items_cap) {
     if (b->d_items) hipFree(b->d_items);
     b->d_items = nullptr;

@@ -150,7 +150,9 @@ int alloc_fields(lb_ctx* c, int nf) {
   c->n_fields = nf;
   c->addr.win.order = c->addr.winz.order =
       plane_order(nf, static_cast<int64_t>(elem_size(c->precision)), static_cast<int64_t>(bytes)) ? c->d_order : nullptr;
-  c->addr.nt = stream_stores(2 * static_cast<int64_t>(bytes));
+  c->addr.nt = stream_stores(2 * static_cast<int64_t>(bytes), nf);
+  c->addr.nt_table =
+      stream_stores(2 * static_cast<int64_t>(bytes), nf, static_cast<int64_t>(sizeof(uint32_t)) * (c->Q - 1) * c->NP);
   c->cur = 0;
   c->post = false;
   c->step_count = 0;

@@ -19,7 +19,8 @@ struct Addr {
   RowAddr rows{};
   RowWin win{};
   RowWinZ winz{};
-  bool nt = true;  // streaming stores (stream_stores)
+  // streaming stores (stream_stores): in the row windows, with the link table
+  bool nt = true, nt_table = true;
 };
 
 // ---- FP64 (reference arithmetic, -ffp-contract=off) ----------------------

@@ -856,15 +856,15 @@ inline dim3 grid_for(int32_t n) { return dim3(static_cast<unsigned>((n + kBlock 
 template <typename F>
 hipError_t step_dispatch(int precision, int lattice, const Addr& ad, int layout, bool first, F&& f) {
   auto by_addr = [&](auto l, auto st) {
-    auto by_store = [&](const auto& a) {
-      if (ad.nt) f(l, st, a, std::true_type{});
+    auto by_store = [&](const auto& a, bool nt) {
+      if (nt) f(l, st, a, std::true_type{});
       else f(l, st, a, std::false_type{});
     };
     if (first) f(l, st, ad.table, std::true_type{});
-    else if (layout == kLayWin) by_store(ad.win);
-    else if (layout == kLayWinZ) by_store(ad.winz);
+    else if (layout == kLayWin) by_store(ad.win, ad.nt);
+    else if (layout == kLayWinZ) by_store(ad.winz, ad.nt);
     else if (layout == kLayRows) f(l, st, ad.rows, std::true_type{});  // buffers above 4 GiB
-    else by_store(ad.table);
+    else by_store(ad.table, ad.nt_table);
   };
   if (lattice == 0) {
     if (precision == 1) by_addr(D2Q9{}, float{});
@@ -1086,7 +1086,8 @@ hipError_t cg_lowp(int precision, int lattice, bool first, bool store, const voi
     using S = decltype(st);
     using A = std::decay_t<decltype(addr)>;
     constexpr bool NT = decltype(nt)::value;
-    if constexpr (!std::is_same_v<A, RowAddr>) {  // the two-phase layouts are the link table and the windows
+    // the two-phase layouts are the link table, with streaming stores, and the windows
+    if constexpr (!std::is_same_v<A, RowAddr> && (NT || !std::is_same_v<A, TableAddr>)) {
       const S* gi = static_cast<const S*>(gin);
       S* go = static_cast<S*>(gout);
       const dim3 g = grid_for(n), b(kBlock);

@@ -893,15 +893,15 @@ inline dim3 grid_for(int32_t n) { return dim3(static_cast<unsigned>((n + kBlock 
 // the link table's.
 template <class F>
 static void step_dispatch(const Addr& ad, int layout, bool first, F&& f) {
-  auto by_store = [&](const auto& a) {
-    if (ad.nt) f(a, std::true_type{});
+  auto by_store = [&](const auto& a, bool nt) {
+    if (nt) f(a, std::true_type{});
     else f(a, std::false_type{});
   };
   if (first) f(ad.table, std::true_type{});
-  else if (layout == kLayWin) by_store(ad.win);
-  else if (layout == kLayWinZ) by_store(ad.winz);
+  else if (layout == kLayWin) by_store(ad.win, ad.nt);
+  else if (layout == kLayWinZ) by_store(ad.winz, ad.nt);
   else if (layout == kLayRows) f(ad.rows, std::true_type{});  // buffers above 4 GiB
-  else by_store(ad.table);
+  else by_store(ad.table, ad.nt_table);
 }
 
 hipError_t bgk_f64(int lattice, bool first, bool store, bool reduce, const double* fin,
@@ -973,7 +973,8 @@ hipError_t cg_f64(int lattice, bool first, bool store, const double* fin, double
     step_dispatch(ad, layout, first, [&](const auto& addr, auto nt) {
       using A = std::decay_t<decltype(addr)>;
       constexpr bool NT = decltype(nt)::value;
-      if constexpr (!std::is_same_v<A, RowAddr>) {  // the two-phase layouts are the link table and the windows
+      // the two-phase layouts are the link table, with streaming stores, and the windows
+      if constexpr (!std::is_same_v<A, RowAddr> && (NT || !std::is_same_v<A, TableAddr>)) {
         if constexpr (std::is_same_v<A, TableAddr> && NT) {
           if (first && store) return k_cg<L, true, true, NT, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);
           if (first) return k_cg<L, true, false, NT, A><<<g, b, 0, s>>>(fin, fout, addr, n, NP, a, phi, wp, dscalar, rho, vel);

@@ -33,8 +33,24 @@ inline bool rowwin_fits(int Q, int64_t NP, int n_fields, int64_t elem_bytes) {
 // 52.9 / 50.9, FP64 256^3 366 / 351.  A batch of 4 packs of 64^3, FP32S (64 MB)
 // 13.5 / 15.6, FP64 (128 MB) 22.6 / 26.8; 3 of 96^3, FP16S 20.6 / 24.7; 4 of
 // 128^3, FP16S 56.1 / 67.4.
-inline bool stream_stores(int64_t both_buffers) {
-  return both_buffers < 20000000 || both_buffers > (int64_t{256} << 20);
+// The link table (link bytes, 0 for the other layouts) is read in every step and
+// counts: FP32S 144^3 (177 MB and 84) 41.0 / 42.8, D2Q9 1000x4000 (202 and 90) 49.9 /
+// 48.0, 160^3 (243 and 115) 66.3 / 61.3; FP64 112^3 (165 and 39) 35.9 / 38.3, 128^3
+// (247 and 59) 56.4 / 54.7, 144^3 (353 and 84) 81.9 / 71.7; FP16S 160^3 (121 and 115)
+// 41.4 / 43.1, 176^3 (162 and 153) 62.0 / 55.3.
+// Two fields, which the colour pass reads before the collision does: plain stores
+// pay from 60 MB on only: FP32S D2Q9 800x400 (32 MB) 13.2 / 12.6,
+// 800x600 (48 MB) 17.0 / 16.4, D3Q19 80^3 (59 MB) 20.1 / 19.9, 96^3 (103 MB) 32.9 /
+// 34.2; FP64 64^3 (60 MB) 20.2 / 20.4, 80^3 (118 MB) 31.5 / 33.5; FP16S 80^3 (30 MB)
+// 17.1 / 16.4, 112^3 (82 MB) 36.6 / 38.4; batches of two-phase solves, FP32S 3 of
+// 48^3 (37 MB) 17.4 / 16.5, 6 (74 MB) 26.1 / 27.3, FP64 8 of 32^3 (56 MB) 21.4 /
+// 21.8, 20 (140 MB) 39.4 / 43.0, FP16S 3 of 64^3 (45 MB) 25.9 / 25.6.  With the link table, which both passes
+// read, they do not pay at all: FP32S 80^3 33.6 / 32.3, 112^3 (165 MB) 86.8 / 83.9, D2Q9
+// 1000x1000 (101 MB) 43.6 / 42.1, FP64 96^3 (206 MB) 74.9 / 74.9; the exception is
+// FP64 80^3 (118 MB) 42.9 / 43.9.
+inline bool stream_stores(int64_t both_buffers, int n_fields = 1, int64_t link = 0) {
+  if (n_fields == 2 && link > 0) return true;
+  return both_buffers < (n_fields == 2 ? 60000000 : 20000000) || both_buffers + link > (int64_t{256} << 20);
 }
 
 // Whether the blocks of the row windows go to the XCDs plane by plane
