@@ -621,7 +621,7 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
   c->n_ghost = 0;
   c->slot_of.clear();
   for (void* p : {static_cast<void*>(c->d_coord), static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win),
-                  static_cast<void*>(c->d_order), static_cast<void*>(c->d_node)})
+                  static_cast<void*>(c->d_order)})
     if (p) hipFree(p);
   c->d_order = nullptr;
   c->d_node = nullptr;
@@ -713,12 +713,12 @@ int setup_topology(lb_ctx* c, int32_t n_nodes, const int32_t* neighbor, const in
       else
         c->bulk_runs.push_back({n, r, 1});
     }
-    if (!std::is_sorted(by_node.begin(), by_node.end())) {
-      if ((rc = dev_alloc(c, &c->d_node, by_node.size())) != LB_OK) return rc;
-      LB_HIP(c, hipMemcpy(c->d_node, by_node.data(), by_node.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    }
+    // one allocation: the ranks, and the order by node where it is not the compact one
+    const bool sorted = std::is_sorted(by_node.begin(), by_node.end());
+    if (!sorted) rank.insert(rank.end(), by_node.begin(), by_node.end());
     if ((rc = dev_alloc(c, &c->d_rank, rank.size())) != LB_OK) return rc;
     LB_HIP(c, hipMemcpy(c->d_rank, rank.data(), rank.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    if (!sorted) c->d_node = c->d_rank + NP;
   }
   c->wall_nodes = walls;
   c->node_type.assign(node_type, node_type + n_nodes);
@@ -777,7 +777,7 @@ int lb_ctx_destroy(lb_ctx* c) {
                   static_cast<void*>(c->d_phi), static_cast<void*>(c->d_phi_wall), static_cast<void*>(c->d_partial),
                   static_cast<void*>(c->d_scalar), static_cast<void*>(c->d_coord),
                   static_cast<void*>(c->d_rows), static_cast<void*>(c->d_win), static_cast<void*>(c->d_table),
-                  static_cast<void*>(c->d_rank), static_cast<void*>(c->d_order), static_cast<void*>(c->d_node)})
+                  static_cast<void*>(c->d_rank), static_cast<void*>(c->d_order)})
     if (p) hipFree(p);
   for (hipEvent_t e : c->stage_ev)
     if (e) hipEventDestroy(e);

@@ -29,7 +29,7 @@ struct lb_ctx {
   // position, length} (lb_download_f_noalloc copies each run in one piece)
   int32_t* d_rank = nullptr;
   std::vector<std::array<int32_t, 3>> bulk_runs;
-  int32_t* d_node = nullptr;    // compact node at each position, null where it is the position itself
+  const int32_t* d_node = nullptr;  // compact node at each position (after the ranks), null where it is the position itself
   hipEvent_t stage_ev[2] = {nullptr, nullptr};  // of a field download's two slabs
   std::vector<int32_t> wall_nodes;  // wall slot -> node number
   // other-rank fluid nodes (type 4, the halo): population slots after the
