@@ -138,6 +138,15 @@ void free_fields(lb_ctx* c) {
   c->n_fields = 0;
 }
 
+// The stores of a call of nsteps steps (stream_stores).
+void choose_stores(lb_ctx* c, int32_t nsteps) {
+  const int64_t both = 2 * static_cast<int64_t>(c->n_fields) * c->Q * c->NP * static_cast<int64_t>(elem_size(c->precision));
+  const int64_t link = static_cast<int64_t>(sizeof(uint32_t)) * (c->Q - 1) * c->NP;
+  const int64_t fields = nsteps <= 2 ? static_cast<int64_t>(sizeof(double)) * (1 + c->nD) * c->NP : 0;
+  c->addr.nt = stream_stores(both, c->n_fields, 0, fields);
+  c->addr.nt_table = stream_stores(both, c->n_fields, link, fields);
+}
+
 int alloc_fields(lb_ctx* c, int nf) {
   if (c->n_fields == nf) return LB_OK;
   free_fields(c);
@@ -150,9 +159,7 @@ int alloc_fields(lb_ctx* c, int nf) {
   c->n_fields = nf;
   c->addr.win.order = c->addr.winz.order =
       plane_order(nf, static_cast<int64_t>(elem_size(c->precision)), static_cast<int64_t>(bytes)) ? c->d_order : nullptr;
-  c->addr.nt = stream_stores(2 * static_cast<int64_t>(bytes), nf);
-  c->addr.nt_table =
-      stream_stores(2 * static_cast<int64_t>(bytes), nf, static_cast<int64_t>(sizeof(uint32_t)) * (c->Q - 1) * c->NP);
+  choose_stores(c, INT32_MAX);
   c->cur = 0;
   c->post = false;
   c->step_count = 0;
@@ -1190,6 +1197,7 @@ hipError_t launch_tile(lb_ctx* c, const BgkArgs& a, int from) {
 
 int step_single(lb_ctx* c, int32_t nsteps, const BgkArgs& a) {
   hipSetDevice(c->device);
+  choose_stores(c, nsteps);
   Timer t(c);
   // n steps in some launches, each of which changes the buffer
   auto advance = [c](int32_t n, int32_t launches) {
@@ -1770,6 +1778,7 @@ int solve_permeability(lb_ctx* c, const char* name, double tau, double tau_anti,
       force[0] == 0.0)
     return fail(c, LB_ERR_ARG, "%s: bad argument", name);
   hipSetDevice(c->device);
+  choose_stores(c, check_every);
   const BgkArgs a = single_phase_args(c, tau, tau_anti, force);
   const double nu = (tau - 0.5) / 3.0;
   double k_prev = 0.0, k = 0.0;

@@ -21,16 +21,17 @@ inline bool rowwin_fits(int Q, int64_t NP, int n_fields, int64_t elem_bytes) {
 }
 
 // Whether the step kernels write populations with streaming stores, for both
-// buffers of a context, or of all active solves of a batch, together.  Up to the
-// MALL's 256 MiB a plain store leaves the values where the next step reads them;
-// above it a plain store only displaces lines that are still to be read.  Below
+// buffers of a context, or of all active solves of a batch, together.  While they
+// fit the MALL's 256 MiB a plain store leaves the values where the next step reads
+// them; beyond, a plain store only displaces lines that are still to be read.  Below
 // 20 MB, where the buffers fit the L2s, a plain store is written back when the
 // kernel ends, after its last node.  Plain / streaming, us per step:
 // FP32S 64^3 pack (16 MB) 5.55 / 5.23, D2Q9 1021x509 (22 MB) 5.6 / 6.0, FP32S
 // 80^3 (30 MB) 7.4 / 8.9, FP64 96^3 (107 MB) 19.3 / 23.7, FP16S 161x143x150
 // (100 MB) 22.2 / 26.8, FP64 128^3 (255 MB) 40.4 / 47.6; two-phase FP64 64^3
 // (62 MB) 22.0 / 22.0, 100^3 (245 MB) 59.1 / 62.4; beyond: FP32S 165^3 (273 MB)
-// 52.9 / 50.9, FP64 256^3 366 / 351.  A batch of 4 packs of 64^3, FP32S (64 MB)
+// 52.9 / 50.9, FP64 256^3 366 / 351; around the limit FP64 128^3 periodic along all
+// axes (255 MB) 46.6 / 49.5, FP32S 200x170x150 (265 MB) 53.5 / 50.7.  A batch of 4 packs of 64^3, FP32S (64 MB)
 // 13.5 / 15.6, FP64 (128 MB) 22.6 / 26.8; 3 of 96^3, FP16S 20.6 / 24.7; 4 of
 // 128^3, FP16S 56.1 / 67.4.
 // The link table (link bytes, 0 for the other layouts) is read in every step and
@@ -38,6 +39,11 @@ inline bool rowwin_fits(int Q, int64_t NP, int n_fields, int64_t elem_bytes) {
 // 48.0, 160^3 (243 and 115) 66.3 / 61.3; FP64 112^3 (165 and 39) 35.9 / 38.3, 128^3
 // (247 and 59) 56.4 / 54.7, 144^3 (353 and 84) 81.9 / 71.7; FP16S 160^3 (121 and 115)
 // 41.4 / 43.1, 176^3 (162 and 153) 62.0 / 55.3.
+// So do density and velocity (fields bytes) in calls of one or two steps, which all
+// write them: FP32S 160^3 (243 MB and 51) 1 step per call 63.6 / 57.9, 2 55.9 / 53.1,
+// 10 42.4 / 48.5; FP64 128^3 (247 and 26) 59.3 / 54.0, 51.0 / 50.8, 42.2 / 48.2; FP16S
+// 200^3 (209 and 88) 77.9 / 73.7, 66.7 / 67.2, 50.9 / 58.6; within the limit FP64 120^3
+// (203 and 22) 40.5 / 45.8, FP32S 150^3 (200 and 42) 42.4 / 48.6.
 // Two fields, which the colour pass reads before the collision does: plain stores
 // pay from 60 MB on only: FP32S D2Q9 800x400 (32 MB) 13.2 / 12.6,
 // 800x600 (48 MB) 17.0 / 16.4, D3Q19 80^3 (59 MB) 20.1 / 19.9, 96^3 (103 MB) 32.9 /
@@ -48,9 +54,9 @@ inline bool rowwin_fits(int Q, int64_t NP, int n_fields, int64_t elem_bytes) {
 // read, they do not pay at all: FP32S 80^3 33.6 / 32.3, 112^3 (165 MB) 86.8 / 83.9, D2Q9
 // 1000x1000 (101 MB) 43.6 / 42.1, FP64 96^3 (206 MB) 74.9 / 74.9; the exception is
 // FP64 80^3 (118 MB) 42.9 / 43.9.
-inline bool stream_stores(int64_t both_buffers, int n_fields = 1, int64_t link = 0) {
+inline bool stream_stores(int64_t both_buffers, int n_fields = 1, int64_t link = 0, int64_t fields = 0) {
   if (n_fields == 2 && link > 0) return true;
-  return both_buffers < (n_fields == 2 ? 60000000 : 20000000) || both_buffers + link > (int64_t{256} << 20);
+  return both_buffers < (n_fields == 2 ? 60000000 : 20000000) || both_buffers + link + fields > 262000000;
 }
 
 // Whether the blocks of the row windows go to the XCDs plane by plane

@@ -37,18 +37,25 @@ def test_block_order_is_the_faster_one(tmp_path):
     assert got == [int(r[3] < r[4]) for r in ORDER]
 
 
-# fields, MB of both buffers, of the link table where the step reads it: plain, streaming stores
+# fields, MB of both buffers, of what else a step reads or writes (the link table; density and velocity): plain,
+# streaming stores
 STORES = [
     (1, 14.9, 7.0, 6.82, 6.52), (1, 29.7, 7.0, 9.44, 10.85), (1, 24.1, 10.7, 6.69, 7.46), (1, 103.1, 24.4, 23.44, 26.34),
     (1, 176.5, 83.6, 40.97, 42.83), (1, 201.4, 44.8, 40.34, 41.32), (1, 121.4, 115.0, 41.41, 43.05),
     (1, 201.5, 89.6, 49.85, 47.95), (1, 246.9, 58.5, 56.37, 54.70), (1, 242.8, 115.0, 66.27, 61.26),
     (1, 353.0, 83.6, 81.88, 71.69), (1, 162.0, 153.4, 62.04, 55.27), (1, 32.1, 0, 6.74, 8.01),
-    (1, 201.4, 0, 31.69, 36.53), (1, 403.0, 0, 73.69, 68.33),
+    (1, 201.4, 0, 31.69, 36.53), (1, 403.0, 0, 73.69, 68.33), (1, 255.0, 0, 46.61, 49.48), (1, 265.0, 0, 53.53, 50.68),
     (2, 14.9, 0, 13.43, 11.96), (2, 32.1, 0, 13.22, 12.57), (2, 48.2, 0, 17.00, 16.39), (2, 29.6, 0, 17.09, 16.44),
     (2, 64.2, 0, 18.69, 19.42), (2, 118.3, 0, 31.52, 33.53), (2, 103.1, 0, 32.86, 34.15), (2, 82.4, 0, 36.62, 38.36),
     (2, 242.8, 0, 96.51, 101.15), (2, 493.9, 0, 139.86, 130.43),
     (2, 29.7, 7.0, 23.14, 22.90), (2, 59.2, 14.0, 33.57, 32.26), (2, 100.6, 22.4, 43.59, 42.10),
     (2, 164.8, 39.0, 86.78, 83.93), (2, 246.9, 58.5, 128.06, 122.50), (2, 705.9, 83.6, 248.03, 236.27),
+]
+# the same for calls of one step, which write density and velocity
+STORES_1 = [
+    (1, 243.0, 51.0, 63.59, 57.87), (1, 247.0, 26.0, 59.32, 53.95), (1, 255.0, 27.0, 61.58, 56.08),
+    (1, 209.0, 88.0, 77.90, 73.71), (1, 203.0, 22.0, 40.52, 45.80), (1, 200.0, 42.0, 42.36, 48.56),
+    (1, 165.0, 18.0, 33.50, 39.39),
 ]
 
 
@@ -56,6 +63,8 @@ STORES = [
 def test_stores_are_the_faster_ones(tmp_path):
     got = rules(tmp_path, ["stream_stores(%d, %d, %d)" % (r[1] * 1e6, r[0], r[2] * 1e6) for r in STORES])
     assert got == [int(r[4] < r[3]) for r in STORES]
+    got = rules(tmp_path, ["stream_stores(%d, %d, 0, %d)" % (r[1] * 1e6, r[0], r[2] * 1e6) for r in STORES_1])
+    assert got == [int(r[4] < r[3]) for r in STORES_1]
 
 
 # bytes per element, tiles, nodes: tiled, plain
