@@ -43,3 +43,19 @@ def test_store_routes_agree(gpu_available, precision, two_phase):
     many = run([big] * 6 + [small], precision, two_phase and [rb] * 6 + [rs] or None)
     assert mid[1] == alone == many[6]
     assert all(m == mid[0] for m in many[:6])
+
+
+@pytest.mark.parametrize("precision", [lbamd.FP64, lbamd.FP32S, lbamd.FP16S])
+def test_store_routes_equal_contexts(gpu_available, precision):
+    """Solves of a batch that writes with plain stores against a context for each."""
+    geos = [lbamd.sphere_pack(n, r, p, s, periodic="x", walls=True)[0]
+            for n, r, p, s in (((96, 96, 96), 9.0, 0.5, 1), ((32, 33, 31), 4.0, 0.45, 2))]
+    for geo, got in zip(geos, run(geos, precision)):
+        topo = lbamd.Topology.from_geometry(geo, lbamd.D3Q19, "x")
+        ctx = lbamd.Context(lbamd.D3Q19, precision)
+        ctx.set_topology_from(topo)
+        ctx.init_equilibrium(1, 0, np.ones(topo.n_nodes), np.zeros((topo.n_nodes, 3)))
+        k, steps = ctx.solve_permeability(TAU, FORCE, 50, 1e-30, 100, float(geo.size))
+        ctx.close()
+        topo.close()
+        assert (got[0], got[2]) == (k, steps)
