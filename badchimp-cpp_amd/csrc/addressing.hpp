@@ -68,10 +68,11 @@ namespace lbamd {
 // On the 256^3 pack runs of 4 blocks are 2.4 % faster than runs of 1 (the
 // plain order) in FP32S and 2 % in FP64; runs of 8-32 give about the same,
 // one contiguous range per XCD (eight fronts) is 3 % slower.  It serves the
-// link table, the rows and the largest FP64 lists; the other row windows and the
-// batched items go to the XCDs plane by plane (block_order, interleave_xcds in
-// rowbuild.hpp).  The mapping only changes which workgroup computes a block:
-// per-block partial sums keep their block index, so results do not change.
+// link table, the rows and the largest lists (plane_order in layout_select.hpp);
+// the other row windows and the batched items go to the XCDs plane by plane
+// (block_order, interleave_xcds in rowbuild.hpp).  The mapping only changes which
+// workgroup computes a block: per-block partial sums keep their block index, so
+// results do not change.
 constexpr int32_t kXcdChunk = 4;
 __device__ __forceinline__ int32_t node_block(int32_t b, int32_t nb) {
   const int32_t full = (nb / (8 * kXcdChunk)) * (8 * kXcdChunk);
@@ -79,12 +80,6 @@ __device__ __forceinline__ int32_t node_block(int32_t b, int32_t nb) {
   const int32_t xcd = b & 7, k = b >> 3;
   return ((k / kXcdChunk) * 8 + xcd) * kXcdChunk + (k % kXcdChunk);
 }
-
-// The same mapping with the dispatch order reversed: a pass that follows
-// another one over the same nodes starts where the first one ended, so its
-// first reads find the lines that the first pass fetched last still in the
-// MALL.  The two-phase collision pass runs this way after the colour pass.
-__device__ __forceinline__ int32_t node_block_rev(int32_t b, int32_t nb) { return node_block(nb - 1 - b, nb); }
 
 // Block of workgroup wg of nb: the layout's block order where it has one
 // (block_order in rowbuild.hpp), else node_block.
@@ -95,6 +90,10 @@ __device__ __forceinline__ int32_t block_of(const A& ad, int32_t wg, int32_t nb)
   }
   return node_block(wg, nb);
 }
+// The same with the dispatch order reversed: a pass that follows another one over
+// the same nodes starts where the first one ended, so its first reads find the
+// lines that the first pass fetched last still in the MALL.  The two-phase
+// collision pass runs this way after the colour pass.
 template <class A>
 __device__ __forceinline__ int32_t block_of_rev(const A& ad, int32_t wg, int32_t nb) {
   return block_of(ad, nb - 1 - wg, nb);

@@ -109,7 +109,10 @@ int lb_set_topology_grid(lb_ctx* ctx, int32_t n_nodes, const int32_t* neighbor,
                          const int16_t* node_type, const int32_t* bulk,
                          int32_t n_bulk, const int32_t* pos, int32_t flags);
 
-/* 0 = per-link table, 1 = row layout, -1 = no topology. */
+/* 0 = per-link table, 1 = row layout, 2 = row windows (a row layout with one
+ * 4-byte word per 8 cells of a row), -1 = no topology.  Windows of a box that is
+ * periodic along the row axis count as 1, and lb_layout_note names them
+ * ("rows (periodic along the row axis)"). */
 int32_t lb_layout(const lb_ctx* ctx);
 const char* lb_layout_note(const lb_ctx* ctx);
 
