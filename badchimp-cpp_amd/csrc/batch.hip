@@ -627,7 +627,7 @@ void prepare(int lattice, const int32_t* dims, const int32_t* geo, int32_t perio
   }
   const RowBuild& rb = pr.rb;
   const int64_t n = static_cast<int64_t>(rb.coord.size());
-  pr.xcd = block_xcd(rb.coord);
+  pr.xcd = block_xcd(rb.coord, kBatchPlaneBlocks);
   // every node's own window must name it (a cheap check of the construction)
   for (int64_t i = 0; i < n; ++i) {
     const auto own = WinNode(rb, pr.wb, i).cell(0, 0, 0);
