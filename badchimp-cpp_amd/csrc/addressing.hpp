@@ -37,7 +37,7 @@
 //            per lane takes the vector L1 about 5 cycles where 16 lanes read
 //            neighbouring words (the nodes of a row do), one of 8 or 16 bytes
 //            takes 17 whatever it reads (measured on tables in L2), and the
-//            step keeps that unit busy 80-90 % of its time.  Against 16-byte
+//            step keeps that unit busy 79-87 % of its time.  Against 16-byte
 //            entries over 32 cells a step takes, on the 256^3 pack, 127 us for
 //            142 (FP16S), 187 for 192 (FP32S) and 350 as before (FP64, bound
 //            by the memory); on a 161 x 143 x 150 pack 26.8 for 30.1 (FP16S).

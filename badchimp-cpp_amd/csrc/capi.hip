@@ -384,13 +384,13 @@ constexpr size_t kFieldStage = size_t{32} << 20;
 
 // Stages are lent to one download at a time and kept for the next one, of any
 // context: pinning 32 MiB takes 1.5 ms with its first use, as long as a small
-// context's download.  At most kIdleStages wait in the process; the last context
-// that is destroyed frees them.
+// context's download.  As many as downloads ran at the same time wait in the
+// process, at most kIdleStages; the last context that is destroyed frees them.
 struct FieldStage {
   double* p = nullptr;
   size_t bytes = 0;
 };
-constexpr size_t kIdleStages = 4;
+constexpr size_t kIdleStages = kMaxHostThreads;
 std::mutex g_stage_mu;
 std::vector<FieldStage> g_idle_stages;
 int g_contexts = 0;

@@ -206,9 +206,9 @@ int lb_init_equilibrium(lb_ctx* ctx, int32_t n_fields, int32_t field,
  * field).  They are the values of the pre-collision state of the last step,
  * as std_case/main.cpp:119-120 and main_TWOPHASE.cpp:241-245,329 store them.
  * They pass through pinned host memory of at most 32 MiB, which the process
- * keeps for the next download of any context (at most four of them, one per
- * download at a time; freed with the last context); where none can be pinned
- * they go through ordinary memory. */
+ * keeps for the next download of any context (one piece per download at a time,
+ * at most 16; freed with the last context); where none can be pinned they go
+ * through ordinary memory. */
 int lb_download_scalar(lb_ctx* ctx, int32_t which, int32_t n_fields, double* s);
 int lb_download_vector(lb_ctx* ctx, int32_t which, int32_t n_fields, double* v);
 
